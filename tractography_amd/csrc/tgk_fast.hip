@@ -482,16 +482,15 @@ __device__ __forceinline__ void wave_segment_test(const MeshView &m, Lane<G> &L,
     }
 }
 
-// nz: this step's Diffusion draws, made by the caller before anything that
-// waits on memory, so they cover the latency of the cell data
-// request_cells asked for.
-template <int MODEL, int ALGO, int DOMAIN, int LMAX, int G, int LDS_VEC, int BLOCK>
-__device__ __forceinline__ void advance(const TrackLaunch &p, bool shared_affine, const float *__restrict__ coeffs,
-                                        uint32_t cstride, Lane<G> &L, float *q, float4 *__restrict__ lds_rows,
-                                        const fast::Noise &nz, bool seg_decided, bool seg_found, uint32_t seg_tri)
+// The tests that end a streamline before its next update, in the reference's
+// order (tracking.py:121-133): the row or the step count is full, the point
+// left the mask or the last segment hit the boundary (`hit` then names the
+// triangle), the point left the field. seg_* is wave_segment_test's answer.
+template <int DOMAIN, int G>
+__device__ __forceinline__ bool stop_test(const TrackLaunch &p, const Lane<G> &L, bool seg_decided, bool seg_found,
+                                          uint32_t seg_tri, uint32_t &hit)
 {
     bool stop = !(L.n < p.n_points && L.steps < p.max_steps);
-    uint32_t hit = NO_HIT;
     if (!stop) {
         if constexpr (DOMAIN == DOMAIN_MASK) {
             stop = L.mask_value == 0u;
@@ -515,8 +514,19 @@ __device__ __forceinline__ void advance(const TrackLaunch &p, bool shared_affine
             }
         }
     }
-    if (!stop)
-        stop = !L.field_ok;
+    return stop || !L.field_ok;
+}
+
+// nz: this step's Diffusion draws, made by the caller before anything that
+// waits on memory, so they cover the latency of the cell data
+// request_cells asked for.
+template <int MODEL, int ALGO, int DOMAIN, int LMAX, int G, int LDS_VEC, int BLOCK>
+__device__ __forceinline__ void advance(const TrackLaunch &p, bool shared_affine, const float *__restrict__ coeffs,
+                                        uint32_t cstride, Lane<G> &L, float *q, float4 *__restrict__ lds_rows,
+                                        const fast::Noise &nz, bool seg_decided, bool seg_found, uint32_t seg_tri)
+{
+    uint32_t hit = NO_HIT;
+    const bool stop = stop_test<DOMAIN>(p, L, seg_decided, seg_found, seg_tri, hit);
     if (stop) {
         store_held(p, L);
         p.lengths[L.g] = L.n;
@@ -752,6 +762,128 @@ void track_fast_kernel(FastLaunch f)
     __builtin_amdgcn_s_waitcnt(0);
     // The wavefront's memory reads of rows and mask values, one atomic each
     // (the launch's totals price the bytes the cell cache had to fetch).
+    if (lane_id == 0) {
+        atomicAdd(&f.stats[0], (unsigned long long)rows_read);
+        atomicAdd(&f.stats[1], (unsigned long long)masks_read);
+    }
+}
+
+// Streamlines tracked by lane groups: fast::GROUP_LANES lanes hold one
+// streamline's state between them, share out the evaluations of its update
+// and do the rest of the step alike (same data, same arithmetic; the first
+// lane of the group stores). One lane per streamline runs a Probabilistic
+// step's 64 candidates one after another, 38 us of latency, and a launch
+// lasts as long as its longest streamline's steps, mostly with idle lanes:
+// 46 ms for 150k SH45 seeds of 235 steps on average and 1200 at most. Eight
+// lanes take about an eighth of that latency per step, for no more
+// evaluations in all (the one-lane form evaluates a block of candidates
+// twice): 17.4 ms, bound by VALU issue (about 1700 instructions per step of
+// a wavefront's eight streamlines) and by the longest streamlines.
+template <int MODEL, int ALGO, int DOMAIN, int LMAX>
+__global__ __launch_bounds__(256) void track_group_kernel(FastLaunch f)
+{
+    constexpr int W = fast::GROUP_LANES;
+    const TrackLaunch &p = f.track;
+    const int lane_id = __lane_id();
+    const int sub = lane_id % W;
+    const bool leader = sub == 0;
+    const float *coeffs = static_cast<const float *>(f.coeffs);
+    const uint64_t to_lane = f.group_jump[sub], to_end = f.group_jump[W];
+    const float one_minus_cos_max = 1.0f - tgk_cosf(p.algo.max_angle);
+    const float step = p.algo.step_size;
+
+    Lane<1> L;
+    L.g = -1;
+    L.point = L.previous = v3(0.0f, 0.0f, 0.0f);
+    L.steps = 0;
+    L.row_read = false;
+    L.mask_read = false;
+    uint64_t rows_read = 0, masks_read = 0;
+    float q[MODEL == MODEL_SH ? Order<LMAX>::TERMS : 6];
+    bool drained = false;
+
+    while (true) {
+        // Refill idle groups, one atomic per wavefront.
+        const uint64_t need = __ballot(leader && L.g < 0);
+        if (need != 0 && !drained) {
+            const int first = __ffsll((unsigned long long)need) - 1;
+            const uint32_t count = (uint32_t)__popcll(need);
+            uint32_t base = 0;
+            if (lane_id == first)
+                base = atomicAdd(f.claims, count);
+            base = __shfl(base, first);
+            if ((uint64_t)base + count >= (uint64_t)p.n_seeds)
+                drained = true;
+            if (L.g < 0) {
+                const uint64_t g = (uint64_t)base + (uint32_t)__popcll(need & ((1ull << (lane_id - sub)) - 1ull));
+                if (g < (uint64_t)p.n_seeds) {
+                    L.g = (int32_t)g;
+                    const float4 s0 = reinterpret_cast<const float4 *>(p.seeds)[2 * g];
+                    const float4 s1 = reinterpret_cast<const float4 *>(p.seeds)[2 * g + 1];
+                    L.point = v3(s0.x, s0.y, s0.z);
+                    L.o = v3(s1.x, s1.y, s1.z);
+                    L.previous = L.point;
+                    if constexpr (ALGO == ALGO_PROBABILISTIC)
+                        L.rng = seed_stream(p, p.first_seed + L.g);
+                    L.time = 0.0;
+                    L.n = 1;  // the seed is the streamline's first point
+                    L.steps = 0;
+                    if (leader)
+                        store_row(p.points, L.g, p.n_points, 0, L.point);
+                    L.field_cell = UNSET_CELL;
+                    L.mask_cell = UNSET_CELL;
+                    L.mask_value = 0;
+                    L.mesh_cell = UNSET_CELL;
+                    request_cells<MODEL, DOMAIN, LMAX, 1, 0, 256>(p, f.shared_affine != 0, coeffs, f.coeff_stride, L,
+                                                                  q, nullptr);
+                }
+            }
+        }
+        if (__ballot(L.g >= 0) == 0)
+            break;
+        bool seg_decided = false, seg_found = false;
+        uint32_t seg_tri = 0;
+        if constexpr (DOMAIN == DOMAIN_MESH) {
+            // Asked once per group.
+            wave_segment_test<1>(p.mesh, L, leader && L.g >= 0, seg_decided, seg_found, seg_tri);
+            seg_decided = __shfl((int)seg_decided, 0, W) != 0;
+            seg_found = __shfl((int)seg_found, 0, W) != 0;
+            seg_tri = __shfl(seg_tri, 0, W);
+        }
+        if (L.g >= 0) {
+            uint32_t hit = NO_HIT;
+            if (stop_test<DOMAIN>(p, L, seg_decided, seg_found, seg_tri, hit)) {
+                if (leader) {
+                    p.lengths[L.g] = L.n;
+                    p.steps[L.g] = L.steps;
+                    p.hits[L.g] = hit;
+                }
+                L.g = -1;
+            } else {
+                L.o = fast::probabilistic_group<MODEL, LMAX>(p.algo, q, L.o, L.rng, to_lane, to_end,
+                                                            one_minus_cos_max, sub);
+                L.steps++;
+                if constexpr (DOMAIN == DOMAIN_MESH)
+                    L.previous = L.point;
+                L.point = v3(L.point.x + step * L.o.x, L.point.y + step * L.o.y, L.point.z + step * L.o.z);
+                L.time += (double)step;
+                if (L.time >= (double)p.save_at) {
+                    L.time -= (double)p.save_at;
+                    const float t = (float)L.time;
+                    if (leader)
+                        store_row(p.points, L.g, p.n_points, L.n,
+                                  v3(L.point.x - t * L.o.x, L.point.y - t * L.o.y, L.point.z - t * L.o.z));
+                    L.n++;
+                }
+                request_cells<MODEL, DOMAIN, LMAX, 1, 0, 256>(p, f.shared_affine != 0, coeffs, f.coeff_stride, L, q,
+                                                              nullptr);
+            }
+        }
+        rows_read += (uint64_t)__popcll(__ballot(leader && L.row_read));
+        masks_read += (uint64_t)__popcll(__ballot(leader && L.mask_read));
+        L.row_read = false;
+        L.mask_read = false;
+    }
     if (lane_id == 0) {
         atomicAdd(&f.stats[0], (unsigned long long)rows_read);
         atomicAdd(&f.stats[1], (unsigned long long)masks_read);
@@ -1147,11 +1279,12 @@ template <int L> hipError_t device_matrix(const double **out)
     return hipSuccess;
 }
 
-// Blocks that fill the current device once, computed on first use per
-// device (atomically published: runtimes on other threads may read it).
-template <int MODEL, int ALGO, int DOMAIN, int LMAX, int S> hipError_t occupancy_grid(int *blocks)
+// Blocks of `block` threads of a kernel that fill the current device once,
+// and the device's CUs, computed on first use per device (atomically
+// published: runtimes on other threads may read it).
+template <auto KERNEL> hipError_t fill_grid(int block, int *blocks, int *cus = nullptr)
 {
-    static std::atomic<int> cache[64] = {};
+    static std::atomic<uint64_t> cache[64] = {};
     int device = 0;
     hipError_t e = hipGetDevice(&device);
     if (e != hipSuccess)
@@ -1160,19 +1293,80 @@ template <int MODEL, int ALGO, int DOMAIN, int LMAX, int S> hipError_t occupancy
         return hipErrorInvalidDevice;
     if (cache[device].load(std::memory_order_acquire) == 0) {
         int per_cu = 0;
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per_cu, reinterpret_cast<const void *>(track_fast_kernel<MODEL, ALGO, DOMAIN, LMAX, S>),
-            shape_block<MODEL, ALGO, LMAX, S>(), 0);
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(KERNEL), block, 0);
         if (e != hipSuccess)
             return e;
-        hipDeviceProp_t prop;
-        e = hipGetDeviceProperties(&prop, device);
+        int count = 0;
+        e = hipDeviceGetAttribute(&count, hipDeviceAttributeMultiprocessorCount, device);
         if (e != hipSuccess)
             return e;
-        cache[device].store(prop.multiProcessorCount * (per_cu > 0 ? per_cu : 1), std::memory_order_release);
+        count = std::max(count, 1);
+        cache[device].store((uint64_t)count << 32 | (uint32_t)(count * std::max(per_cu, 1)),
+                            std::memory_order_release);
     }
-    *blocks = cache[device].load(std::memory_order_acquire);
+    const uint64_t found = cache[device].load(std::memory_order_acquire);
+    *blocks = (int)(uint32_t)found;
+    if (cus)
+        *cus = (int)(found >> 32);
     return hipSuccess;
+}
+
+// A^k 2^64 mod M for MWC64X (mwc64x_jump).
+uint64_t jump_multiplier(uint64_t k)
+{
+    constexpr uint64_t A = 4294883355u, M = (A << 32) - 1;
+    auto times = [](uint64_t a, uint64_t b) { return (uint64_t)((unsigned __int128)a * b % M); };
+    uint64_t result = (uint64_t)(((unsigned __int128)1 << 64) % M);
+    for (uint64_t power = A; k != 0; k >>= 1, power = times(power, power))
+        if (k & 1)
+            result = times(result, power);
+    return result;
+}
+
+// Whether a launch tracks by lane groups. A group's step costs some 500
+// instructions beside its candidates: with 16 candidates or fewer that shows
+// once the streamlines fill the GPU one to a lane (SH45, 600k seeds, one lane
+// per streamline against groups: 12.2 and 17.2 ms with 8 candidates, 20.7 and
+// 19.9 with 16, 35.3 and 30.7 with 32, 68.9 and 44.8 with 64; 20k seeds: 3.9
+// and 2.7 with 2, 48.2 and 7.5 with 64). Past 64 candidates a lane's share no
+// longer fits its registers.
+constexpr int64_t GROUP_FEW_SEEDS = 65536;
+template <int ALGO> bool grouped(const TrackLaunch &p)
+{
+    if constexpr (ALGO == ALGO_PROBABILISTIC)
+        return p.algo.n_samples <= fast::GROUP_LANES * fast::GROUP_CANDIDATES &&
+               (p.algo.n_samples > 16 || p.n_seeds <= GROUP_FEW_SEEDS);
+    return false;
+}
+
+// The grid: whole blocks per CU, as many as the seeds fill and at most three.
+// A launch ends with its longest streamline, whose steps take longer the more
+// wavefronts share its SIMD, and the queue refills what ends early: 150k
+// seeds of the 97 x 116 x 97 SH45 Probabilistic workload took 22.8, 17.3,
+// 17.4 and 18.4 ms at one to four blocks per CU, 600k seeds 49.6, 45.0 and
+// 45.6 ms at two to four, and 20k seeds (625 blocks' worth) 7.2 ms at two
+// blocks per CU and 9.3 ms at 625 blocks.
+constexpr int GROUP_BLOCKS_PER_CU = 3;
+template <int MODEL, int ALGO, int DOMAIN, int LMAX>
+hipError_t launch_group(const FastLaunch &f, int grid_blocks, bool query, hipStream_t stream)
+{
+    int fill = 0, cus = 0;
+    const hipError_t e = fill_grid<track_group_kernel<MODEL, ALGO, DOMAIN, LMAX>>(256, &fill, &cus);
+    if (e != hipSuccess || query)
+        return e;
+    const int64_t needed = (f.track.n_seeds * fast::GROUP_LANES + 255) / 256;
+    if (grid_blocks <= 0)
+        grid_blocks = (int)std::min<int64_t>(std::min(fill, GROUP_BLOCKS_PER_CU * cus),
+                                             std::max<int64_t>(needed / cus, 1) * cus);
+    FastLaunch g = f;
+    const uint64_t per_lane = ((uint64_t)f.track.algo.n_samples + fast::GROUP_LANES - 1) / fast::GROUP_LANES;
+    for (int b = 0; b < fast::GROUP_LANES; b++)
+        g.group_jump[b] = jump_multiplier(2 * per_lane * b);
+    g.group_jump[fast::GROUP_LANES] = jump_multiplier(2 * (uint64_t)f.track.algo.n_samples);
+    zero_generation<<<1, 64, 0, stream>>>(f.claims, f.ended, f.cont_count[0], f.stats);
+    track_group_kernel<MODEL, ALGO, DOMAIN, LMAX>
+        <<<(unsigned)std::min<int64_t>(grid_blocks, needed), 256, 0, stream>>>(g);
+    return hipGetLastError();
 }
 
 // query: only report the lanes of the grid a launch would use.
@@ -1180,8 +1374,16 @@ template <int MODEL, int ALGO, int DOMAIN, int LMAX, int S>
 hipError_t launch_fast(const FastLaunch &f, int grid_blocks, bool query, int64_t *lanes, hipStream_t stream)
 {
     constexpr int BLOCK = shape_block<MODEL, ALGO, LMAX, S>();
+    if constexpr (ALGO == ALGO_PROBABILISTIC) {
+        // Queried for every launch: a later one may be grouped.
+        if (query || grouped<ALGO>(f.track)) {
+            const hipError_t e = launch_group<MODEL, ALGO, DOMAIN, LMAX>(f, grid_blocks, query, stream);
+            if (e != hipSuccess || !query)
+                return e;
+        }
+    }
     if (grid_blocks <= 0) {
-        const hipError_t e = occupancy_grid<MODEL, ALGO, DOMAIN, LMAX, S>(&grid_blocks);
+        const hipError_t e = fill_grid<track_fast_kernel<MODEL, ALGO, DOMAIN, LMAX, S>>(BLOCK, &grid_blocks);
         if (e != hipSuccess)
             return e;
     }

@@ -483,23 +483,30 @@ __device__ __forceinline__ V3 unit_or_z(V3 o)
     return v3(o.x * inv, o.y * inv, o.z * inv);
 }
 
-// algorithm.py:305-376 (Probabilistic), the plain path's weighted choice
-// (choose_candidate) on the polynomial model: candidates are Cartesian
-// already, so a candidate costs one polynomial and one softplus (hardware
-// exp2/log2), with no cart2sph and no trigonometric basis. The azimuth
-// 2 pi u is handed to the hardware sine and cosine as u revolutions.
-template <int MODEL, int LMAX>
-__device__ __forceinline__ V3 probabilistic(const AlgoParams &a, const float *q, V3 o_in, uint2 &rng)
-{
-    const V3 o = unit_or_z(o_in);
-    const bool z_helper = fabsf(o.z) < 0.9f;
-    // cross(helper, o) for helper e_z or e_y, then normalised.
-    const V3 c = z_helper ? v3(-o.y, o.x, 0.0f) : v3(o.z, 0.0f, -o.x);
-    const float ic = __builtin_amdgcn_rsqf(c.x * c.x + c.y * c.y + c.z * c.z);
-    const V3 t1 = v3(c.x * ic, c.y * ic, c.z * ic);
-    const V3 t2 = v3(o.y * t1.z - o.z * t1.y, o.z * t1.x - o.x * t1.z, o.x * t1.y - o.y * t1.x);
-    const float one_minus_cos_max = 1.0f - tgk_cosf(a.max_angle);
-    auto candidate = [&](uint2 &state) {
+// algorithm.py:305-376 (Probabilistic): candidates uniform on the cap around
+// the orientation o. They are Cartesian already, so a candidate costs one
+// polynomial and one softplus (hardware exp2/log2), with no cart2sph and no
+// trigonometric basis. The azimuth 2 pi u is handed to the hardware sine and
+// cosine as u revolutions.
+template <int MODEL, int LMAX> struct CapSampler {
+    const float *q;
+    V3 o, t1, t2;
+    float one_minus_cos_max;
+
+    __device__ __forceinline__ CapSampler(const float *q_in, V3 o_in, float one_minus_cos_max_in)
+    {
+        q = q_in;
+        one_minus_cos_max = one_minus_cos_max_in;
+        o = unit_or_z(o_in);
+        const bool z_helper = fabsf(o.z) < 0.9f;
+        // cross(helper, o) for helper e_z or e_y, then normalised.
+        const V3 c = z_helper ? v3(-o.y, o.x, 0.0f) : v3(o.z, 0.0f, -o.x);
+        const float ic = __builtin_amdgcn_rsqf(c.x * c.x + c.y * c.y + c.z * c.z);
+        t1 = v3(c.x * ic, c.y * ic, c.z * ic);
+        t2 = v3(o.y * t1.z - o.z * t1.y, o.z * t1.x - o.x * t1.z, o.x * t1.y - o.y * t1.x);
+    }
+    __device__ __forceinline__ V3 candidate(uint2 &state) const
+    {
         const float cos_angle = 1.0f - randu(state) * one_minus_cos_max;
         const float sin_angle = __builtin_sqrtf(fmaxf(0.0f, 1.0f - cos_angle * cos_angle));
         const float turns = randu(state);
@@ -507,13 +514,138 @@ __device__ __forceinline__ V3 probabilistic(const AlgoParams &a, const float *q,
         return v3(cos_angle * o.x + sin_angle * (ca * t1.x + sa * t2.x),
                   cos_angle * o.y + sin_angle * (ca * t1.y + sa * t2.y),
                   cos_angle * o.z + sin_angle * (ca * t1.z + sa * t2.z));
-    };
-    auto weight = [&](V3 c) {
+    }
+    __device__ __forceinline__ float weight(V3 c) const
+    {
         const float v = value_at<MODEL, LMAX>(q, c);
         return __builtin_isfinite(v) ? fmaxf(v, 0.0f) : 0.0f;
-    };
+    }
+};
+
+// One lane per streamline: the plain path's weighted choice.
+template <int MODEL, int LMAX>
+__device__ __forceinline__ V3 probabilistic(const AlgoParams &a, const float *q, V3 o_in, uint2 &rng)
+{
+    const CapSampler<MODEL, LMAX> cap(q, o_in, 1.0f - tgk_cosf(a.max_angle));
     V3 chosen;
-    return choose_candidate(a.n_samples, rng, candidate, weight, chosen) ? chosen : o;
+    return choose_candidate(a.n_samples, rng, [&](uint2 &state) { return cap.candidate(state); },
+                            [&](V3 c) { return cap.weight(c); }, chosen)
+               ? chosen
+               : cap.o;
+}
+
+// The noise state k draws later. A draw takes the state v = c 2^32 + x to
+// v A mod M, M = A 2^32 - 1, so k draws multiply by A^k; `multiplier` is
+// A^k 2^64 mod M (group_jump in tgk_fast.hip). Since 2^32 A = 1 mod M, the
+// 128-bit product is divided by 2^32 by adding A times its low word to the
+// rest, twice. The result is the value in [0, M) that the draws one by one
+// reach; M itself, which they leave in place, is kept.
+__device__ __forceinline__ uint2 mwc64x_jump(uint2 s, uint64_t multiplier)
+{
+    constexpr uint64_t A = 4294883355u, M = (A << 32) - 1;
+    const uint64_t v = (uint64_t)s.y << 32 | s.x;
+    const uint64_t lo = v * multiplier, hi = __umul64hi(v, multiplier);
+    const uint64_t add1 = (uint64_t)(uint32_t)lo * A;
+    const uint64_t t = (hi << 32 | lo >> 32) + add1;
+    const uint64_t t_hi = (hi >> 32) + (t < add1 ? 1u : 0u);
+    const uint64_t add2 = (uint64_t)(uint32_t)t * A;
+    uint64_t r = (t_hi << 32 | t >> 32) + add2;
+    if (r < add2 || r >= M)
+        r -= M;
+    if (v == M)
+        r = M;
+    return make_uint2((uint32_t)r, (uint32_t)(r >> 32));
+}
+
+// Probabilistic with GROUP_LANES lanes per streamline (all of them hold its
+// state and call this together) and at most GROUP_LANES * GROUP_CANDIDATES
+// candidates: lane b of the group draws and weighs candidates [b m, (b + 1) m),
+// m = ceil(n / GROUP_LANES), from the stream jumped ahead to its first. The
+// weights are then added in the one order of the reference: each lane adds
+// its own to the running sum that its left neighbour ends with, GROUP_LANES -
+// 1 times over, after which every lane's start is final. The chosen candidate
+// is drawn again by all lanes. Sums, choice and noise state are the bits of
+// the sequential form, without its second evaluation of a block.
+constexpr int GROUP_LANES = 8;
+constexpr int GROUP_CANDIDATES = 8;
+
+// Weights of a lane's `mine` candidates from its stream, 0 (which changes no
+// sum) past them; per_lane, the most any lane has, is the same for all. A
+// list of single floats and not an array, which the compiler would keep as
+// one vector and copy whole around every candidate's branch.
+template <int N> struct GroupWeights {
+    float head;
+    GroupWeights<N - 1> tail;
+
+    template <class Cap> __device__ __forceinline__ void fill(const Cap &cap, int per_lane, int mine, uint2 &state)
+    {
+        head = 0.0f;
+        if (per_lane > 0) {
+            const float weight = cap.weight(cap.candidate(state));
+            head = mine > 0 ? weight : 0.0f;
+        }
+        tail.fill(cap, per_lane - 1, mine - 1, state);
+    }
+    // `sum` and the weights, added one after another.
+    __device__ __forceinline__ float add_to(float sum) const { return tail.add_to(sum + head); }
+    // The first weight with which the sum exceeds `target`: its index from
+    // k on, or GROUP_CANDIDATES.
+    __device__ __forceinline__ int crossing(float sum, float target, int k) const
+    {
+        sum += head;
+        const int later = tail.crossing(sum, target, k + 1);
+        return sum > target ? k : later;
+    }
+};
+template <> struct GroupWeights<0> {
+    template <class Cap> __device__ __forceinline__ void fill(const Cap &, int, int, uint2 &) {}
+    __device__ __forceinline__ float add_to(float sum) const { return sum; }
+    __device__ __forceinline__ int crossing(float, float, int k) const { return k; }
+};
+
+// to_lane and to_end: mwc64x_jump multipliers to the lane's first candidate
+// and past the last one.
+template <int MODEL, int LMAX>
+__device__ __forceinline__ V3 probabilistic_group(const AlgoParams &a, const float *q, V3 o_in, uint2 &rng,
+                                                  uint64_t to_lane, uint64_t to_end, float one_minus_cos_max, int sub)
+{
+    const CapSampler<MODEL, LMAX> cap(q, o_in, one_minus_cos_max);
+    const int n = a.n_samples;
+    const int per_lane = (n + GROUP_LANES - 1) / GROUP_LANES;
+    const uint2 start = mwc64x_jump(rng, to_lane);
+    uint2 state = start;
+    GroupWeights<GROUP_CANDIDATES> w;
+    w.fill(cap, per_lane, min(per_lane, n - sub * per_lane), state);
+    float before = 0.0f, sum = 0.0f;
+#pragma unroll
+    for (int pass = 0; pass < GROUP_LANES; pass++) {
+        sum = w.add_to(before);
+        if (pass + 1 < GROUP_LANES) {
+            // From the lane to the left (row_shr:1; a group is half a row).
+            const float left = __int_as_float(
+                __builtin_amdgcn_update_dpp(0, __float_as_int(sum), 0x111, 0xf, 0xf, true));
+            before = sub == 0 ? 0.0f : left;
+        }
+    }
+    const float total = __shfl(sum, GROUP_LANES - 1, GROUP_LANES);
+    rng = mwc64x_jump(rng, to_end);
+    if (!(total > 0.0f))
+        return cap.o;
+    uint2 target_state = rng;
+    const float target = randu(target_state) * total;
+    const int crossing = w.crossing(before, target, 0);
+    const uint64_t crossed = __ballot(crossing < GROUP_CANDIDATES) >> (__lane_id() - sub);
+    const int owner = __ffs((int)(crossed & ((1u << GROUP_LANES) - 1u))) - 1;
+    if (owner < 0)
+        return cap.o;
+    const int k = __shfl(crossing, owner, GROUP_LANES);
+    uint2 replay = make_uint2((uint32_t)__shfl((int)start.x, owner, GROUP_LANES),
+                              (uint32_t)__shfl((int)start.y, owner, GROUP_LANES));
+    for (int i = 0; i < 2 * k; i++)
+        mwc64x(replay);
+    const V3 chosen = cap.candidate(replay);
+    rng = replay;
+    return chosen;
 }
 
 // Gradient on the sphere: dtheta e_theta + (dphi / sin theta) e_phi, from

@@ -127,6 +127,7 @@ struct FastLaunch {
     uint32_t coeff_stride;      // elements per voxel in `coeffs`
     int32_t sh_order;           // 8 (K <= 45) or 12 (K <= 91): polynomial layout of `coeffs`
     int32_t shape;              // launch shape, 0..FAST_SHAPE_COUNT - 1
+    uint64_t group_jump[9];     // lane-group kernels: noise-stream multipliers to lane b's first draw and, last, past all
 };
 // grid_blocks <= 0 sizes the persistent grid to the device's occupancy
 // (computed once per kernel and device, then cached). n_seeds must be below
