@@ -67,3 +67,24 @@ def test_probabilistic_groups_follow_the_fp64_oracle(fast_runtime, n_samples, or
     r = deviation.report(fast.lengths, fast.steps, fast.points, ref, jump=1e-2)
     assert r["max_deviation"] <= 1e-3
     assert r["compared_fraction"] > 0.5
+
+
+@pytest.mark.parametrize("n", [1, 9, 300])
+@pytest.mark.parametrize("options", [{}, {"max_iterations": 0}, {"max_iterations": 1}, {"tolerance": 0.02},
+                                     {"max_step_size": 0.05}])
+def test_deterministic_groups_follow_the_fp64_oracle(fast_runtime, runtime, options, n, oracle_threads):
+    # Updates that end before, in and after the first iteration, next to one
+    # another in a wavefront; held to twice the plain path's own FP32
+    # deviation, as the Deterministic path's own test.
+    cfg = bench.brain145_diffusion(seed=1, n_seeds=n, shape=(49, 58, 49))
+    field = tg.field.Image(tg.Nifti1Image(cfg["fod"], np.eye(4)))
+    domain = tg.domain.Image(tg.Nifti1Image(cfg["mask"], np.eye(4)))
+    algorithm = tg.algorithm.Deterministic(tg.local.RealSymmetricSphericalHarmonics(45), step_size=0.1, **options)
+    args = (cfg["seeds"], [0], n, 0.25, 30.0)
+    ref = oracle.track(domain, field, algorithm, *args, precision=64, threads=oracle_threads)
+    fast = tg.tracking.track(algorithm, domain, field, *args, fast_runtime)
+    plain = tg.tracking.track(algorithm, domain, field, *args, runtime)
+    rf = deviation.report(fast.lengths, fast.steps, fast.points, ref, jump=1e-2)
+    rp = deviation.report(plain.lengths, plain.steps, plain.points, ref, jump=1e-2)
+    assert rf["max_deviation"] <= max(1e-3, 2.0 * rp["max_deviation"])
+    assert rf["compared_fraction"] > 0.8 * rp["compared_fraction"]

@@ -772,13 +772,17 @@ void track_fast_kernel(FastLaunch f)
 // streamline's state between them, share out the evaluations of its update
 // and do the rest of the step alike (same data, same arithmetic; the first
 // lane of the group stores). One lane per streamline runs a Probabilistic
-// step's 64 candidates one after another, 38 us of latency, and a launch
-// lasts as long as its longest streamline's steps, mostly with idle lanes:
-// 46 ms for 150k SH45 seeds of 235 steps on average and 1200 at most. Eight
-// lanes take about an eighth of that latency per step, for no more
-// evaluations in all (the one-lane form evaluates a block of candidates
-// twice): 17.4 ms, bound by VALU issue (about 1700 instructions per step of
-// a wavefront's eight streamlines) and by the longest streamlines.
+// step's 64 candidates one after another, 38 us of latency, and a
+// Deterministic wavefront its slowest lane's iterations and line search, 70
+// us, and a launch lasts as long as its longest streamline's steps, mostly
+// with idle lanes: 46 ms for 150k SH45 Probabilistic seeds of 235 steps on
+// average and 1200 at most, 206 ms for 100k Deterministic ones of 850 steps
+// and 3000 at most. Eight lanes take about an eighth of that latency per
+// step, for no more evaluations in all (the one-lane Probabilistic form
+// evaluates a block of candidates twice, the Deterministic one waits for its
+// wavefront): 16.1 and 32.4 ms, bound by VALU issue (about 1700 instructions
+// per Probabilistic step of a wavefront's eight streamlines, 950 per
+// Deterministic iteration) and by the longest streamlines.
 template <int MODEL, int ALGO, int DOMAIN, int LMAX>
 __global__ __launch_bounds__(256) void track_group_kernel(FastLaunch f)
 {
@@ -801,6 +805,11 @@ __global__ __launch_bounds__(256) void track_group_kernel(FastLaunch f)
     uint64_t rows_read = 0, masks_read = 0;
     float q[MODEL == MODEL_SH ? Order<LMAX>::TERMS : 6];
     bool drained = false;
+    // Iterations the current update has done; -1: the next step begins.
+    // A pass of the loop does one (a Probabilistic update is one), so that
+    // groups whose updates take few go on to their next step while others
+    // still iterate.
+    int iteration = -1;
 
     while (true) {
         // Refill idle groups, one atomic per wavefront.
@@ -841,16 +850,17 @@ __global__ __launch_bounds__(256) void track_group_kernel(FastLaunch f)
         }
         if (__ballot(L.g >= 0) == 0)
             break;
+        const bool starting = L.g >= 0 && iteration < 0;
         bool seg_decided = false, seg_found = false;
         uint32_t seg_tri = 0;
         if constexpr (DOMAIN == DOMAIN_MESH) {
             // Asked once per group.
-            wave_segment_test<1>(p.mesh, L, leader && L.g >= 0, seg_decided, seg_found, seg_tri);
+            wave_segment_test<1>(p.mesh, L, leader && starting, seg_decided, seg_found, seg_tri);
             seg_decided = __shfl((int)seg_decided, 0, W) != 0;
             seg_found = __shfl((int)seg_found, 0, W) != 0;
             seg_tri = __shfl(seg_tri, 0, W);
         }
-        if (L.g >= 0) {
+        if (starting) {
             uint32_t hit = NO_HIT;
             if (stop_test<DOMAIN>(p, L, seg_decided, seg_found, seg_tri, hit)) {
                 if (leader) {
@@ -860,8 +870,22 @@ __global__ __launch_bounds__(256) void track_group_kernel(FastLaunch f)
                 }
                 L.g = -1;
             } else {
+                iteration = 0;
+                if constexpr (ALGO == ALGO_DETERMINISTIC)
+                    L.o = fast::deterministic_start(L.o);
+            }
+        }
+        if (L.g >= 0) {
+            bool more = false;
+            if constexpr (ALGO == ALGO_PROBABILISTIC)
                 L.o = fast::probabilistic_group<MODEL, LMAX>(p.algo, q, L.o, L.rng, to_lane, to_end,
                                                             one_minus_cos_max, sub);
+            else if (iteration < p.algo.max_iterations)
+                more = fast::deterministic_iteration<MODEL, LMAX>(p.algo, q, L.o, sub) &&
+                       iteration + 1 < p.algo.max_iterations;
+            iteration++;
+            if (!more) {
+                iteration = -1;
                 L.steps++;
                 if constexpr (DOMAIN == DOMAIN_MESH)
                     L.previous = L.point;
@@ -879,10 +903,14 @@ __global__ __launch_bounds__(256) void track_group_kernel(FastLaunch f)
                                                               nullptr);
             }
         }
-        rows_read += (uint64_t)__popcll(__ballot(leader && L.row_read));
-        masks_read += (uint64_t)__popcll(__ballot(leader && L.mask_read));
-        L.row_read = false;
-        L.mask_read = false;
+        // Counted once per step, as one lane per streamline counts them.
+        const bool ended = iteration < 0;
+        rows_read += (uint64_t)__popcll(__ballot(leader && ended && L.row_read));
+        masks_read += (uint64_t)__popcll(__ballot(leader && ended && L.mask_read));
+        if (ended) {
+            L.row_read = false;
+            L.mask_read = false;
+        }
     }
     if (lane_id == 0) {
         atomicAdd(&f.stats[0], (unsigned long long)rows_read);
@@ -1323,30 +1351,41 @@ uint64_t jump_multiplier(uint64_t k)
     return result;
 }
 
-// Whether a launch tracks by lane groups. A group's step costs some 500
-// instructions beside its candidates: with 16 candidates or fewer that shows
-// once the streamlines fill the GPU one to a lane (SH45, 600k seeds, one lane
-// per streamline against groups: 12.2 and 17.2 ms with 8 candidates, 20.7 and
-// 19.9 with 16, 35.3 and 30.7 with 32, 68.9 and 44.8 with 64; 20k seeds: 3.9
-// and 2.7 with 2, 48.2 and 7.5 with 64). Past 64 candidates a lane's share no
-// longer fits its registers.
+// Whether a launch tracks by lane groups. Probabilistic: a group's step costs
+// some 500 instructions beside its candidates: with 16 candidates or fewer
+// that shows once the streamlines fill the GPU one to a lane (SH45, 600k
+// seeds, one lane per streamline against groups: 12.2 and 17.2 ms with 8
+// candidates, 20.7 and 19.9 with 16, 35.3 and 30.7 with 32, 68.9 and 44.8
+// with 64; 20k seeds: 3.9 and 2.7 with 2, 48.2 and 7.5 with 64). Past 64
+// candidates a lane's share no longer fits its registers.
+// Deterministic: every launch of the order-8 SH model (5k, 100k, 600k and
+// 1.5M seeds: 162, 206, 339 and 648 ms one lane per streamline, 13, 32, 113
+// and 257 ms by groups). Order 12 and DTI keep one lane per streamline: their
+// gradients are contracted otherwise (deterministic_iteration), and the DTI
+// evaluations are too short to share out (600k seeds: 47 against 64 ms).
 constexpr int64_t GROUP_FEW_SEEDS = 65536;
+template <int MODEL, int ALGO, int LMAX> constexpr bool groupable()
+{
+    return ALGO == ALGO_PROBABILISTIC || (ALGO == ALGO_DETERMINISTIC && MODEL == MODEL_SH && LMAX == 8);
+}
 template <int ALGO> bool grouped(const TrackLaunch &p)
 {
-    if constexpr (ALGO == ALGO_PROBABILISTIC)
+    if (ALGO == ALGO_PROBABILISTIC)
         return p.algo.n_samples <= fast::GROUP_LANES * fast::GROUP_CANDIDATES &&
                (p.algo.n_samples > 16 || p.n_seeds <= GROUP_FEW_SEEDS);
-    return false;
+    return true;
 }
 
-// The grid: whole blocks per CU, as many as the seeds fill and at most three.
-// A launch ends with its longest streamline, whose steps take longer the more
-// wavefronts share its SIMD, and the queue refills what ends early: 150k
-// seeds of the 97 x 116 x 97 SH45 Probabilistic workload took 22.8, 17.3,
-// 17.4 and 18.4 ms at one to four blocks per CU, 600k seeds 49.6, 45.0 and
-// 45.6 ms at two to four, and 20k seeds (625 blocks' worth) 7.2 ms at two
-// blocks per CU and 9.3 ms at 625 blocks.
-constexpr int GROUP_BLOCKS_PER_CU = 3;
+// The grid: whole blocks per CU, as many as the seeds fill and at most three
+// (Probabilistic) or what fits, four (Deterministic). A launch ends with its
+// longest streamline, whose steps take longer the more wavefronts share its
+// SIMD, and the queue refills what ends early: 150k seeds of the 97 x 116 x
+// 97 SH45 Probabilistic workload took 22.8, 17.3, 17.4 and 18.4 ms at one to
+// four blocks per CU, 600k seeds 49.6, 45.0 and 45.6 ms at two to four, and
+// 20k seeds (625 blocks' worth) 7.2 ms at two blocks per CU and 9.3 ms at 625
+// blocks; Deterministic 50.6, 35.3, 32.4 and 32.9 ms with 100k seeds and 261,
+// 154, 124 and 113 ms with 600k.
+template <int ALGO> constexpr int group_blocks_per_cu() { return ALGO == ALGO_DETERMINISTIC ? 4 : 3; }
 template <int MODEL, int ALGO, int DOMAIN, int LMAX>
 hipError_t launch_group(const FastLaunch &f, int grid_blocks, bool query, hipStream_t stream)
 {
@@ -1356,13 +1395,15 @@ hipError_t launch_group(const FastLaunch &f, int grid_blocks, bool query, hipStr
         return e;
     const int64_t needed = (f.track.n_seeds * fast::GROUP_LANES + 255) / 256;
     if (grid_blocks <= 0)
-        grid_blocks = (int)std::min<int64_t>(std::min(fill, GROUP_BLOCKS_PER_CU * cus),
+        grid_blocks = (int)std::min<int64_t>(std::min(fill, group_blocks_per_cu<ALGO>() * cus),
                                              std::max<int64_t>(needed / cus, 1) * cus);
     FastLaunch g = f;
-    const uint64_t per_lane = ((uint64_t)f.track.algo.n_samples + fast::GROUP_LANES - 1) / fast::GROUP_LANES;
-    for (int b = 0; b < fast::GROUP_LANES; b++)
-        g.group_jump[b] = jump_multiplier(2 * per_lane * b);
-    g.group_jump[fast::GROUP_LANES] = jump_multiplier(2 * (uint64_t)f.track.algo.n_samples);
+    if (ALGO == ALGO_PROBABILISTIC) {
+        const uint64_t per_lane = ((uint64_t)f.track.algo.n_samples + fast::GROUP_LANES - 1) / fast::GROUP_LANES;
+        for (int b = 0; b < fast::GROUP_LANES; b++)
+            g.group_jump[b] = jump_multiplier(2 * per_lane * b);
+        g.group_jump[fast::GROUP_LANES] = jump_multiplier(2 * (uint64_t)f.track.algo.n_samples);
+    }
     zero_generation<<<1, 64, 0, stream>>>(f.claims, f.ended, f.cont_count[0], f.stats);
     track_group_kernel<MODEL, ALGO, DOMAIN, LMAX>
         <<<(unsigned)std::min<int64_t>(grid_blocks, needed), 256, 0, stream>>>(g);
@@ -1374,14 +1415,6 @@ template <int MODEL, int ALGO, int DOMAIN, int LMAX, int S>
 hipError_t launch_fast(const FastLaunch &f, int grid_blocks, bool query, int64_t *lanes, hipStream_t stream)
 {
     constexpr int BLOCK = shape_block<MODEL, ALGO, LMAX, S>();
-    if constexpr (ALGO == ALGO_PROBABILISTIC) {
-        // Queried for every launch: a later one may be grouped.
-        if (query || grouped<ALGO>(f.track)) {
-            const hipError_t e = launch_group<MODEL, ALGO, DOMAIN, LMAX>(f, grid_blocks, query, stream);
-            if (e != hipSuccess || !query)
-                return e;
-        }
-    }
     if (grid_blocks <= 0) {
         const hipError_t e = fill_grid<track_fast_kernel<MODEL, ALGO, DOMAIN, LMAX, S>>(BLOCK, &grid_blocks);
         if (e != hipSuccess)
@@ -1412,23 +1445,44 @@ hipError_t launch_fast(const FastLaunch &f, int grid_blocks, bool query, int64_t
     return hipGetLastError();
 }
 
+// By lane groups where they track, else one lane per streamline.
+template <int MODEL, int ALGO, int DOMAIN, int LMAX, int S>
+hipError_t launch_tracks(const FastLaunch &f, int grid, bool query, int64_t *lanes, hipStream_t stream)
+{
+    if constexpr (groupable<MODEL, ALGO, LMAX>()) {
+        // Queried for every launch: a later one may be grouped.
+        if (query || grouped<ALGO>(f.track)) {
+            const hipError_t e = launch_group<MODEL, ALGO, DOMAIN, LMAX>(f, grid, query, stream);
+            if (e != hipSuccess || !query)
+                return e;
+        }
+        if constexpr (ALGO == ALGO_DETERMINISTIC) {
+            if (lanes)
+                *lanes = 0;  // groups save no streamlines
+            return hipSuccess;
+        }
+    }
+    if constexpr (!groupable<MODEL, ALGO, LMAX>() || ALGO != ALGO_DETERMINISTIC)
+        return launch_fast<MODEL, ALGO, DOMAIN, LMAX, S>(f, grid, query, lanes, stream);
+}
+
 template <int MODEL, int ALGO, int DOMAIN>
 hipError_t launch_fast_order(const FastLaunch &f, int grid, bool query, int64_t *lanes, hipStream_t stream)
 {
     if constexpr (MODEL == MODEL_SH) {
         if (f.sh_order == 12)
-            return launch_fast<MODEL, ALGO, DOMAIN, 12, 0>(f, grid, query, lanes, stream);
+            return launch_tracks<MODEL, ALGO, DOMAIN, 12, 0>(f, grid, query, lanes, stream);
     }
     if constexpr (shaped<MODEL, ALGO, 8>()) {
         switch (f.shape) {
-        case 1: return launch_fast<MODEL, ALGO, DOMAIN, 8, 1>(f, grid, query, lanes, stream);
-        case 2: return launch_fast<MODEL, ALGO, DOMAIN, 8, 2>(f, grid, query, lanes, stream);
-        case 3: return launch_fast<MODEL, ALGO, DOMAIN, 8, 3>(f, grid, query, lanes, stream);
-        case 4: return launch_fast<MODEL, ALGO, DOMAIN, 8, 4>(f, grid, query, lanes, stream);
+        case 1: return launch_tracks<MODEL, ALGO, DOMAIN, 8, 1>(f, grid, query, lanes, stream);
+        case 2: return launch_tracks<MODEL, ALGO, DOMAIN, 8, 2>(f, grid, query, lanes, stream);
+        case 3: return launch_tracks<MODEL, ALGO, DOMAIN, 8, 3>(f, grid, query, lanes, stream);
+        case 4: return launch_tracks<MODEL, ALGO, DOMAIN, 8, 4>(f, grid, query, lanes, stream);
         default: break;
         }
     }
-    return launch_fast<MODEL, ALGO, DOMAIN, 8, 0>(f, grid, query, lanes, stream);
+    return launch_tracks<MODEL, ALGO, DOMAIN, 8, 0>(f, grid, query, lanes, stream);
 }
 
 template <int MODEL, int ALGO>

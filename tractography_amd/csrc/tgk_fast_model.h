@@ -728,6 +728,144 @@ __device__ __forceinline__ V3 deterministic(const AlgoParams &a, const float *q,
     return o;
 }
 
+// ---- Deterministic on lane groups ----
+//
+// The one-lane form above is compiled with cross-statement contraction, so
+// which product of a sum is rounded before it is added was the compiler's
+// choice there. Here the choices it made in the tracking kernels are written
+// out (fmaf; the rest contracts per expression), so that a group follows the
+// same tracks bit for bit.
+
+template <int L, int M>
+__device__ __forceinline__ void sh_order_terms_fused(const float *q, float z, float w, float s, float u1r, float u1i,
+                                                     Powers &pw, Raw &r)
+{
+    if constexpr (M <= L) {
+        using O = Order<L>;
+        if constexpr (M > 1) {
+            const float nvr = pw.vr * u1r - pw.vi * u1i;
+            pw.vi = M == 2 ? __builtin_fmaf(pw.vi, u1r, pw.vr * u1i) : __builtin_fmaf(pw.vr, u1i, pw.vi * u1r);
+            pw.vr = nvr;
+        }
+        const float nur = pw.ur * u1r - pw.ui * u1i;
+        pw.ui = M <= 2 ? __builtin_fmaf(pw.ui, u1r, pw.ur * u1i) : __builtin_fmaf(pw.ur, u1i, pw.ui * u1r);
+        pw.ur = nur;
+        float a, ad, b, bd;
+        poly_m<M, O::poly_terms(M)>(q + O::a_offset(M), z, w, a, ad);
+        poly_m<M, O::poly_terms(M)>(q + O::b_offset(M), z, w, b, bd);
+        const float du = M == 1 ? __builtin_fmaf(bd, pw.ui, ad * pw.ur) : __builtin_fmaf(ad, pw.ur, bd * pw.ui);
+        const float turn = (float)M * z * (a * pw.vr + b * pw.vi) - s * du;
+        if constexpr (M == 1) {
+            r.value += __builtin_fmaf(b, pw.ui, a * pw.ur);
+            r.dtheta = __builtin_fmaf(-s, r.dtheta, turn);  // dtheta holds A_0' so far
+        } else {
+            r.value += a * pw.ur + b * pw.ui;
+            r.dtheta += turn;
+        }
+        r.dphi += (float)M * (b * pw.vr - a * pw.vi);
+        sh_order_terms_fused<L, M + 1>(q, z, w, s, u1r, u1i, pw, r);
+    }
+}
+
+template <int MODEL, int LMAX>
+__device__ __forceinline__ ModelOut model_at_fused(const float *q, V3 c, const Direction &dir)
+{
+    if constexpr (MODEL == MODEL_SH) {
+        using O = Order<LMAX>;
+        const float z = dir.z, s = dir.s, w = z * z;
+        Raw raw;
+        poly_m<0, O::poly_terms(0)>(q + O::a_offset(0), z, w, raw.value, raw.dtheta);
+        raw.dphi = 0.0f;
+        Powers pw{1.0f, 0.0f, dir.c1, dir.s1};
+        sh_order_terms_fused<LMAX, 1>(q, z, w, s, s * dir.c1, s * dir.s1, pw, raw);
+        ModelOut m;
+        float d;
+        softplus(raw.value, m.value, d);
+        m.dtheta = raw.dtheta * d;
+        m.dphi = raw.dphi * d;
+        return m;
+    } else {
+        return dti_model(q, c, dir);
+    }
+}
+
+// Deterministic with GROUP_LANES lanes per streamline (all of them hold its
+// state and call this together): where the update's iterations start, and one
+// iteration, false when the update ends with `o` as it is. The model
+// evaluations of an iteration are independent: lane 0 takes the point itself,
+// lanes 1 to 4 the four offsets of the central differences, and the eight
+// step lengths of the line search go to one lane each; the longest accepted
+// one, the first that the sequential search would accept, wins. The rest is
+// computed alike by all lanes.
+__device__ __forceinline__ V3 deterministic_start(V3 o)
+{
+    const float n2 = o.x * o.x + o.y * o.y + o.z * o.z;
+    const float inv = __builtin_amdgcn_rsqf(n2);
+    return v3(o.x * inv, o.y * inv, o.z * inv);
+}
+
+template <int MODEL, int LMAX>
+__device__ __forceinline__ bool deterministic_iteration(const AlgoParams &a, const float *q, V3 &o, int sub)
+{
+    const float h = 1e-2f, inv_2h = 50.0f;
+    const float side = sub == 2 || sub == 4 ? -h : h;
+    const float length = __uint_as_float((127u - (uint32_t)sub) << 23);  // 2^-sub
+    auto from = [](float v, int lane) { return __shfl(v, lane, GROUP_LANES); };
+    const Direction d = direction_of(o);
+    const V3 e1 = v3(d.z * d.c1, d.z * d.s1, -d.s);
+    const V3 e = sub <= 2 ? e1 : v3(-d.s1, d.c1, 0.0f);
+    const V3 offset = exps2(o, v3(side * e.x, side * e.y, side * e.z));
+    const V3 p = sub == 0 ? o : offset;
+    const Direction dp = direction_of(p);
+    const ModelOut m = model_at_fused<MODEL, LMAX>(q, p, dp);
+    const float gx = m.dtheta * (dp.z * dp.c1) - m.dphi * dp.s1;
+    const float gy = m.dtheta * (dp.z * dp.s1) + m.dphi * dp.c1;
+    const float f0 = from(m.value, 0), g1 = from(m.dtheta, 0), g2 = from(m.dphi, 0);
+    const float gradient_norm = __builtin_sqrtf(g1 * g1 + g2 * g2);
+    if (gradient_norm <= a.tolerance)
+        return false;
+    // Gradient differences along e1 (lanes 1, 2) and e2 (lanes 3, 4);
+    // the z component of a gradient is -dtheta s.
+    const V3 dg1 = v3(from(gx, 1) - from(gx, 2), from(gy, 1) - from(gy, 2),
+                      __builtin_fmaf(from(dp.s, 2), from(m.dtheta, 2), -(from(dp.s, 1) * from(m.dtheta, 1))));
+    const V3 dg2 = v3(from(gx, 3) - from(gx, 4), from(gy, 3) - from(gy, 4),
+                      __builtin_fmaf(from(dp.s, 4), from(m.dtheta, 4), -(from(dp.s, 3) * from(m.dtheta, 3))));
+    const float h11 = (dg1.x * e1.x + dg1.y * e1.y + dg1.z * e1.z) * inv_2h;
+    const float h22 = __builtin_fmaf(dg2.y, d.c1, -(dg2.x * d.s1)) * inv_2h;
+    const float cross = (dg2.x * e1.x + dg2.y * e1.y + dg2.z * e1.z) +
+                        __builtin_fmaf(dg1.y, d.c1, -(dg1.x * d.s1));
+    const float h12 = 0.5f * cross * inv_2h;
+    const float determinant = h11 * h22 - h12 * h12;
+    float d1, d2;
+    if (h11 < -1e-7f && h22 < -1e-7f && determinant > 1e-12f) {
+        const float r = __builtin_amdgcn_rcpf(determinant);
+        d1 = __builtin_fmaf(h12, g2, -(h22 * g1)) * r;
+        d2 = (h12 * g1 - h11 * g2) * r;
+    } else {
+        const float r = 0.1f * __builtin_amdgcn_rcpf(gradient_norm);
+        d1 = g1 * r;
+        d2 = g2 * r;
+    }
+    float step_norm = __builtin_sqrtf(__builtin_fmaf(d2, d2, d1 * d1));
+    if (step_norm > a.max_step_size) {
+        const float scale = a.max_step_size / step_norm;
+        d1 *= scale;
+        d2 *= scale;
+        step_norm = __builtin_sqrtf(__builtin_fmaf(d2, d2, d1 * d1));
+    }
+    if (step_norm <= 1e-7f)
+        return false;
+    const V3 tangent = v3(d1 * e1.x - d2 * d.s1, __builtin_fmaf(d2, d.c1, d1 * e1.y), d1 * e1.z);
+    const V3 c = exps2(o, v3(length * tangent.x, length * tangent.y, length * tangent.z));
+    const bool gain = value_at<MODEL, LMAX>(q, c) > f0 + 1e-7f;
+    const uint64_t gains = __ballot(gain) >> (__lane_id() - sub);
+    const int winner = __ffs((int)(gains & ((1u << GROUP_LANES) - 1u))) - 1;
+    if (winner < 0)
+        return false;
+    o = v3(from(c.x, winner), from(c.y, winner), from(c.z, winner));
+    return true;
+}
+
 // The reference's 45-term real symmetric SH basis (order 8, MRtrix order:
 // index l(l+1)/2 + m for even l; spharm.cl:10-207, core.py:36-69) at the
 // direction of o, without angles. With z = cos(theta) and u = (x + iy) / r =
