@@ -176,14 +176,14 @@ __global__ void math_kernel(int fn, const float *__restrict__ x, const float *__
     if (g >= n)
         return;
     const float a = x[g];
-    float r;
+    float r, other;
     switch (fn) {
-    case 0: r = tgk_sinf(a); break;
-    case 1: r = tgk_cosf(a); break;
-    case 2: r = tgk_atan2f(a, y[g]); break;
-    case 3: r = tgk_acosf(a); break;
-    case 4: r = tgk_expf(a); break;
-    case 5: r = tgk_logf(a); break;
+    case 0: dm::sincosf(a, &r, &other); break;
+    case 1: dm::sincosf(a, &other, &r); break;
+    case 2: r = dm::atan2f(a, y[g]); break;
+    case 3: r = dm::acosf(a); break;
+    case 4: r = dm::expf(a); break;
+    case 5: r = dm::logf(a); break;
     case 6: r = tgk_sqrtf(a); break;
     default: r = a / y[g]; break;
     }

@@ -10,6 +10,7 @@
 #include <type_traits>
 
 #include "tgk_device.h"
+#include "tgk_math_device.h"
 
 namespace tgk {
 namespace plain {
@@ -22,33 +23,34 @@ struct ModelValue {
 __device__ __forceinline__ void cart2sph(V3 c, float &azimuth, float &colatitude)
 {
     const float radius = length3(c);
-    if (radius <= 0.0f) {
-        azimuth = 0.0f;
-        colatitude = 0.0f;
-        return;
-    }
-    float az = tgk_atan2f(c.y, c.x);
-    if (az < 0.0f)
-        az += 2.0f * 3.14159265359f;
-    azimuth = az;
-    colatitude = tgk_acosf(fminf(fmaxf(c.z / radius, -1.0f), 1.0f));
+    const bool zero = radius <= 0.0f;
+    const float az = dm::atan2f(c.y, c.x);
+    const float turned = az < 0.0f ? az + 2.0f * 3.14159265359f : az;
+    const float col = dm::acosf(fminf(fmaxf(c.z / radius, -1.0f), 1.0f));
+    azimuth = zero ? 0.0f : turned;
+    colatitude = zero ? 0.0f : col;
 }
 
 // core.cl:101-109
 __device__ __forceinline__ V3 exps2(V3 p, V3 x)
 {
     const float n = length3(x);
-    if (n <= 0.0f)
-        return p;
+    const bool zero = n <= 0.0f;
     float s, c;
-    tgk_sincosf(n, &s, &c);
+    dm::sincosf(n, &s, &c);
     const float q = s / n;
-    return v3(c * p.x + x.x * q, c * p.y + x.y * q, c * p.z + x.z * q);
+    const V3 r = v3(c * p.x + x.x * q, c * p.y + x.y * q, c * p.z + x.z * q);
+    return v3(zero ? p.x : r.x, zero ? p.y : r.y, zero ? p.z : r.z);
 }
 
 // core.cl:111-120, k = 100
-__device__ __forceinline__ float softplus(float x) { return x * 100.0f < 30.0f ? tgk_logf(1.0f + tgk_expf(100.0f * x)) / 100.0f : x; }
-__device__ __forceinline__ float dsoftplus(float x) { return 1.0f / (1.0f + tgk_expf(-100.0f * x)); }
+__device__ __forceinline__ float softplus(float x)
+{
+    // The logarithm's argument is at least 1, and finite where it is taken.
+    const float soft = dm::logf_normal(1.0f + dm::expf(100.0f * x)) / 100.0f;
+    return x * 100.0f < 30.0f ? soft : x;
+}
+__device__ __forceinline__ float dsoftplus(float x) { return 1.0f / (1.0f + dm::expf(-100.0f * x)); }
 
 // core.cl:240-245
 __device__ __forceinline__ float randn(uint2 &s)
@@ -56,7 +58,8 @@ __device__ __forceinline__ float randn(uint2 &s)
     float n = randu(s);
     while (n <= 0.0f)
         n = randu(s);
-    return tgk_sqrtf(-2.0f * tgk_logf(n)) * tgk_cosf((2.0f * 3.14159265359f) * randu(s));
+    // n is a positive multiple of 2^-24.
+    return tgk_sqrtf(-2.0f * dm::logf_normal(n)) * dm::cosf_small((2.0f * 3.14159265359f) * randu(s));
 }
 
 // SH model contraction (local.py:91-120): value, d/dtheta and
@@ -183,8 +186,8 @@ __device__ __forceinline__ ModelValue dti_model(const float *__restrict__ row, V
     const float t2 = (m4 * o.x + m5 * o.y) + m2 * o.z;
     float az, col, sp, cp, st, ct;
     cart2sph(o, az, col);
-    tgk_sincosf(az, &sp, &cp);
-    tgk_sincosf(col, &st, &ct);
+    dm::sincosf_small(az, &sp, &cp);
+    dm::sincosf_small(col, &st, &ct);
     const float etx = ct * cp, ety = ct * sp, etz = -st;
     const float epx = -sp, epy = cp, epz = 0.0f;
     ModelValue r;
@@ -255,8 +258,8 @@ struct VoxelModel {
             const float t2 = (c[4] * o.x + c[5] * o.y) + c[2] * o.z;
             float az, col, sp, cp, st, ct;
             cart2sph(o, az, col);
-            tgk_sincosf(az, &sp, &cp);
-            tgk_sincosf(col, &st, &ct);
+            dm::sincosf_small(az, &sp, &cp);
+            dm::sincosf_small(col, &st, &ct);
             r.value = (o.x * t0 + o.y * t1) + o.z * t2;
             r.dtheta = 2.0f * ((t0 * (ct * cp) + t1 * (ct * sp)) + t2 * (-st));
             r.dphi = 2.0f * ((t0 * (-sp) + t1 * cp) + t2 * 0.0f);
@@ -286,13 +289,13 @@ __device__ __forceinline__ V3 probabilistic_update(const AlgoParams &a, const fl
     const V3 helper = fabsf(o.z) < 0.9f ? v3(0.0f, 0.0f, 1.0f) : v3(0.0f, 1.0f, 0.0f);
     const V3 t1 = normalize3(cross3(helper, o));
     const V3 t2 = cross3(o, t1);
-    const float cos_max = tgk_cosf(a.max_angle);
+    const float cos_max = dm::cosf_small(a.max_angle);
     auto candidate = [&](uint2 &state) {
         const float cos_angle = 1.0f - randu(state) * (1.0f - cos_max);
         const float sin_angle = tgk_sqrtf(fmaxf(0.0f, 1.0f - cos_angle * cos_angle));
         const float azimuth = (2.0f * 3.14159265359f) * randu(state);
         float sa, ca;
-        tgk_sincosf(azimuth, &sa, &ca);
+        dm::sincosf_small(azimuth, &sa, &ca);
         return v3(cos_angle * o.x + sin_angle * (ca * t1.x + sa * t2.x),
                   cos_angle * o.y + sin_angle * (ca * t1.y + sa * t2.y),
                   cos_angle * o.z + sin_angle * (ca * t1.z + sa * t2.z));
@@ -313,8 +316,8 @@ __device__ __forceinline__ V3 sphere_gradient(const VoxelModel<MODEL, KT> &vox, 
     const ModelValue m = vox.eval(o);
     float az, col, sp, cp, st, ct;
     cart2sph(o, az, col);
-    tgk_sincosf(az, &sp, &cp);
-    tgk_sincosf(col, &st, &ct);
+    dm::sincosf_small(az, &sp, &cp);
+    dm::sincosf_small(col, &st, &ct);
     return v3(m.dtheta * (ct * cp) + m.dphi * (-sp), m.dtheta * (ct * sp) + m.dphi * cp,
               m.dtheta * (-st) + m.dphi * 0.0f);
 }
@@ -337,8 +340,8 @@ __device__ __forceinline__ V3 deterministic_update(const AlgoParams &a, const fl
     for (int iteration = 0; iteration < a.max_iterations; iteration++) {
         float az, col, sp, cp, st, ct;
         cart2sph(o, az, col);
-        tgk_sincosf(az, &sp, &cp);
-        tgk_sincosf(col, &st, &ct);
+        dm::sincosf_small(az, &sp, &cp);
+        dm::sincosf_small(col, &st, &ct);
         const V3 e1 = v3(ct * cp, ct * sp, -st);
         const V3 e2 = v3(-sp, cp, 0.0f);
         const ModelValue current = vox.eval(o);
@@ -411,8 +414,8 @@ __device__ __forceinline__ V3 update(const AlgoParams &a, const float *__restric
     const ModelValue mv = model_evaluate<MODEL, KT>(row, a.n_parameters, o, terms);
     float az, col, sp, cp, st, ct;
     cart2sph(o, az, col);
-    tgk_sincosf(az, &sp, &cp);
-    tgk_sincosf(col, &st, &ct);
+    dm::sincosf_small(az, &sp, &cp);
+    dm::sincosf_small(col, &st, &ct);
     const float etx = ct * cp, ety = ct * sp, etz = -st;
     const float epx = -sp, epy = cp, epz = 0.0f;
     const float m = fmaxf(mv.value, 1e-6f);

@@ -109,7 +109,11 @@ __device__ __forceinline__ float model_value(const float *__restrict__ row, cons
         for (int k = 0; k < 45; k++)
             if (KT == 45 || k < K)
                 v += c[k] * row[k];
-        return plain::softplus(v);
+        // plain::softplus, skipped where no lane's value needs it: the lanes
+        // of a wavefront take the same direction, often off every fibre.
+        if (v * 100.0f < 30.0f)
+            v = dm::logf_normal(1.0f + dm::expf(100.0f * v)) / 100.0f;
+        return v;
     }
 }
 
