@@ -520,6 +520,106 @@ __device__ inline bool grid_segment_hit(const MeshView &m, V3 start, V3 end, boo
     return grid_candidates_hit(m, m.cell_start[cell], m.cell_start[cell + 1], st, dir, hit, hit_t);
 }
 
+// A lane's cached range [first, last) of the candidate lists: that of culling
+// cell `cell` (UNSET_CELL: none yet).
+constexpr uint32_t UNSET_CELL = 0xfffffffeu;
+struct SegmentCandidates {
+    uint32_t cell, first, last;
+};
+
+// Boundary test of the wavefront's last segments against their start cells'
+// candidate lists, the (lane, candidate) pairs spread over the wavefront's
+// lanes. Lanes near a surface are few (about one in twenty per step), so
+// looping per lane would run the longest list for all 64 lanes; here a step
+// costs one round of 64 pairs while the lists sum to 64 or fewer. Each pair
+// is tested with the bound 1 (grid_triangle_hit), and a lane keeps its
+// smallest t, the last in list order among equal t: the candidate that
+// testing its list in order with "t <= best replaces" ends on
+// (grid_segment_hit), so the hit is the same. Called by every lane of the
+// wavefront; `decided` is false where the lists cannot decide (the caller
+// then asks the BVH), `found`/`tri` give the hit.
+__device__ __forceinline__ void wave_segment_test(const MeshView &m, V3 start, V3 point, bool live,
+                                                  SegmentCandidates &near, bool &decided, bool &found, uint32_t &tri)
+{
+    decided = false;
+    found = false;
+    tri = 0;
+    const int lane = __lane_id();
+    const float sx = start.x, sy = start.y, sz = start.z;
+    const float dx = point.x - sx, dy = point.y - sy, dz = point.z - sz;
+    uint32_t first = 0, count = 0;
+    if (live && m.cell_start != nullptr && m.reach > 0.0f &&
+        (dx * dx + dy * dy) + dz * dz <= m.reach * m.reach) {
+        const int64_t cell = mesh_grid_cell(m, start);
+        if (cell >= 0) {
+            decided = true;
+            if ((uint32_t)cell != near.cell) {
+                near.cell = (uint32_t)cell;
+                near.first = m.cell_start[cell];
+                near.last = m.cell_start[cell + 1];
+            }
+            first = near.first;
+            count = near.last - near.first;
+        }
+    }
+    if (__ballot(count != 0) == 0)
+        return;
+    // Pairs [begin, end) of the flattened list belong to this lane. A list
+    // holds fewer than 2^26 candidates (tgk_domain_set_segment_grid), so the
+    // sum of 64 fits 32 bits with room for the last round's base + 64.
+    uint32_t end = count;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t v = __shfl_up(end, d);
+        if (lane >= d)
+            end += v;
+    }
+    const uint32_t total = __shfl(end, 63);
+    const uint32_t begin = end - count;
+    float best_t = 1.0f;
+    uint32_t best_index = 0;
+    for (uint32_t base = 0; base < total; base += 64) {
+        const uint32_t k = base + (uint32_t)lane;
+        // Owner of pair k: the last lane whose begin is at most k (begins
+        // never decrease along the lanes; lanes after the owner begin past k).
+        int owner = 0;
+#pragma unroll
+        for (int step = 32; step >= 1; step >>= 1) {
+            if (__shfl(begin, owner + step) <= k)
+                owner += step;
+        }
+        const uint32_t index = __shfl(first, owner) + (k - __shfl(begin, owner));
+        const float st[3] = {__shfl(sx, owner), __shfl(sy, owner), __shfl(sz, owner)};
+        const float dir[3] = {__shfl(dx, owner), __shfl(dy, owner), __shfl(dz, owner)};
+        bool h = false;
+        float t = 0.0f;
+        uint32_t slot = 0;
+        if (k < total) {
+            const float4 a = m.cell_entries[3 * (size_t)index];
+            const float4 e1 = m.cell_entries[3 * (size_t)index + 1];
+            const float4 e2 = m.cell_entries[3 * (size_t)index + 2];
+            h = grid_triangle_hit(a, e1, e2, st, dir, 1.0f, t);
+            slot = __float_as_uint(a.w);
+        }
+        // Hits are rare: hand each to its owner in turn.
+        uint64_t hits = __ballot(h);
+        while (hits != 0) {
+            const int j = __ffsll((unsigned long long)hits) - 1;
+            hits &= hits - 1;
+            const int oj = __shfl(owner, j);
+            const float tj = __shfl(t, j);
+            const uint32_t ij = __shfl(index, j);
+            const uint32_t sj = __shfl(slot, j);
+            if (lane == oj && (!found || tj < best_t || (tj == best_t && ij > best_index))) {
+                found = true;
+                best_t = tj;
+                best_index = ij;
+                tri = sj;
+            }
+        }
+    }
+}
+
 // True when the culling grid proves that a segment from `start` of squared
 // length `len2` cannot reach any boundary triangle.
 __device__ __forceinline__ bool mesh_far(const MeshView &m, V3 start, float len2)

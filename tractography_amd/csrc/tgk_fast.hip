@@ -63,7 +63,6 @@ __device__ __forceinline__ int64_t mask_cell(const MaskView &m, V3 p)
 // Cell ids of the tracking kernel are 32-bit: the fast path takes mask and
 // field grids of fewer than 2^32 - 2 voxels.
 constexpr uint32_t NO_CELL = 0xffffffffu;     // outside the grid
-constexpr uint32_t UNSET_CELL = 0xfffffffeu;  // nothing cached yet
 
 // The cell of rounded voxel coordinates (rx, ry, rz) on a grid, C order.
 __device__ __forceinline__ uint32_t grid_cell(float rx, float ry, float rz, const uint32_t dims[3])
@@ -102,9 +101,7 @@ template <int G> struct Lane {
     uint32_t field_cell; // cell ids of `point` (UNSET_CELL: none yet); their data is requested by request_cells
     uint32_t mask_cell;
     uint32_t mask_value; // the mask at mask_cell (0 outside the mask image)
-    // Mesh domains: culling-grid cell of the last tested segment's start
-    // (UNSET_CELL: none yet) and its candidate range [cand_first, cand_last).
-    uint32_t mesh_cell, cand_first, cand_last;
+    SegmentCandidates near;  // mesh domains: of the last tested segment's start
     bool field_ok;       // `point` is inside the field image
     bool row_read;       // request_cells read a row / a mask value this iteration
     bool mask_read;
@@ -388,100 +385,6 @@ __device__ __forceinline__ void request_cells(const TrackLaunch &p, bool shared_
     }
 }
 
-// Boundary test of the wavefront's last segments against their start cells'
-// candidate lists, the (lane, candidate) pairs spread over the wavefront's
-// lanes. Lanes near a surface are few (about one in twenty per step), so
-// looping per lane would run the longest list for all 64 lanes; here a step
-// costs one round of 64 pairs while the lists sum to 64 or fewer. Each pair
-// is tested with the bound 1 (grid_triangle_hit), and a lane keeps its
-// smallest t, the last in list order among equal t: the candidate that
-// testing its list in order with "t <= best replaces" ends on
-// (grid_segment_hit), so the hit is the same. Called by every lane of the
-// wavefront; `decided` is false where the lists cannot decide (the caller
-// then asks the BVH), `found`/`tri` give the hit.
-template <int G>
-__device__ __forceinline__ void wave_segment_test(const MeshView &m, Lane<G> &L, bool live, bool &decided,
-                                                  bool &found, uint32_t &tri)
-{
-    decided = false;
-    found = false;
-    tri = 0;
-    const int lane = __lane_id();
-    const float sx = L.previous.x, sy = L.previous.y, sz = L.previous.z;
-    const float dx = L.point.x - sx, dy = L.point.y - sy, dz = L.point.z - sz;
-    uint32_t first = 0, count = 0;
-    if (live && L.steps > 0 && m.cell_start != nullptr && m.reach > 0.0f &&
-        (dx * dx + dy * dy) + dz * dz <= m.reach * m.reach) {
-        const int64_t cell = mesh_grid_cell(m, L.previous);
-        if (cell >= 0) {
-            decided = true;
-            if ((uint32_t)cell != L.mesh_cell) {
-                L.mesh_cell = (uint32_t)cell;
-                L.cand_first = m.cell_start[cell];
-                L.cand_last = m.cell_start[cell + 1];
-            }
-            first = L.cand_first;
-            count = L.cand_last - L.cand_first;
-        }
-    }
-    if (__ballot(count != 0) == 0)
-        return;
-    // Pairs [begin, end) of the flattened list belong to this lane. A list
-    // holds fewer than 2^26 candidates (tgk_domain_set_segment_grid), so the
-    // sum of 64 fits 32 bits with room for the last round's base + 64.
-    uint32_t end = count;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t v = __shfl_up(end, d);
-        if (lane >= d)
-            end += v;
-    }
-    const uint32_t total = __shfl(end, 63);
-    const uint32_t begin = end - count;
-    float best_t = 1.0f;
-    uint32_t best_index = 0;
-    for (uint32_t base = 0; base < total; base += 64) {
-        const uint32_t k = base + (uint32_t)lane;
-        // Owner of pair k: the last lane whose begin is at most k (begins
-        // never decrease along the lanes; lanes after the owner begin past k).
-        int owner = 0;
-#pragma unroll
-        for (int step = 32; step >= 1; step >>= 1) {
-            if (__shfl(begin, owner + step) <= k)
-                owner += step;
-        }
-        const uint32_t index = __shfl(first, owner) + (k - __shfl(begin, owner));
-        const float st[3] = {__shfl(sx, owner), __shfl(sy, owner), __shfl(sz, owner)};
-        const float dir[3] = {__shfl(dx, owner), __shfl(dy, owner), __shfl(dz, owner)};
-        bool h = false;
-        float t = 0.0f;
-        uint32_t slot = 0;
-        if (k < total) {
-            const float4 a = m.cell_entries[3 * (size_t)index];
-            const float4 e1 = m.cell_entries[3 * (size_t)index + 1];
-            const float4 e2 = m.cell_entries[3 * (size_t)index + 2];
-            h = grid_triangle_hit(a, e1, e2, st, dir, 1.0f, t);
-            slot = __float_as_uint(a.w);
-        }
-        // Hits are rare: hand each to its owner in turn.
-        uint64_t hits = __ballot(h);
-        while (hits != 0) {
-            const int j = __ffsll((unsigned long long)hits) - 1;
-            hits &= hits - 1;
-            const int oj = __shfl(owner, j);
-            const float tj = __shfl(t, j);
-            const uint32_t ij = __shfl(index, j);
-            const uint32_t sj = __shfl(slot, j);
-            if (lane == oj && (!found || tj < best_t || (tj == best_t && ij > best_index))) {
-                found = true;
-                best_t = tj;
-                best_index = ij;
-                tri = sj;
-            }
-        }
-    }
-}
-
 // The tests that end a streamline before its next update, in the reference's
 // order (tracking.py:121-133): the row or the step count is full, the point
 // left the mask or the last segment hit the boundary (`hit` then names the
@@ -514,7 +417,9 @@ __device__ __forceinline__ bool stop_test(const TrackLaunch &p, const Lane<G> &L
             }
         }
     }
-    return stop || !L.field_ok;
+    if (!stop)
+        stop = !L.field_ok;
+    return stop;
 }
 
 // nz: this step's Diffusion draws, made by the caller before anything that
@@ -678,7 +583,7 @@ void track_fast_kernel(FastLaunch f)
                     L.field_cell = UNSET_CELL;
                     L.mask_cell = UNSET_CELL;
                     L.mask_value = 0;
-                    L.mesh_cell = UNSET_CELL;
+                    L.near.cell = UNSET_CELL;
                     request_cells<MODEL, DOMAIN, LMAX, G, LDS_VEC, BLOCK>(p, f.shared_affine != 0, coeffs, cstride,
                                                                           L, q, lds_rows);
                 }
@@ -731,7 +636,8 @@ void track_fast_kernel(FastLaunch f)
         bool seg_decided = false, seg_found = false;
         uint32_t seg_tri = 0;
         if constexpr (DOMAIN == DOMAIN_MESH)
-            wave_segment_test<G>(p.mesh, L, L.g >= 0, seg_decided, seg_found, seg_tri);
+            wave_segment_test(p.mesh, L.previous, L.point, L.g >= 0 && L.steps > 0, L.near, seg_decided, seg_found,
+                              seg_tri);
         if (L.g >= 0)
             advance<MODEL, ALGO, DOMAIN, LMAX, G, LDS_VEC, BLOCK>(p, f.shared_affine != 0, coeffs, cstride, L, q,
                                                                  lds_rows, nz, seg_decided, seg_found, seg_tri);
@@ -842,7 +748,7 @@ __global__ __launch_bounds__(256) void track_group_kernel(FastLaunch f)
                     L.field_cell = UNSET_CELL;
                     L.mask_cell = UNSET_CELL;
                     L.mask_value = 0;
-                    L.mesh_cell = UNSET_CELL;
+                    L.near.cell = UNSET_CELL;
                     request_cells<MODEL, DOMAIN, LMAX, 1, 0, 256>(p, f.shared_affine != 0, coeffs, f.coeff_stride, L,
                                                                   q, nullptr);
                 }
@@ -855,7 +761,8 @@ __global__ __launch_bounds__(256) void track_group_kernel(FastLaunch f)
         uint32_t seg_tri = 0;
         if constexpr (DOMAIN == DOMAIN_MESH) {
             // Asked once per group.
-            wave_segment_test<1>(p.mesh, L, leader && starting, seg_decided, seg_found, seg_tri);
+            wave_segment_test(p.mesh, L.previous, L.point, leader && starting && L.steps > 0, L.near, seg_decided,
+                              seg_found, seg_tri);
             seg_decided = __shfl((int)seg_decided, 0, W) != 0;
             seg_found = __shfl((int)seg_found, 0, W) != 0;
             seg_tri = __shfl(seg_tri, 0, W);

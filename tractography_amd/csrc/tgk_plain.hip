@@ -30,30 +30,19 @@ __device__ __forceinline__ void store_point(float *dense, uint32_t n_points, uin
     dst[2] = p.z;
 }
 
-// Waves per SIMD the compiler must fit in the SH tracking kernels, which
-// otherwise take 146-148 VGPRs (Transport, Diffusion; three waves), 164-170
-// (Probabilistic; three) or 291-295 (Deterministic; one). The Deterministic
-// kernel is held to two waves (75% faster at 145x174x145 SH45, spilling
-// some 30-50 VGPRs; 3.52 against 5.95 s at one wave on persistent lanes).
-// The others: held to four, they spill 10-54 VGPRs. With one lane per seed
-// for the whole launch that was still 5% (Transport, Diffusion) and 12%
-// (Probabilistic) faster than three waves. On persistent lanes, mask
-// domains run faster at three waves (SH45 Diffusion 74.4 against 91.5 ms
-// per launch) and mesh domains, whose boundary tests wait on dependent
-// node loads, at four (the two-mesh shell 326 against 361 ms). DTI
-// kernels keep the compiler's allocation (already below 128 VGPRs, they
-// lost 11% when held to exactly four). The connectome and TOD kernels are
-// held to two waves for Deterministic only (296 and 342 VGPRs, one wave
-// otherwise: 1.52x faster each); the SH Diffusion connectome held to four
-// waves ran 11% slower.
-template <int MODEL, int ALGO, int DOMAIN> constexpr int plain_min_waves()
+// Waves per SIMD the compiler must fit in the SH tracking kernels: three for
+// Transport, Diffusion and Probabilistic (136-168 VGPRs; held to four they
+// spill, 91.5 against 74.4 ms per SH45 Diffusion launch on a mask domain and,
+// with the boundary tested on candidate lists, 28.7 against 25.6 ms per
+// two-surface launch of 200k seeds), two for Deterministic, which takes some
+// 200 VGPRs and had taken 291-295 with its cases in branches (3.52 against
+// 5.95 s at one wave). DTI kernels keep the compiler's allocation (already
+// below 128 VGPRs, they lost 11% when held to exactly four). The connectome
+// and TOD kernels are held to two waves for Deterministic only; the SH
+// Diffusion connectome held to four waves ran 11% slower.
+template <int MODEL, int ALGO> constexpr int plain_min_waves()
 {
-    if constexpr (MODEL != MODEL_SH)
-        return 1;
-    else if constexpr (ALGO == ALGO_DETERMINISTIC)
-        return 2;
-    else
-        return DOMAIN == DOMAIN_MESH ? 4 : 3;
+    return MODEL != MODEL_SH ? 1 : ALGO == ALGO_DETERMINISTIC ? 2 : 3;
 }
 
 // ------------------------------------------------------ one-op drivers ---
@@ -248,7 +237,7 @@ __device__ __forceinline__ int64_t claim_seed(bool idle, uint32_t *queue, int64_
 // stream are those of its seed index, whichever lane runs it, so the
 // results do not change.
 template <int MODEL, int ALGO, int DOMAIN, int KT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(plain_min_waves<MODEL, ALGO, DOMAIN>())))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(plain_min_waves<MODEL, ALGO>())))
 void track_plain_kernel(TrackLaunch p)
 {
     const float step = p.algo.step_size;
@@ -261,6 +250,7 @@ void track_plain_kernel(TrackLaunch p)
     uint32_t n = 0, steps = 0, hit = NO_HIT;
     float time = 0.0f;
     bool first = true;
+    SegmentCandidates near{UNSET_CELL, 0u, 0u};
     while (true) {
         const int64_t claimed = claim_seed(g < 0, p.queue, p.n_seeds, drained);
         if (claimed >= 0) {
@@ -281,6 +271,11 @@ void track_plain_kernel(TrackLaunch p)
         }
         if (__ballot(g >= 0) == 0)
             break;
+        bool decided = false, found = false;
+        if constexpr (DOMAIN == DOMAIN_MESH) {
+            uint32_t candidate;
+            wave_segment_test(p.mesh, previous, point, g >= 0 && !first, near, decided, found, candidate);
+        }
         if (g < 0)
             continue;
         // One pass of the reference loop; `stop` is its break.
@@ -289,8 +284,15 @@ void track_plain_kernel(TrackLaunch p)
             if constexpr (DOMAIN == DOMAIN_MASK) {
                 stop = !mask_contains(p.mask, point);
             } else if (!first) {
+                // The candidate lists hold every triangle that the traversal
+                // could hit, so a segment that hits none of them needs no
+                // traversal; one that does takes the traversal's answer. A
+                // lane in twenty is near a surface on a step, so nearly every
+                // wavefront traversed on every step: 60.3 -> 28.7 ms per
+                // launch of 200k SH45 seeds between two surfaces of 40k
+                // triangles.
                 const float dx = point.x - previous.x, dy = point.y - previous.y, dz = point.z - previous.z;
-                if (!mesh_far(p.mesh, previous, (dx * dx + dy * dy) + dz * dz)) {
+                if (decided ? found : !mesh_far(p.mesh, previous, (dx * dx + dy * dy) + dz * dz)) {
                     uint32_t tri;
                     float t;
                     if (bvh_segment_hit(p.mesh, previous, point, tri, t)) {
