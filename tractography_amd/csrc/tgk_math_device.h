@@ -132,6 +132,26 @@ __device__ __forceinline__ float expf(float x)
     return x != x ? x : bounded;
 }
 
+// n / d, correctly rounded, where neither operand nor quotient comes near the
+// ends of the exponent range: the steps of the compiler's division without
+// the scaling and special cases around them.
+__device__ __forceinline__ float divide_inner(float n, float d)
+{
+    float r = __builtin_amdgcn_rcpf(d);
+    r = fmaf(fmaf(-d, r, 1.0f), r, r);
+    float q = n * r;
+    q = fmaf(fmaf(-d, q, n), r, q);
+    return fmaf(fmaf(-d, q, n), r, q);
+}
+
+// x / 100, correctly rounded, for 0 and 2^-32 <= x <= 64 (all of them
+// checked against the division).
+__device__ __forceinline__ float divide_100(float x)
+{
+    const float q = x * 0.01f;
+    return fmaf(fmaf(-100.0f, q, x), 0.01f, q);
+}
+
 // tgk_logf for normal positive finite x.
 __device__ __forceinline__ float logf_normal(float x)
 {
@@ -140,7 +160,7 @@ __device__ __forceinline__ float logf_normal(float x)
     const bool upper = mb > 0x3fb504f3u;
     const int e = (int)(ix >> 23) - (upper ? 126 : 127);
     const float f = tgk_as_f32(upper ? mb - 0x00800000u : mb) - 1.0f;
-    const float s = f / (2.0f + f);
+    const float s = divide_inner(f, 2.0f + f);
     const float w = s * s;
     float p = fmaf(w, 2.428623587e-01f, 2.849848568e-01f);
     p = fmaf(w, p, 4.000097513e-01f);
@@ -148,6 +168,23 @@ __device__ __forceinline__ float logf_normal(float x)
     const float correction = s * fmaf(-w, p, f);
     const float ef = (float)e;
     return fmaf(ef, TGK_LN2_HI, f - fmaf(-ef, TGK_LN2_LO, correction));
+}
+
+// log(1 + exp(x)) / 100 for x < 30, as tgk_logf(1 + tgk_expf(x)) / 100
+// rounds it: below -20 the sum rounds to 1, whatever the exponential.
+__device__ __forceinline__ float log1pexp_100(float x)
+{
+    const float xc = fmaxf(x, -20.0f);
+    const float k = rintf(xc * TGK_LOG2E);
+    float r = fmaf(-k, TGK_LN2_HI, xc);
+    r = fmaf(-k, TGK_LN2_LO, r);
+    float p = fmaf(r, 1.974024926e-04f, 1.393507817e-03f);
+    p = fmaf(r, p, 8.333570324e-03f);
+    p = fmaf(r, p, 4.166646302e-02f);
+    p = fmaf(r, p, 1.666666567e-01f);
+    p = fmaf(r, p, 5.000000000e-01f);
+    const float e = fmaf(r * r, p, r) + 1.0f;
+    return divide_100(logf_normal(1.0f + __builtin_ldexpf(e, (int)k)));
 }
 
 __device__ __forceinline__ float logf(float x)

@@ -46,8 +46,7 @@ __device__ __forceinline__ V3 exps2(V3 p, V3 x)
 // core.cl:111-120, k = 100
 __device__ __forceinline__ float softplus(float x)
 {
-    // The logarithm's argument is at least 1, and finite where it is taken.
-    const float soft = dm::logf_normal(1.0f + dm::expf(100.0f * x)) / 100.0f;
+    const float soft = dm::log1pexp_100(100.0f * x);
     return x * 100.0f < 30.0f ? soft : x;
 }
 __device__ __forceinline__ float dsoftplus(float x) { return 1.0f / (1.0f + dm::expf(-100.0f * x)); }

@@ -2,8 +2,8 @@
 //
 // VALU method (bit-identical to the reference's arithmetic):
 // Every seed evaluates its voxel's model on the same 1000 Fibonacci
-// directions, twice (once for the total weight, once for the cumulative
-// search). The reference recomputes the direction and its 45 SH basis values
+// directions, twice in the reference (once for the total weight, once for the
+// cumulative search). The reference recomputes the direction and its 45 SH basis values
 // for every evaluation; here they are computed once per launch into a table
 // (basis_table_kernel, with the plain path's bit-exact basis code) and each
 // evaluation is the in-order contraction of the seed's coefficients with a
@@ -39,7 +39,9 @@ namespace {
 
 constexpr int N_DIRECTIONS = 1000;
 constexpr int TABLE_STRIDE = 48;
-constexpr int DIRECTION_BLOCK = 4;  // directions evaluated together by the VALU method
+constexpr int SUM_BLOCKS = 25;      // running sums the VALU method keeps
+constexpr int BLOCK_DIRECTIONS = N_DIRECTIONS / SUM_BLOCKS;
+static_assert(SUM_BLOCKS * BLOCK_DIRECTIONS == N_DIRECTIONS, "blocks cover the directions");
 
 // seeds.cl:12-25 (host and device: the MFMA table is built on the host at
 // the same FP32 directions).
@@ -92,10 +94,11 @@ __global__ void basis_table_kernel(float *__restrict__ table)
 // Model value at direction i (models/*.cl evaluate_interpolated_model):
 // SH: softplus of the in-order contraction of the first K terms; DTI:
 // o . (D o). The contraction is unrolled so that c stays in registers (a
-// loop to a run-time K indexed it in scratch memory); KT = 45 needs no
-// test, otherwise each term is taken while k < K (a uniform branch).
+// loop to a run-time K indexed it in scratch memory, and a test of k < K per
+// term took 10.7 ms per 1M seeds at K = 15 against 1.7). KT terms are taken, K rounded up to a whole order (15, 28 or 45);
+// the coefficients past K are zeros, which leave the sum as it is.
 template <int MODEL, int KT>
-__device__ __forceinline__ float model_value(const float *__restrict__ row, const float c[45], int K)
+__device__ __forceinline__ float model_value(const float *__restrict__ row, const float c[45])
 {
     if constexpr (MODEL == MODEL_DTI) {
         const float ox = row[45], oy = row[46], oz = row[47];
@@ -106,13 +109,12 @@ __device__ __forceinline__ float model_value(const float *__restrict__ row, cons
     } else {
         float v = 0.0f;
 #pragma unroll
-        for (int k = 0; k < 45; k++)
-            if (KT == 45 || k < K)
-                v += c[k] * row[k];
+        for (int k = 0; k < KT; k++)
+            v += c[k] * row[k];
         // plain::softplus, skipped where no lane's value needs it: the lanes
         // of a wavefront take the same direction, often off every fibre.
         if (v * 100.0f < 30.0f)
-            v = dm::logf_normal(1.0f + dm::expf(100.0f * v)) / 100.0f;
+            v = dm::log1pexp_100(100.0f * v);
         return v;
     }
 }
@@ -139,38 +141,50 @@ __global__ __launch_bounds__(256) void seeds_from_fod_kernel(const float *__rest
     voxel.z += jz;
     float c[45];
 #pragma unroll
-    for (int k = 0; k < 45; k++)
+    for (int k = 0; k < KT; k++)
         c[k] = k < K ? fod[(int64_t)index * K + k] : 0.0f;
 
-    // seeds.cl:28-62. Directions are evaluated DIRECTION_BLOCK at a time: their
-    // contractions are independent chains the wavefront can interleave (one
-    // at a time, each waited on its own dependent adds and table loads),
-    // and their weights are then added to the sums in direction order, so
-    // every rounding is the reference's.
-    static_assert(N_DIRECTIONS % DIRECTION_BLOCK == 0, "directions come in whole blocks");
+    // seeds.cl:28-62, the weights added in direction order, so every rounding
+    // is the reference's. The reference sums all weights for the total, then
+    // again until the sum passes the threshold. Both are the same sums, so
+    // the first pass keeps the one it reaches at the start of each of
+    // SUM_BLOCKS blocks, and the second evaluates one block, the first whose
+    // end passes the threshold: 1000 + 40 evaluations for up to 2000. 1M
+    // SH45 seeds: 6.4 -> 3.1 ms, of which VALU issue is about 2.8 (138
+    // instructions per direction). One direction at a time: the words of four
+    // rows do not fit the scalar registers (4.2 ms; two at a time 3.4).
+    float starts[SUM_BLOCKS];
     float sum = 0.0f;
-    for (int i = 0; i < N_DIRECTIONS; i += DIRECTION_BLOCK) {
-        float w[DIRECTION_BLOCK];
 #pragma unroll
-        for (int d = 0; d < DIRECTION_BLOCK; d++)
-            w[d] = fmaxf(model_value<MODEL, KT>(table + (i + d) * TABLE_STRIDE, c, K), 0.0f);
-#pragma unroll
-        for (int d = 0; d < DIRECTION_BLOCK; d++)
-            sum += w[d];
+    for (int b = 0; b < SUM_BLOCKS; b++) {
+        starts[b] = sum;
+        for (int i = b * BLOCK_DIRECTIONS; i < (b + 1) * BLOCK_DIRECTIONS; i++)
+            sum += fmaxf(model_value<MODEL, KT>(table + i * TABLE_STRIDE, c), 0.0f);
     }
     const float threshold = randu(state) * sum;
-    float cs = 0.0f;
     int selected = N_DIRECTIONS;
-    for (int i = 0; i < N_DIRECTIONS; i += DIRECTION_BLOCK) {
-        float w[DIRECTION_BLOCK];
+    // The sums never decrease, so the first to pass the threshold lies in the
+    // first block whose end does; none does where the last end does not (a
+    // zero or non-finite total).
+    int block = SUM_BLOCKS;
+    float cs = 0.0f;
 #pragma unroll
-        for (int d = 0; d < DIRECTION_BLOCK; d++)
-            w[d] = fmaxf(model_value<MODEL, KT>(table + (i + d) * TABLE_STRIDE, c, K), 0.0f);
-#pragma unroll
-        for (int d = 0; d < DIRECTION_BLOCK; d++) {
-            cs += w[d];
-            if (selected == N_DIRECTIONS && cs > threshold)
-                selected = i + d;
+    for (int b = SUM_BLOCKS - 1; b >= 0; b--) {
+        if ((b + 1 < SUM_BLOCKS ? starts[b + 1] : sum) > threshold) {
+            block = b;
+            cs = starts[b];
+        }
+    }
+    if (block < SUM_BLOCKS) {
+        // Lanes read their own block's rows here: 12 words of 16 bytes each,
+        // from L2.
+        const float *rows = table + block * (BLOCK_DIRECTIONS * TABLE_STRIDE);
+        for (int i = 0; i < BLOCK_DIRECTIONS; i++) {
+            cs += fmaxf(model_value<MODEL, KT>(rows + i * TABLE_STRIDE, c), 0.0f);
+            if (cs > threshold) {
+                selected = block * BLOCK_DIRECTIONS + i;
+                break;
+            }
         }
     }
     float ox = 0.0f, oy = 0.0f, oz = 1.0f;
@@ -429,6 +443,16 @@ void launch_mfma(const float *fod, int K, const float *voxels, uint32_t nnz, con
         static_cast<const float4 *>(dirs), reinterpret_cast<uint2 *>(states), n, out);
 }
 
+template <int MODEL, int KT>
+void launch_valu(const float *fod, int K, const float *voxels, uint32_t nnz, const float *affine, const void *table,
+                 uint32_t *states, int64_t n, float *out, hipStream_t stream)
+{
+    const unsigned blocks = (unsigned)((n + 255) / 256);
+    seeds_from_fod_kernel<MODEL, KT><<<blocks, 256, 0, stream>>>(
+        fod, K, reinterpret_cast<const float4 *>(voxels), nnz, affine, static_cast<const float *>(table),
+        reinterpret_cast<uint2 *>(states), n, out);
+}
+
 }  // namespace
 
 size_t seeds_from_fod_workspace_bytes(int model, int K, int64_t n, int32_t method)
@@ -475,7 +499,6 @@ hipError_t launch_seeds_from_fod_prepared(int model, int K, const float *fod, co
         return hipSuccess;
     if (nnz == 0)
         return hipErrorInvalidValue;
-    const unsigned blocks = (unsigned)((n + 255) / 256);
     if (method == SEEDS_MFMA) {
         const void *ddirs = static_cast<const char *>(table) + mfma_table_bytes(K);
         if (model == MODEL_DTI)
@@ -488,19 +511,14 @@ hipError_t launch_seeds_from_fod_prepared(int model, int K, const float *fod, co
             launch_mfma<MODEL_SH, 6>(fod, K, voxels, nnz, affine, table, ddirs, states, n, out, stream);
         return hipGetLastError();
     }
-    const float *t = static_cast<const float *>(table);
     if (model == MODEL_DTI)
-        seeds_from_fod_kernel<MODEL_DTI, 0><<<blocks, 256, 0, stream>>>(
-            fod, K, reinterpret_cast<const float4 *>(voxels), nnz, affine, t, reinterpret_cast<uint2 *>(states), n,
-            out);
-    else if (K == 45)
-        seeds_from_fod_kernel<MODEL_SH, 45><<<blocks, 256, 0, stream>>>(
-            fod, K, reinterpret_cast<const float4 *>(voxels), nnz, affine, t, reinterpret_cast<uint2 *>(states), n,
-            out);
+        launch_valu<MODEL_DTI, 6>(fod, K, voxels, nnz, affine, table, states, n, out, stream);
+    else if (K <= 15)
+        launch_valu<MODEL_SH, 15>(fod, K, voxels, nnz, affine, table, states, n, out, stream);
+    else if (K <= 28)
+        launch_valu<MODEL_SH, 28>(fod, K, voxels, nnz, affine, table, states, n, out, stream);
     else
-        seeds_from_fod_kernel<MODEL_SH, 0><<<blocks, 256, 0, stream>>>(
-            fod, K, reinterpret_cast<const float4 *>(voxels), nnz, affine, t, reinterpret_cast<uint2 *>(states), n,
-            out);
+        launch_valu<MODEL_SH, 45>(fod, K, voxels, nnz, affine, table, states, n, out, stream);
     return hipGetLastError();
 }
 
