@@ -88,6 +88,8 @@ struct DeviceBuffer {
 // saved-streamline counts (u32).
 constexpr size_t FAST_STATS_OFFSET = 64;
 constexpr size_t FAST_CONT_COUNT_OFFSET = 136;
+// The plain kernels' two saved-streamline counts (u32).
+constexpr size_t PLAIN_COUNT_OFFSET = 144;
 
 // tgk_track's device buffers for one chunk of seeds, kept by the runtime.
 struct TrackBuffers {
@@ -100,6 +102,7 @@ struct tgk_runtime {
     DeviceBuffer workspace;
     DeviceBuffer queue;        // counters of the persistent kernels (layout: FAST_*_OFFSET)
     DeviceBuffer continuations[2];  // streamlines saved between generations of the fast kernel
+    DeviceBuffer plain_saved;       // streamlines saved between launches of the plain kernels (allocated once)
     DeviceBuffer fast_counters;     // claim counter and ended-streamline shards of the fast kernel
     TrackBuffers track_buffers;     // tgk_track's working buffers
     DeviceBuffer seeds_table;  // prepared FOD-seeding table for seeds_key
@@ -1209,6 +1212,28 @@ int tgk_tracks_destroy(tgk_tracks *tracks)
 
 namespace {
 
+// Workspace of a plain tracking launch. The room for saved streamlines (10
+// MiB) is allocated before the first launch that can use it; while a graph is
+// being recorded, a launch without it runs in one piece.
+int plain_work(tgk_runtime *rt, const tgk_algorithm *algorithm, int64_t n_seeds, tgk::PlainWork *w)
+{
+    constexpr size_t half = (size_t)tgk::PLAIN_HALF_ROOM * tgk::PLAIN_SAVED_BYTES;
+    constexpr size_t split = (size_t)tgk::PLAIN_SPLIT_SEEDS * tgk::PLAIN_SAVED_BYTES;
+    const bool resumes = algorithm->model == TGK_MODEL_SH &&
+                         (algorithm->algorithm == TGK_ALGO_TRANSPORT || algorithm->algorithm == TGK_ALGO_DIFFUSION);
+    if (resumes && n_seeds > tgk::PLAIN_SPLIT_SEEDS && !rt->plain_saved.ptr && !rt->capturing)
+        TGK_HIP(rt->plain_saved.allocate(half + split), "saved streamlines");
+    memset(w, 0, sizeof *w);
+    w->ended = rt->fast_counters.as<uint32_t>() + 32;
+    if (rt->plain_saved.ptr) {
+        w->saved[0] = rt->plain_saved.as<float4>();
+        w->saved[1] = reinterpret_cast<float4 *>(rt->plain_saved.as<char>() + half);
+        for (int i = 0; i < 2; i++)
+            w->count[i] = reinterpret_cast<uint32_t *>(rt->queue.as<char>() + PLAIN_COUNT_OFFSET + 4 * i);
+    }
+    return TGK_OK;
+}
+
 int run_track(tgk_runtime *rt, const tgk_domain *domain, tgk_field *field, const tgk_algorithm *algorithm,
               int32_t path, const float *d_seeds, int64_t first_seed, int64_t n_seeds, const uint32_t *d_rng_seeds,
               int64_t batch_size, uint32_t n_points, float save_at, uint32_t *d_lengths, uint32_t *d_steps,
@@ -1223,7 +1248,10 @@ int run_track(tgk_runtime *rt, const tgk_domain *domain, tgk_field *field, const
     // time.
     p.queue = rt->queue.as<uint32_t>();
     if (path == TGK_PATH_PLAIN) {
-        TGK_HIP(tgk::launch_track_plain(p, rt->stream), "plain tracking kernel");
+        tgk::PlainWork w;
+        if (int r = plain_work(rt, algorithm, n_seeds, &w))
+            return r;
+        TGK_HIP(tgk::launch_track_plain(p, w, rt->stream), "plain tracking kernel");
         return TGK_OK;
     }
     tgk::FastLaunch f;
@@ -1881,7 +1909,11 @@ int tgk_track_prepare(tgk_runtime *rt, const tgk_domain *domain, const tgk_field
         return r;
     if (int r = ensure_workspace(rt, tgk::offsets_workspace_bytes(max_seeds)))
         return r;
-    if (path == TGK_PATH_FAST) {
+    if (path == TGK_PATH_PLAIN) {
+        tgk::PlainWork w;
+        if (int r = plain_work(rt, algorithm, max_seeds, &w))
+            return r;
+    } else {
         const tgk::TrackLaunch p = make_launch(domain, field, algorithm, nullptr, 0, 0, nullptr, 1, 1, 1.0f, nullptr,
                                                nullptr, nullptr, nullptr);
         tgk::FastLaunch f;

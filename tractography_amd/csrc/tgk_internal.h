@@ -12,10 +12,40 @@ namespace tgk {
 // Sets the thread's tgk_last_error() message and returns `code`.
 int report_error(int code, const char *fmt, ...);
 
-// Plain FP32 path (tgk_plain.hip): persistent lanes claiming seeds through
-// p.queue (zeroed by the launch), seed-major dense output (compacted by
-// launch_compact_seed_major, as the fast path's).
-hipError_t launch_track_plain(const TrackLaunch &p, hipStream_t stream);
+// Counters of streamlines that left a generation: FAST_END_SHARDS u32, one
+// per FAST_END_STRIDE u32 (128 bytes), after a first 128-byte line holding
+// the claim counter.
+constexpr int FAST_END_SHARDS = 32;
+constexpr int FAST_END_STRIDE = 32;
+// The plain path's SH Transport and Diffusion launches: at most this many
+// seeds run as split wavefronts, and larger launches hand their last ones
+// over to them (launch_plain_tail). 145 x 174 x 145 SH45 Diffusion, one
+// wavefront per 64 streamlines against split: 10.5 and 8.3 ms with 16k seeds,
+// 10.5 and 9.2 with 32k, 10.6 and 11.2 with 48k; 32^3 Transport: 13.9 and 8.7
+// ms with 16k, 15.1 and 10.4 with 32k, 14.5 and 11.6 with 48k.
+constexpr int64_t PLAIN_SPLIT_SEEDS = 32768;
+// Saved streamlines of a launch cut short at half its lanes.
+constexpr int64_t PLAIN_HALF_ROOM = 131072;
+constexpr size_t PLAIN_SAVED_BYTES = 64;
+// One launch's end of a sequence of them: the streamlines it resumes (in:
+// nullptr for seeds) and those it saves once fewer than stop_below are left
+// (0: none).
+struct PlainTail {
+    const float4 *in;
+    const uint32_t *in_count;
+    float4 *out;
+    uint32_t *out_count;
+    uint32_t *ended;  // FAST_END_SHARDS counters, zeroed per launch
+    uint32_t stop_below;
+};
+// Device memory for them: room for PLAIN_HALF_ROOM and PLAIN_SPLIT_SEEDS
+// streamlines, or nullptr.
+struct PlainWork {
+    uint32_t *ended;
+    float4 *saved[2];
+    uint32_t *count[2];
+};
+hipError_t launch_track_plain(const TrackLaunch &p, const PlainWork &w, hipStream_t stream);
 
 // Boundary connectome (tgk_plain.hip, plain arithmetic): a mask domain, its
 // boundary surface with BVH, 9 (row, col, weight) entries per seed.
@@ -96,11 +126,6 @@ constexpr uint32_t FAST_MIN_REPACK = 16384;
 constexpr uint32_t FAST_MIN_REPACK_MESH = 65536;
 // float4s per saved streamline.
 constexpr int FAST_CONTINUATION_VEC4 = 4;
-// Counters of streamlines that left a generation: FAST_END_SHARDS u32, one
-// per FAST_END_STRIDE u32 (128 bytes), after a first 128-byte line holding
-// the claim counter.
-constexpr int FAST_END_SHARDS = 32;
-constexpr int FAST_END_STRIDE = 32;
 constexpr size_t FAST_COUNTER_BYTES = 128 + (size_t)FAST_END_SHARDS * FAST_END_STRIDE * 4;
 // Launch shapes of the order-8 SH Transport and Diffusion tracking kernels
 // (lanes per block, coefficients in LDS), indexed 0..FAST_SHAPE_COUNT - 1:

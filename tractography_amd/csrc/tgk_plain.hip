@@ -15,6 +15,8 @@
 // measurable either way.)
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "tgk_internal.h"
 #include "tgk_plain_model.h"
 
@@ -236,98 +238,333 @@ __device__ __forceinline__ int64_t claim_seed(bool idle, uint32_t *queue, int64_
 // about half of them masked off. Each streamline's arithmetic and noise
 // stream are those of its seed index, whichever lane runs it, so the
 // results do not change.
+//
+// Once the queue is empty, lanes go idle while their wavefronts go on with
+// the streamlines left, at the full grid's time per step. SH Transport and
+// Diffusion launches stop there (PlainTail): when fewer than `stop_below`
+// streamlines are in flight, every wavefront saves its own and ends, and the
+// next launch resumes them packed together (launch_plain_tail).
+template <int MODEL, int ALGO> constexpr bool has_tail()
+{
+    return MODEL == MODEL_SH && (ALGO == ALGO_TRANSPORT || ALGO == ALGO_DIFFUSION);
+}
+
+// A streamline in flight between two launches, in four float4.
+struct PlainStreamline {
+    V3 point, o, previous;
+    float time;
+    int64_t g;  // below 2^31
+    uint32_t n, steps;
+    uint2 rng;
+};
+__device__ __forceinline__ void save_streamline(float4 *slot, const PlainStreamline &s)
+{
+    slot[0] = make_float4(s.point.x, s.point.y, s.point.z, s.o.x);
+    slot[1] = make_float4(s.o.y, s.o.z, s.previous.x, s.previous.y);
+    slot[2] = make_float4(s.previous.z, s.time, __uint_as_float((uint32_t)s.g), __uint_as_float(s.n));
+    slot[3] = make_float4(__uint_as_float(s.steps), __uint_as_float(s.rng.x), __uint_as_float(s.rng.y), 0.0f);
+}
+__device__ __forceinline__ PlainStreamline saved_streamline(const float4 *slot)
+{
+    const float4 a = slot[0], b = slot[1], c = slot[2], d = slot[3];
+    PlainStreamline s;
+    s.point = v3(a.x, a.y, a.z);
+    s.o = v3(a.w, b.x, b.y);
+    s.previous = v3(b.z, b.w, c.x);
+    s.time = c.y;
+    s.g = (int64_t)__float_as_uint(c.z);
+    s.n = __float_as_uint(c.w);
+    s.steps = __float_as_uint(d.x);
+    s.rng = make_uint2(__float_as_uint(d.y), __float_as_uint(d.z));
+    return s;
+}
+// Seed g's streamline before its first step.
+template <int ALGO> __device__ __forceinline__ PlainStreamline seeded_streamline(const TrackLaunch &p, int64_t g)
+{
+    const float4 s0 = reinterpret_cast<const float4 *>(p.seeds)[2 * g];
+    const float4 s1 = reinterpret_cast<const float4 *>(p.seeds)[2 * g + 1];
+    PlainStreamline s;
+    s.point = s.previous = v3(s0.x, s0.y, s0.z);
+    s.o = v3(s1.x, s1.y, s1.z);
+    s.time = 0.0f;
+    s.g = g;
+    s.n = 1;
+    s.steps = 0;
+    s.rng = make_uint2(0u, 0u);
+    if constexpr (ALGO == ALGO_DIFFUSION || ALGO == ALGO_PROBABILISTIC)
+        s.rng = seed_stream(p, p.first_seed + g);
+    return s;
+}
+
 template <int MODEL, int ALGO, int DOMAIN, int KT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(plain_min_waves<MODEL, ALGO>())))
-void track_plain_kernel(TrackLaunch p)
+void track_plain_kernel(TrackLaunch p, PlainTail tail)
 {
+    constexpr bool TAIL = has_tail<MODEL, ALGO>();
     const float step = p.algo.step_size;
     const float save = p.save_at;
     const uint32_t stride = p.field.stride;
-    int64_t g = -1;
+    const bool resume = TAIL && tail.in != nullptr;
+    const int64_t n_work = resume ? (int64_t)*tail.in_count : p.n_seeds;
+    const int lane = __lane_id();
+    uint32_t *const shard =
+        TAIL ? tail.ended + ((blockIdx.x * 4 + (threadIdx.x >> 6)) % FAST_END_SHARDS) * FAST_END_STRIDE : nullptr;
     bool drained = false;
-    V3 point = v3(0.0f, 0.0f, 0.0f), o = point, previous = point;
-    uint2 rng = make_uint2(0u, 0u);
-    uint32_t n = 0, steps = 0, hit = NO_HIT;
-    float time = 0.0f;
-    bool first = true;
+    PlainStreamline s;
+    s.g = -1;
+    s.point = s.o = s.previous = v3(0.0f, 0.0f, 0.0f);
+    s.rng = make_uint2(0u, 0u);
+    s.n = s.steps = 0;
+    s.time = 0.0f;
     SegmentCandidates near{UNSET_CELL, 0u, 0u};
+    // Streamlines that ended here and are not yet in the shard, passes since
+    // the queue was drained, and the streamlines in flight at the last count.
+    uint32_t ended = 0, passes = 0, in_flight = 0xffffffffu, counted = 0;
+    bool counting = false;
     while (true) {
-        const int64_t claimed = claim_seed(g < 0, p.queue, p.n_seeds, drained);
+        const int64_t claimed = claim_seed(s.g < 0, p.queue, n_work, drained);
         if (claimed >= 0) {
-            g = claimed;
-            const float4 s0 = reinterpret_cast<const float4 *>(p.seeds)[2 * g];
-            const float4 s1 = reinterpret_cast<const float4 *>(p.seeds)[2 * g + 1];
-            point = v3(s0.x, s0.y, s0.z);
-            o = v3(s1.x, s1.y, s1.z);
-            if constexpr (ALGO == ALGO_DIFFUSION || ALGO == ALGO_PROBABILISTIC)
-                rng = seed_stream(p, p.first_seed + g);
-            store_point(p.points, p.n_points, 0, g, point);
-            n = 1;
-            steps = 0;
-            hit = NO_HIT;
-            time = 0.0f;
-            previous = point;
-            first = true;
+            if (resume) {
+                s = saved_streamline(tail.in + 4 * claimed);
+            } else {
+                s = seeded_streamline<ALGO>(p, claimed);
+                store_point(p.points, p.n_points, 0, s.g, s.point);
+            }
+            near.cell = UNSET_CELL;
         }
-        if (__ballot(g >= 0) == 0)
+        const uint64_t live = __ballot(s.g >= 0);
+        if (live == 0)
             break;
+        if constexpr (TAIL) {
+            if (counting) {
+                uint32_t left = counted;
+#pragma unroll
+                for (int d = 32; d >= 1; d >>= 1)
+                    left += __shfl_xor(left, d);
+                in_flight = (uint32_t)n_work - min(left, (uint32_t)n_work);
+                counting = false;
+            }
+            if (in_flight < tail.stop_below) {
+                const int leader = __ffsll((unsigned long long)live) - 1;
+                const uint32_t count = (uint32_t)__popcll(live);
+                uint32_t base = 0;
+                if (lane == leader) {
+                    base = atomicAdd(tail.out_count, count);
+                    atomicAdd(shard, ended + count);
+                }
+                base = __shfl(base, leader);
+                if (s.g >= 0)
+                    save_streamline(
+                        tail.out + 4 * ((uint64_t)base + (uint32_t)__popcll(live & ((1ull << lane) - 1ull))), s);
+                break;
+            }
+        }
         bool decided = false, found = false;
         if constexpr (DOMAIN == DOMAIN_MESH) {
             uint32_t candidate;
-            wave_segment_test(p.mesh, previous, point, g >= 0 && !first, near, decided, found, candidate);
+            wave_segment_test(p.mesh, s.previous, s.point, s.g >= 0 && s.steps > 0, near, decided, found, candidate);
         }
-        if (g < 0)
-            continue;
-        // One pass of the reference loop; `stop` is its break.
-        bool stop = !(n < p.n_points && steps < p.max_steps);
-        if (!stop) {
-            if constexpr (DOMAIN == DOMAIN_MASK) {
-                stop = !mask_contains(p.mask, point);
-            } else if (!first) {
-                // The candidate lists hold every triangle that the traversal
-                // could hit, so a segment that hits none of them needs no
-                // traversal; one that does takes the traversal's answer. A
-                // lane in twenty is near a surface on a step, so nearly every
-                // wavefront traversed on every step: 60.3 -> 28.7 ms per
-                // launch of 200k SH45 seeds between two surfaces of 40k
-                // triangles.
-                const float dx = point.x - previous.x, dy = point.y - previous.y, dz = point.z - previous.z;
-                if (decided ? found : !mesh_far(p.mesh, previous, (dx * dx + dy * dy) + dz * dz)) {
-                    uint32_t tri;
-                    float t;
-                    if (bvh_segment_hit(p.mesh, previous, point, tri, t)) {
-                        hit = tri;
-                        stop = true;
+        if (s.g >= 0) {
+            // One pass of the reference loop; `stop` is its break.
+            bool stop = !(s.n < p.n_points && s.steps < p.max_steps);
+            uint32_t hit = NO_HIT;
+            if (!stop) {
+                if constexpr (DOMAIN == DOMAIN_MASK) {
+                    stop = !mask_contains(p.mask, s.point);
+                } else if (s.steps > 0) {
+                    // The candidate lists hold every triangle that the
+                    // traversal could hit, so a segment that hits none of
+                    // them needs no traversal; one that does takes the
+                    // traversal's answer. A lane in twenty is near a surface
+                    // on a step, so nearly every wavefront traversed on every
+                    // step: 60.3 -> 28.7 ms per launch of 200k SH45 seeds
+                    // between two surfaces of 40k triangles.
+                    const float dx = s.point.x - s.previous.x, dy = s.point.y - s.previous.y,
+                                dz = s.point.z - s.previous.z;
+                    if (decided ? found : !mesh_far(p.mesh, s.previous, (dx * dx + dy * dy) + dz * dz)) {
+                        uint32_t tri;
+                        float t;
+                        if (bvh_segment_hit(p.mesh, s.previous, s.point, tri, t)) {
+                            hit = tri;
+                            stop = true;
+                        }
                     }
                 }
             }
+            int64_t voxel = -1;
+            if (!stop) {
+                voxel = field_voxel(p.field, s.point);
+                stop = voxel < 0;
+            }
+            if (!stop) {
+                s.o = plain::update<MODEL, ALGO, KT>(p.algo, p.field.data + voxel * stride, s.o, s.rng);
+                s.steps++;
+                s.previous = s.point;
+                s.point.x += step * s.o.x;
+                s.point.y += step * s.o.y;
+                s.point.z += step * s.o.z;
+                s.time += step;
+                if (s.time >= save) {
+                    s.time -= save;
+                    store_point(p.points, p.n_points, s.n, s.g,
+                                v3(s.point.x - s.time * s.o.x, s.point.y - s.time * s.o.y,
+                                   s.point.z - s.time * s.o.z));
+                    s.n++;
+                }
+            } else {
+                p.lengths[s.g] = s.n;
+                p.steps[s.g] = s.steps;
+                p.hits[s.g] = hit;
+                s.g = -1;
+            }
         }
-        int64_t voxel = -1;
-        if (!stop) {
-            voxel = field_voxel(p.field, point);
-            stop = voxel < 0;
+        if constexpr (TAIL) {
+            ended += (uint32_t)__popcll(live & ~__ballot(s.g >= 0));
+            // Every eighth pass once every claim is made: this wavefront's
+            // ended streamlines to its shard, and all shards read (summed in
+            // the next pass).
+            if (tail.stop_below != 0 && drained && (++passes & 7u) == 0u) {
+                if (ended != 0 && lane == 0)
+                    atomicAdd(shard, ended);
+                ended = 0;
+                counted = lane < FAST_END_SHARDS
+                              ? __hip_atomic_load(tail.ended + lane * FAST_END_STRIDE, __ATOMIC_RELAXED,
+                                                  __HIP_MEMORY_SCOPE_AGENT)
+                              : 0u;
+                counting = true;
+            }
         }
-        if (!stop) {
-            o = plain::update<MODEL, ALGO, KT>(p.algo, p.field.data + voxel * stride, o, rng);
+    }
+    if (TAIL && tail.stop_below != 0 && ended != 0 && lane == 0 && !(in_flight < tail.stop_below))
+        atomicAdd(shard, ended);
+}
+
+// Transport and Diffusion with the SH model, 64 streamlines to a block whose
+// wavefronts share out each step: wavefront 0 sums the model value, 1 and 2
+// its two derivatives, 3 (Diffusion) draws the noise. Each holds the
+// streamlines' state and does the rest of the step alike; the parts go
+// through LDS, one barrier per step (two buffers: a wavefront writes the next
+// step's part while another still reads this one's).
+//
+// A lone wavefront issues one instruction in about four cycles, so with fewer
+// streamlines than the SIMDs have lanes a step of the one-wavefront form
+// takes its 2000 instructions and the wait for its row one after another,
+// on a quarter of the SIMDs or less. Here the longest part is about half of
+// that, and the row is asked for before the angles are taken: 5.2 -> 2.7 us
+// per step (32^3 SH45 Transport, 10k seeds, 3000 steps at most: 15.3 -> 8.2
+// ms per call), now the angles' chain, the derivative sum's products and the
+// exponential map one after another. Every sum is one wavefront's, in the
+// reference's order: same bits.
+template <int ALGO> constexpr int split_waves() { return ALGO == ALGO_DIFFUSION ? 4 : 3; }
+template <int ALGO, int DOMAIN, int KT>
+__global__ __launch_bounds__(64 * split_waves<ALGO>()) void track_split_kernel(TrackLaunch p, PlainTail tail)
+{
+    __shared__ float part[2][6][64];
+    __shared__ uint32_t boundary[2][64];
+    const int lane = threadIdx.x & 63;
+    const int role = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const bool writer = role == split_waves<ALGO>() - 1;
+    const float step = p.algo.step_size;
+    const float save = p.save_at;
+    const uint32_t stride = p.field.stride;
+    const bool resume = tail.in != nullptr;
+    const int64_t slot = (int64_t)blockIdx.x * 64 + lane;
+    bool live = slot < (resume ? (int64_t)*tail.in_count : p.n_seeds);
+    PlainStreamline s;
+    s.g = 0;
+    s.point = s.o = s.previous = v3(0.0f, 0.0f, 0.0f);
+    s.rng = make_uint2(0u, 0u);
+    s.n = s.steps = 0;
+    s.time = 0.0f;
+    if (live) {
+        if (resume) {
+            s = saved_streamline(tail.in + 4 * slot);
+        } else {
+            s = seeded_streamline<ALGO>(p, slot);
+            if (writer)
+                store_point(p.points, p.n_points, 0, s.g, s.point);
+        }
+    }
+    const int64_t g = s.g;
+    V3 point = s.point, o = s.o, previous = s.previous;
+    uint2 rng = s.rng;
+    uint32_t n = s.n, steps = s.steps;
+    float time = s.time;
+    SegmentCandidates near{UNSET_CELL, 0u, 0u};
+    int buffer = 0;
+    while (__ballot(live) != 0) {
+        // The point's row and mask value are asked for first.
+        const int64_t voxel = live ? field_voxel(p.field, point) : -1;
+        float c[45];
+        if (role < 3)
+            plain::load_sh_coefficients<KT>(p.field.data + (voxel >= 0 ? voxel : 0) * stride, p.algo.n_parameters, c);
+        bool stop = voxel < 0 || !(n < p.n_points && steps < p.max_steps);
+        if constexpr (DOMAIN == DOMAIN_MASK)
+            stop = stop || !mask_contains(p.mask, point);
+        const plain::Frame f = plain::tangent_frame(o);
+        if (role == 0) {
+            const float v = plain::sh45_sum<0>(c, f.az, f.col);
+            part[buffer][0][lane] = fmaxf(plain::softplus(v), 1e-6f);
+            part[buffer][1][lane] = plain::dsoftplus(v);
+            if constexpr (DOMAIN == DOMAIN_MESH) {
+                bool decided, found;
+                uint32_t tri = NO_HIT;
+                float t;
+                wave_segment_test(p.mesh, previous, point, live && steps > 0, near, decided, found, tri);
+                uint32_t hit = NO_HIT;
+                const float dx = point.x - previous.x, dy = point.y - previous.y, dz = point.z - previous.z;
+                if (live && steps > 0 && n < p.n_points && steps < p.max_steps &&
+                    (decided ? found : !mesh_far(p.mesh, previous, (dx * dx + dy * dy) + dz * dz)) &&
+                    bvh_segment_hit(p.mesh, previous, point, tri, t))
+                    hit = tri;
+                boundary[buffer][lane] = hit;
+            }
+        } else if (role == 1) {
+            part[buffer][2][lane] = plain::sh45_sum<1>(c, f.az, f.col);
+        } else if (role == 2) {
+            part[buffer][3][lane] = plain::sh45_sum<2>(c, f.az, f.col);
+        } else if (p.algo.noise_variance > 0.0f) {
+            part[buffer][4][lane] = live ? plain::randn(rng) : 0.0f;
+            part[buffer][5][lane] = live ? plain::randn(rng) : 0.0f;
+        }
+        __syncthreads();
+        const float m = part[buffer][0][lane], d = part[buffer][1][lane];
+        const float dtheta = part[buffer][2][lane] * d, dphi = part[buffer][3][lane] * d;
+        float r1 = 0.0f, r2 = 0.0f;
+        if (ALGO == ALGO_DIFFUSION && p.algo.noise_variance > 0.0f) {
+            r1 = part[buffer][4][lane];
+            r2 = part[buffer][5][lane];
+        }
+        uint32_t hit = NO_HIT;
+        if constexpr (DOMAIN == DOMAIN_MESH) {
+            hit = boundary[buffer][lane];
+            stop = stop || hit != NO_HIT;
+        }
+        buffer ^= 1;
+        if (live && stop) {
+            live = false;
+            if (writer) {
+                p.lengths[g] = n;
+                p.steps[g] = steps;
+                p.hits[g] = hit;
+            }
+        }
+        if (live) {
+            o = plain::drift_and_turn<ALGO>(p.algo, f, m, dtheta, dphi, o, r1, r2);
             steps++;
             previous = point;
             point.x += step * o.x;
             point.y += step * o.y;
             point.z += step * o.z;
-            first = false;
             time += step;
             if (time >= save) {
                 time -= save;
-                store_point(p.points, p.n_points, n, g,
-                            v3(point.x - time * o.x, point.y - time * o.y, point.z - time * o.z));
+                if (writer)
+                    store_point(p.points, p.n_points, n, g,
+                                v3(point.x - time * o.x, point.y - time * o.y, point.z - time * o.z));
                 n++;
             }
-            continue;
         }
-        p.lengths[g] = n;
-        p.steps[g] = steps;
-        p.hits[g] = hit;
-        g = -1;
     }
 }
 
@@ -710,42 +947,120 @@ hipError_t launch_persistent(Kernel kernel, const Launch &args, uint32_t *queue,
     return hipGetLastError();
 }
 
-template <int MODEL, int ALGO, int DOMAIN>
-hipError_t launch_plain_kt(const TrackLaunch &p, hipStream_t stream)
+__global__ void zero_tail(uint32_t *queue, uint32_t *ended, uint32_t *out_count)
 {
-    if (MODEL == MODEL_SH && p.algo.n_parameters == 45)
-        return launch_persistent(track_plain_kernel<MODEL, ALGO, DOMAIN, 45>, p, p.queue, p.n_seeds, stream);
-    return launch_persistent(track_plain_kernel<MODEL, ALGO, DOMAIN, 0>, p, p.queue, p.n_seeds, stream);
-}
-
-template <int MODEL, int ALGO>
-hipError_t launch_plain_domain(const TrackLaunch &p, hipStream_t stream)
-{
-    if (p.domain_kind == DOMAIN_MESH)
-        return launch_plain_kt<MODEL, ALGO, DOMAIN_MESH>(p, stream);
-    return launch_plain_kt<MODEL, ALGO, DOMAIN_MASK>(p, stream);
-}
-
-template <int MODEL>
-hipError_t launch_plain_algo(const TrackLaunch &p, hipStream_t stream)
-{
-    switch (p.algo.algorithm) {
-    case ALGO_DIFFUSION: return launch_plain_domain<MODEL, ALGO_DIFFUSION>(p, stream);
-    case ALGO_PROBABILISTIC: return launch_plain_domain<MODEL, ALGO_PROBABILISTIC>(p, stream);
-    case ALGO_DETERMINISTIC: return launch_plain_domain<MODEL, ALGO_DETERMINISTIC>(p, stream);
-    default: return launch_plain_domain<MODEL, ALGO_TRANSPORT>(p, stream);
+    if (threadIdx.x < FAST_END_SHARDS)
+        ended[threadIdx.x * FAST_END_STRIDE] = 0u;
+    if (threadIdx.x == 0) {
+        *queue = 0u;
+        *out_count = 0u;
     }
 }
 
-hipError_t launch_track_plain(const TrackLaunch &p, hipStream_t stream)
+// SH Transport and Diffusion launches. Up to PLAIN_SPLIT_SEEDS seeds:
+// wavefronts that share the steps (track_split_kernel). More: persistent
+// lanes, cut short when half of them are idle, then half the grid on the
+// streamlines left, and split wavefronts once PLAIN_SPLIT_SEEDS are left.
+// Without room for saved streamlines the persistent lanes run to the end.
+// 145 x 174 x 145 SH45 Diffusion, in one launch and so: 28.2 -> 24.7 ms with
+// 300k seeds, 66.0 -> 61.3 with 1M; 200k seeds between two surfaces 24.6 ->
+// 17.8 ms.
+template <int ALGO, int DOMAIN, int KT>
+hipError_t launch_plain_tail(const TrackLaunch &p, const PlainWork &w, hipStream_t stream)
+{
+    auto *const kernel = track_plain_kernel<MODEL_SH, ALGO, DOMAIN, KT>;
+    PlainTail t{};
+    t.ended = w.ended;
+    if (p.n_seeds <= PLAIN_SPLIT_SEEDS) {
+        track_split_kernel<ALGO, DOMAIN, KT>
+            <<<(unsigned)((p.n_seeds + 63) / 64), 64 * split_waves<ALGO>(), 0, stream>>>(p, t);
+        return hipGetLastError();
+    }
+    unsigned blocks = 0;
+    const hipError_t e = persistent_blocks(kernel, p.n_seeds, &blocks);
+    if (e != hipSuccess)
+        return e;
+    if (w.saved[0] == nullptr || w.saved[1] == nullptr) {
+        zero_u32_kernel<<<1, 64, 0, stream>>>(p.queue);
+        kernel<<<blocks, 256, 0, stream>>>(p, t);
+        return hipGetLastError();
+    }
+    const int64_t half = std::min<int64_t>(std::min<int64_t>(p.n_seeds, (int64_t)blocks * 256) / 2, PLAIN_HALF_ROOM);
+    if (half > 2 * PLAIN_SPLIT_SEEDS) {
+        t.out = w.saved[0];
+        t.out_count = w.count[0];
+        t.stop_below = (uint32_t)half;
+        zero_tail<<<1, 64, 0, stream>>>(p.queue, t.ended, t.out_count);
+        kernel<<<blocks, 256, 0, stream>>>(p, t);
+        t.in = w.saved[0];
+        t.in_count = w.count[0];
+        blocks = (unsigned)((half + 255) / 256);
+    }
+    t.out = w.saved[1];
+    t.out_count = w.count[1];
+    t.stop_below = PLAIN_SPLIT_SEEDS;
+    zero_tail<<<1, 64, 0, stream>>>(p.queue, t.ended, t.out_count);
+    kernel<<<blocks, 256, 0, stream>>>(p, t);
+    t.in = t.out;
+    t.in_count = t.out_count;
+    t.stop_below = 0;
+    track_split_kernel<ALGO, DOMAIN, KT>
+        <<<(unsigned)(PLAIN_SPLIT_SEEDS / 64), 64 * split_waves<ALGO>(), 0, stream>>>(p, t);
+    return hipGetLastError();
+}
+
+template <int MODEL, int ALGO, int DOMAIN, int KT>
+hipError_t launch_plain_tracks(const TrackLaunch &p, const PlainWork &w, hipStream_t stream)
+{
+    if constexpr (has_tail<MODEL, ALGO>()) {
+        return launch_plain_tail<ALGO, DOMAIN, KT>(p, w, stream);
+    } else {
+        unsigned blocks = 0;
+        const hipError_t e = persistent_blocks(track_plain_kernel<MODEL, ALGO, DOMAIN, KT>, p.n_seeds, &blocks);
+        if (e != hipSuccess)
+            return e;
+        zero_u32_kernel<<<1, 64, 0, stream>>>(p.queue);
+        track_plain_kernel<MODEL, ALGO, DOMAIN, KT><<<blocks, 256, 0, stream>>>(p, PlainTail{});
+        return hipGetLastError();
+    }
+}
+
+template <int MODEL, int ALGO, int DOMAIN>
+hipError_t launch_plain_kt(const TrackLaunch &p, const PlainWork &w, hipStream_t stream)
+{
+    if (MODEL == MODEL_SH && p.algo.n_parameters == 45)
+        return launch_plain_tracks<MODEL, ALGO, DOMAIN, 45>(p, w, stream);
+    return launch_plain_tracks<MODEL, ALGO, DOMAIN, 0>(p, w, stream);
+}
+
+template <int MODEL, int ALGO>
+hipError_t launch_plain_domain(const TrackLaunch &p, const PlainWork &w, hipStream_t stream)
+{
+    if (p.domain_kind == DOMAIN_MESH)
+        return launch_plain_kt<MODEL, ALGO, DOMAIN_MESH>(p, w, stream);
+    return launch_plain_kt<MODEL, ALGO, DOMAIN_MASK>(p, w, stream);
+}
+
+template <int MODEL>
+hipError_t launch_plain_algo(const TrackLaunch &p, const PlainWork &w, hipStream_t stream)
+{
+    switch (p.algo.algorithm) {
+    case ALGO_DIFFUSION: return launch_plain_domain<MODEL, ALGO_DIFFUSION>(p, w, stream);
+    case ALGO_PROBABILISTIC: return launch_plain_domain<MODEL, ALGO_PROBABILISTIC>(p, w, stream);
+    case ALGO_DETERMINISTIC: return launch_plain_domain<MODEL, ALGO_DETERMINISTIC>(p, w, stream);
+    default: return launch_plain_domain<MODEL, ALGO_TRANSPORT>(p, w, stream);
+    }
+}
+
+hipError_t launch_track_plain(const TrackLaunch &p, const PlainWork &w, hipStream_t stream)
 {
     if (p.n_seeds == 0)
         return hipSuccess;
     if (!p.queue)
         return hipErrorInvalidValue;
     if (p.algo.model == MODEL_DTI)
-        return launch_plain_algo<MODEL_DTI>(p, stream);
-    return launch_plain_algo<MODEL_SH>(p, stream);
+        return launch_plain_algo<MODEL_DTI>(p, w, stream);
+    return launch_plain_algo<MODEL_SH>(p, w, stream);
 }
 
 template <int MODEL, int ALGO>

@@ -83,6 +83,17 @@ __device__ __forceinline__ void sh45_contract(const float c[45], float phi, floa
     ph = sph;
 }
 
+// One of the three sums of the contraction: 0 the value, 1 d/dtheta, 2
+// (d/dphi)/sin(theta).
+template <int SUM> __device__ __forceinline__ float sh45_sum(const float c[45], float phi, float theta)
+{
+    float sum = 0.0f;
+#define TGK_ACC(i, Y, DP, DT) sum += c[i] * (SUM == 0 ? (Y) : SUM == 1 ? (DT) : (DP));
+#include "tgk_sh45_body.inc"
+#undef TGK_ACC
+    return sum;
+}
+
 // No use for the basis values beyond the contraction.
 struct NoTerms {
     __device__ __forceinline__ void operator()(int, float) const {}
@@ -396,6 +407,47 @@ __device__ __forceinline__ V3 deterministic_update(const AlgoParams &a, const fl
     return o;
 }
 
+// The angles of o, their sines and cosines, and the tangent frame they give.
+struct Frame {
+    float az, col, sp, cp, st, ct;
+};
+__device__ __forceinline__ Frame tangent_frame(V3 o)
+{
+    Frame f;
+    cart2sph(o, f.az, f.col);
+    dm::sincosf_small(f.az, &f.sp, &f.cp);
+    dm::sincosf_small(f.col, &f.st, &f.ct);
+    return f;
+}
+
+// Transport / Diffusion from the model at o (value bounded from below by
+// 1e-6, derivatives) and, for Diffusion with a positive noise variance, its
+// two normal draws.
+template <int ALGO>
+__device__ __forceinline__ V3 drift_and_turn(const AlgoParams &a, const Frame &f, float m, float dtheta, float dphi,
+                                             V3 o, float r1, float r2)
+{
+    const float etx = f.ct * f.cp, ety = f.ct * f.sp, etz = -f.st;
+    const float epx = -f.sp, epy = f.cp, epz = 0.0f;
+    const float dx = (dtheta * etx + dphi * epx) / m;
+    const float dy = (dtheta * ety + dphi * epy) / m;
+    const float dz = (dtheta * etz + dphi * epz) / m;
+    const float scale_drift = a.gamma * a.step_size;
+    if constexpr (ALGO == ALGO_TRANSPORT) {
+        return exps2(o, v3(scale_drift * dx, scale_drift * dy, scale_drift * dz));
+    } else {
+        float nx = 0.0f, ny = 0.0f, nz = 0.0f;
+        if (a.noise_variance > 0.0f) {
+            nx = r1 * etx + r2 * epx;
+            ny = r1 * ety + r2 * epy;
+            nz = r1 * etz + r2 * epz;
+        }
+        const float scale_noise = tgk_sqrtf(a.noise_variance * a.gamma * a.step_size);
+        return exps2(o, v3(scale_drift * dx + scale_noise * nx, scale_drift * dy + scale_noise * ny,
+                           scale_drift * dz + scale_noise * nz));
+    }
+}
+
 // algorithm.py:83-112 (Transport), 198-228 (Diffusion), 305-376
 // (Probabilistic) and 484-617 (Deterministic); for Diffusion the left randn
 // of the noise expression is drawn first. For the SH model under Transport
@@ -411,32 +463,13 @@ __device__ __forceinline__ V3 update(const AlgoParams &a, const float *__restric
     if constexpr (ALGO == ALGO_DETERMINISTIC)
         return deterministic_update<MODEL, KT>(a, row, o);
     const ModelValue mv = model_evaluate<MODEL, KT>(row, a.n_parameters, o, terms);
-    float az, col, sp, cp, st, ct;
-    cart2sph(o, az, col);
-    dm::sincosf_small(az, &sp, &cp);
-    dm::sincosf_small(col, &st, &ct);
-    const float etx = ct * cp, ety = ct * sp, etz = -st;
-    const float epx = -sp, epy = cp, epz = 0.0f;
-    const float m = fmaxf(mv.value, 1e-6f);
-    const float dx = (mv.dtheta * etx + mv.dphi * epx) / m;
-    const float dy = (mv.dtheta * ety + mv.dphi * epy) / m;
-    const float dz = (mv.dtheta * etz + mv.dphi * epz) / m;
-    const float scale_drift = a.gamma * a.step_size;
-    if constexpr (ALGO == ALGO_TRANSPORT) {
-        return exps2(o, v3(scale_drift * dx, scale_drift * dy, scale_drift * dz));
-    } else {
-        float nx = 0.0f, ny = 0.0f, nz = 0.0f;
-        if (a.noise_variance > 0.0f) {
-            const float r1 = randn(rng);
-            const float r2 = randn(rng);
-            nx = r1 * etx + r2 * epx;
-            ny = r1 * ety + r2 * epy;
-            nz = r1 * etz + r2 * epz;
-        }
-        const float scale_noise = tgk_sqrtf(a.noise_variance * a.gamma * a.step_size);
-        return exps2(o, v3(scale_drift * dx + scale_noise * nx, scale_drift * dy + scale_noise * ny,
-                           scale_drift * dz + scale_noise * nz));
+    const Frame f = tangent_frame(o);
+    float r1 = 0.0f, r2 = 0.0f;
+    if (ALGO == ALGO_DIFFUSION && a.noise_variance > 0.0f) {
+        r1 = randn(rng);
+        r2 = randn(rng);
     }
+    return drift_and_turn<ALGO>(a, f, fmaxf(mv.value, 1e-6f), mv.dtheta, mv.dphi, o, r1, r2);
 }
 
 }  // namespace plain
