@@ -129,6 +129,14 @@ int tgk_track_timed(tgk_runtime *rt, const tgk_domain *domain, const tgk_field *
                     int32_t path, const float *seeds, int64_t n_seeds, uint32_t n_points, float save_at,
                     int32_t repeats, float *milliseconds, uint64_t *steps);
 
+/* No counterpart in the reference (its results come back in memory of its
+ * own, opencl.py:200-230). Page-locked host memory of `bytes` bytes: as the
+ * output of a blocking call it is filled by DMA at the link's rate, where
+ * pageable memory is staged through buffers of the driver and faulted in page
+ * by page. Any thread may free it, once, after the last use. */
+int tgk_host_alloc(size_t bytes, void **ptr);
+int tgk_host_free(void *ptr);
+
 /* ------------------------------------------------------ field, domain --- */
 
 /* Replaces field.Image.get_args (field.py:117-122): uploads the (X, Y, Z, K)

@@ -50,6 +50,13 @@ def _validate_algorithm(tracking_algorithm: BaseAlgorithm) -> None:
         raise TypeError("algorithm must be a BaseAlgorithm instance.")
 
 
+def _nonzero_domain(values, affine):
+    """The default domain of an image field: its nonzero voxels. Only for
+    callers without a domain of their own: it reads the whole volume (25 ms
+    at 97x116x97x45)."""
+    return Nifti1Image(np.any(values != 0, axis=-1).astype(np.uint8), affine)
+
+
 def tractogram(
     field,
     seeds: npt.NDArray[np.float32] | int,
@@ -88,18 +95,14 @@ def tractogram(
         if field.ndim != 4:
             raise ValueError("The tracking image must be four-dimensional.")
         tracking_field = field_module.Image(field)
-        domain_image = Nifti1Image(
-            np.any(np.asanyarray(field.dataobj) != 0, axis=-1).astype(np.uint8), field.affine
-        )
+        domain_image = _nonzero_domain(np.asanyarray(field.dataobj), field.affine) if domain is None else None
         local_model = local.from_shape(field.shape)
     elif isinstance(field, field_module.BaseField):
         tracking_field = field
         local_model = local.from_shape((field.n_parameters,)) if algorithm is None else None
-        if isinstance(field, field_module.Image):
-            affine = np.linalg.inv(field.inverse_affine)
-            domain_image = Nifti1Image(np.any(field.values != 0, axis=-1).astype(np.uint8), affine)
-        else:
-            domain_image = None
+        domain_image = None
+        if domain is None and isinstance(field, field_module.Image):
+            domain_image = _nonzero_domain(field.values, np.linalg.inv(field.inverse_affine))
     else:
         raise TypeError("field must be a Nifti1Image or a BaseField instance.")
 
@@ -195,9 +198,7 @@ def tod(
         if field.ndim != 4:
             raise ValueError("The tracking image must be four-dimensional.")
         tracking_field = field_module.Image(field)
-        domain_image = Nifti1Image(
-            np.any(np.asanyarray(field.dataobj) != 0, axis=-1).astype(np.uint8), field.affine
-        )
+        domain_image = _nonzero_domain(np.asanyarray(field.dataobj), field.affine) if domain is None else None
         local_model = local.from_shape(field.shape)
         grid_shape, grid_affine, grid_like = tuple(field.shape[:3]), field.affine, field
     elif isinstance(field, field_module.BaseField):
@@ -205,7 +206,7 @@ def tod(
         local_model = local.from_shape((field.n_parameters,)) if algorithm is None else None
         if isinstance(field, field_module.Image):
             affine = np.linalg.inv(field.inverse_affine)
-            domain_image = Nifti1Image(np.any(field.values != 0, axis=-1).astype(np.uint8), affine)
+            domain_image = _nonzero_domain(field.values, affine) if domain is None else None
             grid_shape, grid_affine, grid_like = tuple(int(s) for s in field.dims[:3]), affine, None
         else:
             domain_image = grid_shape = grid_affine = grid_like = None
@@ -314,17 +315,14 @@ def connectome(
         if len(field.shape) != 4:
             raise ValueError("The tracking image must be four-dimensional.")
         tracking_field = field_module.Image(field)
-        domain_image = Nifti1Image(np.any(np.asanyarray(field.dataobj) != 0, axis=-1).astype(np.uint8),
-                                   field.affine)
+        domain_image = _nonzero_domain(np.asanyarray(field.dataobj), field.affine) if domain is None else None
         local_model = local.from_shape(field.shape)
     elif isinstance(field, field_module.BaseField):
         tracking_field = field
         local_model = local.from_shape((field.n_parameters,)) if algorithm is None else None
-        if isinstance(field, field_module.Image):
-            domain_image = Nifti1Image(np.any(field.values != 0, axis=-1).astype(np.uint8),
-                                       np.linalg.inv(field.inverse_affine))
-        else:
-            domain_image = None
+        domain_image = None
+        if domain is None and isinstance(field, field_module.Image):
+            domain_image = _nonzero_domain(field.values, np.linalg.inv(field.inverse_affine))
     else:
         raise TypeError("field must be a Nifti1Image or a BaseField instance.")
 

@@ -105,6 +105,7 @@ struct tgk_runtime {
     DeviceBuffer plain_saved;       // streamlines saved between launches of the plain kernels (allocated once)
     DeviceBuffer fast_counters;     // claim counter and ended-streamline shards of the fast kernel
     TrackBuffers track_buffers;     // tgk_track's working buffers
+    DeviceBuffer product;           // tgk_tod's grid, tgk_connectome's entries (kept, as those)
     DeviceBuffer seeds_table;  // prepared FOD-seeding table for seeds_key
     int32_t seeds_key[3] = {-1, -1, -1};  // model, K, method
     bool capturing = false;    // the stream is being recorded into a graph
@@ -442,6 +443,27 @@ int tgk_runtime_destroy(tgk_runtime *rt)
         (void)hipStreamDestroy(rt->stream);
     }
     delete rt;
+    return TGK_OK;
+}
+
+int tgk_host_alloc(size_t bytes, void **ptr)
+{
+    if (!ptr || bytes == 0)
+        return fail(TGK_ERR_INVALID, "NULL argument or empty allocation");
+    *ptr = nullptr;
+    const hipError_t e = hipHostMalloc(ptr, bytes, hipHostMallocDefault);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();  // clear the failed allocation's error
+        *ptr = nullptr;
+        return fail(TGK_ERR_NO_MEMORY, "page-locked memory (%zu bytes): %s", bytes, hipGetErrorString(e));
+    }
+    return TGK_OK;
+}
+
+int tgk_host_free(void *ptr)
+{
+    if (ptr)
+        TGK_HIP(hipHostFree(ptr), "hipHostFree");
     return TGK_OK;
 }
 
@@ -1568,15 +1590,10 @@ int tgk_connectome(tgk_runtime *rt, const tgk_domain *domain, const tgk_domain *
         return TGK_OK;
     if (int r = select_device(rt))
         return r;
-    Staging st;
-    int32_t *drows, *dcols;
-    float *dweights;
-    if (int r = st.out((size_t)n_seeds * 9, &drows))
+    if (int r = reserve(rt, rt->product, (size_t)n_seeds * 9 * 12, "connectome entries"))
         return r;
-    if (int r = st.out((size_t)n_seeds * 9, &dcols))
-        return r;
-    if (int r = st.out((size_t)n_seeds * 9, &dweights))
-        return r;
+    int32_t *drows = rt->product.as<int32_t>(), *dcols = drows + 9 * n_seeds;
+    float *dweights = reinterpret_cast<float *>(dcols + 9 * n_seeds);
     tgk::ConnectomeLaunch c;
     memset(&c, 0, sizeof c);
     c.mask = mask_view(domain);
@@ -1713,10 +1730,9 @@ int tgk_tod(tgk_runtime *rt, const tgk_domain *domain, const tgk_domain *boundar
         return TGK_OK;
     if (int r = select_device(rt))
         return r;
-    Staging st;
-    float *dout;
-    if (int r = st.out((size_t)n_values, &dout))
+    if (int r = reserve(rt, rt->product, (size_t)n_values * sizeof(float), "output grid"))
         return r;
+    float *dout = rt->product.as<float>();
     if (int r = enqueue_tod(rt, const_cast<tgk_field *>(field), algorithm, path, t, n_values, normalize, dout))
         return r;
     return fetch(coefficients, dout, (size_t)n_values, rt->stream);
