@@ -896,6 +896,7 @@ int fast_launch(tgk_runtime *rt, tgk_field *field, const tgk_algorithm *algorith
     f->track = p;
     char *words = rt->queue.as<char>();
     f->claims = rt->fast_counters.as<uint32_t>();
+    f->tail = rt->fast_counters.as<uint32_t>() + 8;
     f->ended = rt->fast_counters.as<uint32_t>() + 32;
     f->stats = reinterpret_cast<unsigned long long *>(words + FAST_STATS_OFFSET);
     f->precision = field->fast_precision;

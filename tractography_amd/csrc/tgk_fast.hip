@@ -494,8 +494,9 @@ template <int MODEL, int ALGO, int DOMAIN, int LMAX, int S = 0> constexpr int fa
 // `stop_below` (half its work), every wavefront saves its live lanes and
 // ends, and the next generation resumes them packed into full wavefronts,
 // a quarter or half as many per SIMD, each running correspondingly faster.
-// The last generation, or one with little work, runs to completion. Which
-// lane tracks which streamline, and when, changes no result.
+// The last generation, or one with little work, runs to completion, by
+// track_split_fast_kernel where there is one. Which lane tracks which
+// streamline, and when, changes no result.
 template <int MODEL, int ALGO, int DOMAIN, int LMAX, int S>
 __global__ __launch_bounds__((shape_block<MODEL, ALGO, LMAX, S>()))
 __attribute__((amdgpu_waves_per_eu(fast_min_waves<MODEL, ALGO, DOMAIN, LMAX, S>())))
@@ -671,6 +672,301 @@ void track_fast_kernel(FastLaunch f)
     if (lane_id == 0) {
         atomicAdd(&f.stats[0], (unsigned long long)rows_read);
         atomicAdd(&f.stats[1], (unsigned long long)masks_read);
+    }
+}
+
+// Order-8 SH Transport and Diffusion, 64 streamlines to a block of four
+// wavefronts that share out each step: 0, 1 and 2 evaluate orders 0-2, 3-5
+// and 6-8 of the model from their parts of the row, 3 draws the noise, tests
+// the boundary, stores the points and reads ahead. All hold the streamlines'
+// state and do the rest of the step alike; the parts go through LDS, one
+// barrier per step (two buffers: a wavefront writes the next step's parts
+// while another still reads this one's).
+//
+// A lone wavefront of track_fast_kernel issues its 650 instructions per step
+// at about one per four cycles and then waits for the row, a third of the
+// step. Here the chain is some 300 instructions, and the row comes from the
+// CU's own cache where the streamline keeps its direction: 145 x 174 x 145
+// SH45 Diffusion, 5000 seeds, 3000 steps at most: 5.2 -> 3.8 ms per call;
+// 32^3 SH45 Transport, 10k seeds: 5.1 -> 3.95.
+// Bound by that chain: row, three orders, exchange, sums, exponential map.
+// Every sum keeps its order: same bits.
+constexpr int FAST_SPLIT_WAVES = 4;
+// float4 columns FIRST .. FIRST + N - 1 of a row, and its coefficients from
+// the first of them on.
+template <int FIRST, int N> __device__ __forceinline__ void load_part(const float4 *row, float4 *part)
+{
+#pragma unroll
+    for (int j = 0; j < N; j++)
+        part[j] = row[FIRST + j];
+}
+
+template <int FIRST, int N> __device__ __forceinline__ void read_part(const float4 *part, float *q)
+{
+#pragma unroll
+    for (int j = 0; j < N; j++) {
+        q[4 * (FIRST + j)] = part[j].x;
+        q[4 * (FIRST + j) + 1] = part[j].y;
+        q[4 * (FIRST + j) + 2] = part[j].z;
+        q[4 * (FIRST + j) + 3] = part[j].w;
+    }
+}
+
+__device__ __forceinline__ void put_term(float4 *at, const fast::CartesianTerm &t)
+{
+    *at = make_float4(t.v, t.gx, t.gy, t.gz);
+}
+
+template <int M> __device__ __forceinline__ void add_put_term(const float4 *at, fast::Cartesian &g)
+{
+    const float4 t = *at;
+    fast::add_term<M>(fast::CartesianTerm{t.x, t.y, t.z, t.w}, g);
+}
+
+template <int ALGO, int DOMAIN>
+__global__ __launch_bounds__(64 * FAST_SPLIT_WAVES) void track_split_fast_kernel(FastLaunch f)
+{
+    constexpr int LMAX = 8;
+    __shared__ float4 terms[2][7][64];       // orders 0-2 summed, then orders 3 to 8
+    __shared__ float2 noise[2][64];
+    __shared__ uint32_t test[2][64];         // mask domains: the mask value; mesh domains: the triangle hit
+    const TrackLaunch &p = f.track;
+    const int lane = threadIdx.x & 63;
+    const int role = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const float *coeffs = static_cast<const float *>(f.coeffs);
+    const uint32_t cstride = f.coeff_stride;
+    const float step = p.algo.step_size;
+    const bool resume = f.cont_in != nullptr;
+    const uint32_t n_work = resume ? f.tail[0] : (uint32_t)p.n_seeds;
+    const float4 *const saved = resume && f.tail[1] != 0 ? f.cont[1] : f.cont[0];
+    uint64_t reads = 0;                      // rows (wavefront 0), mask values (2)
+    int buffer = 0;
+    for (uint32_t base = blockIdx.x * 64; base < n_work; base += gridDim.x * 64) {
+        const uint32_t j = base + lane;
+        bool live = j < n_work;
+        Lane<1> L;
+        L.g = 0;
+        L.point = L.o = L.previous = v3(0.0f, 0.0f, 0.0f);
+        L.rng = make_uint2(0u, 0u);
+        L.time = 0.0;
+        L.n = L.steps = 0;
+        if (live) {
+            if (resume) {
+                resume_lane<DOMAIN, 1>(saved + FAST_CONTINUATION_VEC4 * (uint64_t)j, L);
+            } else {
+                L.g = (int32_t)j;
+                const float4 s0 = reinterpret_cast<const float4 *>(p.seeds)[2 * (uint64_t)j];
+                const float4 s1 = reinterpret_cast<const float4 *>(p.seeds)[2 * (uint64_t)j + 1];
+                L.point = L.previous = v3(s0.x, s0.y, s0.z);
+                L.o = v3(s1.x, s1.y, s1.z);
+                if (ALGO == ALGO_DIFFUSION && role == 3)
+                    L.rng = seed_stream(p, p.first_seed + L.g);
+                L.n = 1;
+            }
+        }
+        float *const row = p.points + (int64_t)L.g * p.n_points * 3;
+        if (live && !resume && role == 3) {
+            row[0] = L.point.x;
+            row[1] = L.point.y;
+            row[2] = L.point.z;
+        }
+        L.field_cell = L.mask_cell = L.near.cell = UNSET_CELL;
+        L.mask_value = 0;
+        float4 part[6];
+#pragma unroll
+        for (int i = 0; i < 6; i++)
+            part[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        float ahead0 = 0.0f, ahead1 = 0.0f;
+        // As track_fast_kernel counts: a streamline's first two requests, made
+        // in one iteration there, count once, and a mask value not at all
+        // when the second leaves the image.
+        uint64_t first = 0;
+        int request = 0;
+        const auto count_reads = [&](bool read, bool left) {
+            const uint64_t lanes = __ballot(read);
+            reads += (uint64_t)__popcll(request == 1 ? lanes & ~first : lanes);
+            if (request == 1)
+                reads -= (uint64_t)__popcll(__ballot(left) & first);
+            first = lanes;
+            request = min(request + 1, 2);
+        };
+        // The loads above end here: a wait left to their first use would
+        // stand inside the loop, where it waits for everything in flight.
+        __builtin_amdgcn_s_waitcnt(0);
+        while (true) {
+            // This point's cells, and its row's part on a change of cell.
+            uint32_t cell = NO_CELL;
+            {
+                const float fx = affine_row(p.field.inv, 0, L.point);
+                const float fy = affine_row(p.field.inv, 1, L.point);
+                const float fz = affine_row(p.field.inv, 2, L.point);
+                cell = grid_cell(rintf(fx), rintf(fy), rintf(fz), p.field.dims);
+                if (DOMAIN == DOMAIN_MASK && role == 2) {
+                    float mx = fx, my = fy, mz = fz;
+                    if (f.shared_affine == 0) {
+                        mx = affine_row(p.mask.inv, 0, L.point);
+                        my = affine_row(p.mask.inv, 1, L.point);
+                        mz = affine_row(p.mask.inv, 2, L.point);
+                    }
+                    const uint32_t m =
+                        grid_cell(floorf(mx + 0.5f), floorf(my + 0.5f), floorf(mz + 0.5f), p.mask.dims);
+                    const bool read = live && m != L.mask_cell && m != NO_CELL;
+                    count_reads(read, live && m == NO_CELL && m != L.mask_cell);
+                    if (live && m != L.mask_cell) {
+                        L.mask_cell = m;
+                        L.mask_value = 0;
+                        if (m != NO_CELL)
+                            L.mask_value = p.mask.mask[m];
+                    }
+                }
+            }
+            const bool change = live && cell != NO_CELL && cell != L.field_cell;
+            if (role == 0)
+                count_reads(change, false);
+            if (change) {
+                L.field_cell = cell;
+                const float4 *at = reinterpret_cast<const float4 *>(coeffs + (int64_t)cell * cstride);
+                if (role == 0)
+                    load_part<0, 6>(at, part);
+                else if (role == 1)
+                    load_part<5, 5>(at, part);
+                else if (role == 2)
+                    load_part<9, 3>(at, part);
+            }
+            const V3 n = fast::unit_direction(L.o);
+            const float w = n.z * n.z;
+            float q[48];
+            if (role == 0) {
+                read_part<0, 6>(part, q);
+                const fast::Cartesian g = fast::sh_cartesian<LMAX, 2>(q, n);
+                terms[buffer][0][lane] = make_float4(g.value, g.gx, g.gy, g.gz);
+            } else if (role < 3) {
+                // u^2, as the sums over all orders reach it.
+                float pr = n.x * n.x - n.y * n.y, pi = n.x * n.y + n.y * n.x;
+                if (role == 1) {
+                    read_part<5, 5>(part, q);
+                    put_term(&terms[buffer][1][lane], fast::sh_cartesian_term<LMAX, 3>(q, n.z, w, n.x, n.y, pr, pi));
+                    put_term(&terms[buffer][2][lane], fast::sh_cartesian_term<LMAX, 4>(q, n.z, w, n.x, n.y, pr, pi));
+                    put_term(&terms[buffer][3][lane], fast::sh_cartesian_term<LMAX, 5>(q, n.z, w, n.x, n.y, pr, pi));
+                } else {
+                    read_part<9, 3>(part, q);
+#pragma unroll
+                    for (int m = 3; m <= 5; m++) {
+                        const float ur = pr * n.x - pi * n.y;
+                        pi = pr * n.y + pi * n.x;
+                        pr = ur;
+                    }
+                    put_term(&terms[buffer][4][lane], fast::sh_cartesian_term<LMAX, 6>(q, n.z, w, n.x, n.y, pr, pi));
+                    put_term(&terms[buffer][5][lane], fast::sh_cartesian_term<LMAX, 7>(q, n.z, w, n.x, n.y, pr, pi));
+                    put_term(&terms[buffer][6][lane], fast::sh_cartesian_term<LMAX, 8>(q, n.z, w, n.x, n.y, pr, pi));
+                    if constexpr (DOMAIN == DOMAIN_MASK)
+                        test[buffer][lane] = L.mask_value;
+                }
+            } else {
+                if constexpr (ALGO == ALGO_DIFFUSION) {
+                    fast::Noise nz{0.0f, 0.0f};
+                    if (live)
+                        nz = fast::draw_noise<ALGO>(p.algo, L.rng);
+                    noise[buffer][lane] = make_float2(nz.r1, nz.r2);
+                }
+                if constexpr (DOMAIN == DOMAIN_MESH) {
+                    bool decided = false, found = false;
+                    uint32_t tri = 0, hit = NO_HIT;
+                    wave_segment_test(p.mesh, L.previous, L.point, live && L.steps > 0, L.near, decided, found, tri);
+                    if (live && L.steps > 0 && L.n < p.n_points && L.steps < p.max_steps) {
+                        if (found) {
+                            hit = tri;
+                        } else if (!decided) {
+                            float t;
+                            const float dx = L.point.x - L.previous.x, dy = L.point.y - L.previous.y,
+                                        dz = L.point.z - L.previous.z;
+                            if (!mesh_far(p.mesh, L.previous, dx * dx + dy * dy + dz * dz) &&
+                                bvh_segment_hit(p.mesh, L.previous, L.point, tri, t))
+                                hit = tri;
+                        }
+                    }
+                    test[buffer][lane] = hit;
+                }
+            }
+            __syncthreads();
+            uint32_t hit = NO_HIT;
+            bool stop = !(L.n < p.n_points && L.steps < p.max_steps) || cell == NO_CELL;
+            if constexpr (DOMAIN == DOMAIN_MASK) {
+                stop = stop || test[buffer][lane] == 0u;
+            } else {
+                hit = test[buffer][lane];
+                stop = stop || hit != NO_HIT;
+            }
+            if (live && stop) {
+                live = false;
+                if (role == 3) {
+                    p.lengths[L.g] = L.n;
+                    p.steps[L.g] = L.steps;
+                    p.hits[L.g] = hit;
+                }
+            }
+            if (__ballot(live) == 0)
+                break;
+            const float4 g0 = terms[buffer][0][lane];
+            fast::Cartesian g{g0.x, g0.y, g0.z, g0.w};
+            add_put_term<3>(&terms[buffer][1][lane], g);
+            add_put_term<4>(&terms[buffer][2][lane], g);
+            add_put_term<5>(&terms[buffer][3][lane], g);
+            add_put_term<6>(&terms[buffer][4][lane], g);
+            add_put_term<7>(&terms[buffer][5][lane], g);
+            add_put_term<8>(&terms[buffer][6][lane], g);
+            fast::Noise nz{0.0f, 0.0f};
+            if constexpr (ALGO == ALGO_DIFFUSION) {
+                const float2 drawn = noise[buffer][lane];
+                nz = fast::Noise{drawn.x, drawn.y};
+            }
+            buffer ^= 1;
+            if (live) {
+                L.o = fast::cartesian_turn<ALGO>(p.algo, n, g, L.o, nz);
+                L.steps++;
+                if constexpr (DOMAIN == DOMAIN_MESH)
+                    L.previous = L.point;
+                L.point = v3(L.point.x + step * L.o.x, L.point.y + step * L.o.y, L.point.z + step * L.o.z);
+                L.time += (double)step;
+                const bool save = L.time >= (double)p.save_at;
+                if (save)
+                    L.time -= (double)p.save_at;
+                if (role == 3) {
+                    // The last step's reads ahead have arrived (waited for
+                    // here, before the store that would be waited for too).
+                    asm volatile("" ::"v"(ahead0), "v"(ahead1));
+                    if (save) {
+                        const float t = (float)L.time;
+                        float *at = row + 3 * (int64_t)L.n;
+                        at[0] = L.point.x - t * L.o.x;
+                        at[1] = L.point.y - t * L.o.y;
+                        at[2] = L.point.z - t * L.o.z;
+                    }
+                    // The lines of the row one straight step ahead, towards this
+                    // CU, a step before the others ask for them.
+                    const V3 next = v3(L.point.x + step * L.o.x, L.point.y + step * L.o.y, L.point.z + step * L.o.z);
+                    const uint32_t c = grid_cell(rintf(affine_row(p.field.inv, 0, next)),
+                                                 rintf(affine_row(p.field.inv, 1, next)),
+                                                 rintf(affine_row(p.field.inv, 2, next)), p.field.dims);
+                    if (c != NO_CELL && c != L.field_cell) {
+                        const float *at = coeffs + (int64_t)c * cstride;
+                        ahead0 = at[0];
+                        ahead1 = at[32];
+                    }
+                }
+                L.n += save ? 1u : 0u;
+            }
+        }
+        // Ended at the break after a barrier: every wavefront is past the
+        // parts it reads there but this one's buffer, so the next 64
+        // streamlines start on the other.
+        buffer ^= 1;
+    }
+    if (lane == 0 && reads != 0) {
+        if (role == 0)
+            atomicAdd(&f.stats[0], (unsigned long long)reads);
+        else if (role == 2)
+            atomicAdd(&f.stats[1], (unsigned long long)reads);
     }
 }
 
@@ -1057,18 +1353,30 @@ __global__ void zero_counter(uint32_t *counter) { *counter = 0u; }
 // A generation's claim counter, ended-streamline shards and saved-streamline
 // count; before generation 0 also the launch's row and mask read totals.
 // One block of 64 threads.
-__global__ void zero_generation(uint32_t *claims, uint32_t *ended, uint32_t *cont_count, unsigned long long *stats)
+// Clears a generation's counters. Streamlines that the generation would run
+// to their ends (fewer than twice min_repack, or the last generation's) go to
+// track_split_fast_kernel instead where it may take them (up to split_limit):
+// their buffer and number to f.tail, and none to this generation.
+__global__ void zero_generation(FastLaunch f, bool first, uint32_t split_limit)
 {
     const int t = threadIdx.x;
     if (t < FAST_END_SHARDS)
-        ended[t * FAST_END_STRIDE] = 0u;
+        f.ended[t * FAST_END_STRIDE] = 0u;
     if (t == 0) {
-        *claims = 0u;
-        *cont_count = 0u;
-        if (stats) {
-            stats[0] = 0ull;
-            stats[1] = 0ull;
+        *f.claims = 0u;
+        if (first) {
+            f.stats[0] = 0ull;
+            f.stats[1] = 0ull;
+            f.tail[0] = 0u;
+        } else {
+            const uint32_t work = *f.cont_in_count;
+            if (work != 0 && work <= split_limit && (f.last || work / 2 < f.min_repack)) {
+                f.tail[0] = work;
+                f.tail[1] = f.cont_in == f.cont[1];
+                *f.cont_in_count = 0u;
+            }
         }
+        *f.cont_out_count = 0u;
     }
 }
 
@@ -1311,18 +1619,28 @@ hipError_t launch_group(const FastLaunch &f, int grid_blocks, bool query, hipStr
             g.group_jump[b] = jump_multiplier(2 * per_lane * b);
         g.group_jump[fast::GROUP_LANES] = jump_multiplier(2 * (uint64_t)f.track.algo.n_samples);
     }
-    zero_generation<<<1, 64, 0, stream>>>(f.claims, f.ended, f.cont_count[0], f.stats);
+    g.cont_out_count = f.cont_count[0];
+    zero_generation<<<1, 64, 0, stream>>>(g, true, 0u);
     track_group_kernel<MODEL, ALGO, DOMAIN, LMAX>
         <<<(unsigned)std::min<int64_t>(grid_blocks, needed), 256, 0, stream>>>(g);
     return hipGetLastError();
 }
 
+// Streamlines that track_split_fast_kernel takes at most, a launch's all or
+// its last ones: two wavefronts per SIMD where one lane per streamline leaves
+// half the SIMDs idle. Mask domains, 145 x 174 x 145 SH45 Diffusion, one lane
+// per streamline against split: 28k seeds 5.4 and 4.2 ms, the last ones of
+// 100k 6.2 and 5.8, of 1M 22.5 and 21.9 (21.95 taken from 49152 on, 22.15
+// from 65536); mesh domains, whose one-lane step is longer: 40k seeds 7.3 and
+// 6.6 ms, the last ones of 500k 12.85 and 12.77 from 65536 on.
+template <int DOMAIN> constexpr uint32_t split_lanes() { return DOMAIN == DOMAIN_MESH ? 65536 : 32768; }
 // query: only report the lanes of the grid a launch would use.
 template <int MODEL, int ALGO, int DOMAIN, int LMAX, int S>
 hipError_t launch_fast(const FastLaunch &f, int grid_blocks, bool query, int64_t *lanes, hipStream_t stream)
 {
     constexpr int BLOCK = shape_block<MODEL, ALGO, LMAX, S>();
-    if (grid_blocks <= 0) {
+    const bool own_grid = grid_blocks <= 0;
+    if (own_grid) {
         const hipError_t e = fill_grid<track_fast_kernel<MODEL, ALGO, DOMAIN, LMAX, S>>(BLOCK, &grid_blocks);
         if (e != hipSuccess)
             return e;
@@ -1339,15 +1657,30 @@ hipError_t launch_fast(const FastLaunch &f, int grid_blocks, bool query, int64_t
     const uint64_t first_work = std::min<uint64_t>((uint64_t)f.track.n_seeds, (uint64_t)grid_blocks * BLOCK);
     const int generations = first_work / 2 >= f.min_repack ? FAST_GENERATIONS : 1;
     FastLaunch gen = f;
+    constexpr bool SPLIT = shaped<MODEL, ALGO, LMAX>();
+    const bool split_all = SPLIT && generations == 1 && own_grid && f.track.n_seeds <= split_lanes<DOMAIN>();
+    // What the last generation can be handed (see above).
+    const bool split_last = SPLIT && generations > 1 &&
+                            ((int64_t)grid_blocks * BLOCK >> (FAST_GENERATIONS - 1)) <= split_lanes<DOMAIN>();
     for (int g = 0; g < generations; g++) {
         gen.cont_in = g == 0 ? nullptr : f.cont[(g - 1) % 2];
         gen.cont_in_count = g == 0 ? nullptr : f.cont_count[(g - 1) % 2];
         gen.cont_out = f.cont[g % 2];
         gen.cont_out_count = f.cont_count[g % 2];
         gen.last = g == generations - 1;
-        zero_generation<<<1, 64, 0, stream>>>(f.claims, f.ended, gen.cont_out_count, g == 0 ? f.stats : nullptr);
+        const uint32_t split_limit = !SPLIT ? 0u : gen.last && split_last ? 0xffffffffu : split_lanes<DOMAIN>();
+        zero_generation<<<1, 64, 0, stream>>>(gen, g == 0, split_limit);
         const int blocks_g = std::max(1, grid_blocks >> g);
-        track_fast_kernel<MODEL, ALGO, DOMAIN, LMAX, S><<<blocks_g, BLOCK, 0, stream>>>(gen);
+        if (!split_all && !(gen.last && split_last))
+            track_fast_kernel<MODEL, ALGO, DOMAIN, LMAX, S><<<blocks_g, BLOCK, 0, stream>>>(gen);
+    }
+    if constexpr (SPLIT) {
+        if (split_all || generations > 1) {
+            gen.cont_in = split_all ? nullptr : f.cont[0];
+            track_split_fast_kernel<ALGO, DOMAIN>
+                <<<(unsigned)((std::min<uint64_t>(first_work, split_lanes<DOMAIN>()) + 63) / 64), 64 * FAST_SPLIT_WAVES, 0,
+                   stream>>>(gen);
+        }
     }
     return hipGetLastError();
 }

@@ -212,40 +212,63 @@ struct Cartesian {
     float value, gx, gy, gz;
 };
 
+// Order M > 0's parts of the sums: (value, gx, gy, gz) grow by
+// (v, M gx, M gy, gz). (pr, pi) is u^(M-1) and becomes u^M.
+struct CartesianTerm {
+    float v, gx, gy, gz;
+};
 template <int L, int M>
-__device__ __forceinline__ void sh_cartesian_terms(const float *q, float z, float w, float x, float y, float &pr,
-                                                   float &pi, Cartesian &g)
+__device__ __forceinline__ CartesianTerm sh_cartesian_term(const float *q, float z, float w, float x, float y,
+                                                           float &pr, float &pi)
 {
-    if constexpr (M <= L) {
-        using O = Order<L>;
-        float ur, ui;
-        if constexpr (M == 1) {
-            ur = x;
-            ui = y;
-        } else {
-            ur = pr * x - pi * y;
-            ui = pr * y + pi * x;
-        }
-        float a, ad, b, bd;
-        poly_m<M, O::poly_terms(M)>(q + O::a_offset(M), z, w, a, ad);
-        poly_m<M, O::poly_terms(M)>(q + O::b_offset(M), z, w, b, bd);
-        g.value += a * ur + b * ui;
-        g.gz += ad * ur + bd * ui;
-        if constexpr (M == 1) {
-            g.gx += a;
-            g.gy += b;
-        } else {
-            g.gx += (float)M * (a * pr + b * pi);
-            g.gy += (float)M * (b * pr - a * pi);
-        }
-        pr = ur;
-        pi = ui;
-        sh_cartesian_terms<L, M + 1>(q, z, w, x, y, pr, pi, g);
+    using O = Order<L>;
+    float ur, ui;
+    if constexpr (M == 1) {
+        ur = x;
+        ui = y;
+    } else {
+        ur = pr * x - pi * y;
+        ui = pr * y + pi * x;
+    }
+    float a, ad, b, bd;
+    poly_m<M, O::poly_terms(M)>(q + O::a_offset(M), z, w, a, ad);
+    poly_m<M, O::poly_terms(M)>(q + O::b_offset(M), z, w, b, bd);
+    CartesianTerm t;
+    t.v = a * ur + b * ui;
+    t.gz = ad * ur + bd * ui;
+    t.gx = M == 1 ? a : a * pr + b * pi;
+    t.gy = M == 1 ? b : b * pr - a * pi;
+    pr = ur;
+    pi = ui;
+    return t;
+}
+
+template <int M> __device__ __forceinline__ void add_term(const CartesianTerm &t, Cartesian &g)
+{
+    g.value += t.v;
+    g.gz += t.gz;
+    if constexpr (M == 1) {
+        g.gx += t.gx;
+        g.gy += t.gy;
+    } else {
+        g.gx += (float)M * t.gx;
+        g.gy += (float)M * t.gy;
     }
 }
 
-// Raw (pre-softplus) value and ambient gradient of P at the unit vector n.
-template <int L>
+template <int L, int M, int LAST>
+__device__ __forceinline__ void sh_cartesian_terms(const float *q, float z, float w, float x, float y, float &pr,
+                                                   float &pi, Cartesian &g)
+{
+    if constexpr (M <= LAST) {
+        add_term<M>(sh_cartesian_term<L, M>(q, z, w, x, y, pr, pi), g);
+        sh_cartesian_terms<L, M + 1, LAST>(q, z, w, x, y, pr, pi, g);
+    }
+}
+
+// Raw (pre-softplus) value and ambient gradient of P at the unit vector n,
+// the orders up to LAST.
+template <int L, int LAST = L>
 __device__ __forceinline__ Cartesian sh_cartesian(const float *q, V3 n)
 {
     using O = Order<L>;
@@ -255,7 +278,7 @@ __device__ __forceinline__ Cartesian sh_cartesian(const float *q, V3 n)
     g.gx = 0.0f;
     g.gy = 0.0f;
     float pr = 1.0f, pi = 0.0f;
-    sh_cartesian_terms<L, 1>(q, n.z, w, n.x, n.y, pr, pi, g);
+    sh_cartesian_terms<L, 1, LAST>(q, n.z, w, n.x, n.y, pr, pi, g);
     return g;
 }
 
@@ -366,11 +389,9 @@ __device__ __forceinline__ V3 update(const AlgoParams &a, const ModelOut &mv, co
 // model gradient taken in Cartesian form (sh_cartesian). The tangent frame
 // (e_theta, e_phi) is formed only for the Diffusion noise, which is drawn
 // in it.
-template <int ALGO, int L>
-__device__ __forceinline__ V3 sh_update(const AlgoParams &a, const float *q, V3 o, const Noise &nz)
+template <int ALGO>
+__device__ __forceinline__ V3 cartesian_turn(const AlgoParams &a, V3 n, const Cartesian &g, V3 o, const Noise &nz)
 {
-    const V3 n = unit_direction(o);
-    const Cartesian g = sh_cartesian<L>(q, n);
     float value, d;
     softplus(g.value, value, d);
     const float normal = g.gx * n.x + g.gy * n.y + g.gz * n.z;
@@ -398,6 +419,13 @@ __device__ __forceinline__ V3 sh_update(const AlgoParams &a, const float *q, V3 
         }
     }
     return exps2(o, v3(tx, ty, tz));
+}
+
+template <int ALGO, int L>
+__device__ __forceinline__ V3 sh_update(const AlgoParams &a, const float *q, V3 o, const Noise &nz)
+{
+    const V3 n = unit_direction(o);
+    return cartesian_turn<ALGO>(a, n, sh_cartesian<L>(q, n), o, nz);
 }
 
 // ------------------------------------------ Probabilistic, Deterministic ---

@@ -139,9 +139,10 @@ struct FastLaunch {
     unsigned long long *stats;  // [0] coefficient rows, [1] mask values read from memory (zeroed before generation 0)
     float4 *cont[2];            // saved streamlines, FAST_CONTINUATION_VEC4 float4 each; room for the grid's lanes
     uint32_t *cont_count[2];    // entries in cont[i]
+    uint32_t *tail;             // streamlines left to track_split_fast_kernel: how many, in which cont
     // Set per generation by launch_track_fast:
     const float4 *cont_in;      // the previous generation's saved streamlines (nullptr: claim seeds)
-    const uint32_t *cont_in_count;
+    uint32_t *cont_in_count;
     float4 *cont_out;
     uint32_t *cont_out_count;
     int32_t last;               // the last generation runs every streamline to its end
