@@ -422,6 +422,19 @@ __device__ __forceinline__ bool stop_test(const TrackLaunch &p, const Lane<G> &L
     return stop;
 }
 
+// track_fast_kernel's arguments (its only parameter) read afresh, for what few
+// iterations use: kept in scalar registers over the loop they push hot values
+// out of them, into vector lanes, an instruction and a wait per use (26 SGPRs
+// spilled on mask domains and 102 on mesh domains, SH Diffusion; now 0 and
+// 28). 145 x 174 x 145 DTI Transport, 500k seeds: 8.42 -> 8.27 ms; SH45
+// Transport between two surfaces, 500k seeds: 12.8 -> 12.3.
+__device__ __forceinline__ const FastLaunch &cold()
+{
+    auto *args = __builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(args));
+    return *(const FastLaunch *)args;
+}
+
 // nz: this step's Diffusion draws, made by the caller before anything that
 // waits on memory, so they cover the latency of the cell data
 // request_cells asked for.
@@ -433,10 +446,11 @@ __device__ __forceinline__ void advance(const TrackLaunch &p, bool shared_affine
     uint32_t hit = NO_HIT;
     const bool stop = stop_test<DOMAIN>(p, L, seg_decided, seg_found, seg_tri, hit);
     if (stop) {
-        store_held(p, L);
-        p.lengths[L.g] = L.n;
-        p.steps[L.g] = L.steps;
-        p.hits[L.g] = hit;
+        const TrackLaunch &c = cold().track;
+        store_held(c, L);
+        c.lengths[L.g] = L.n;
+        c.steps[L.g] = L.steps;
+        c.hits[L.g] = hit;
         L.g = -1;
         return;
     }
@@ -551,11 +565,12 @@ void track_fast_kernel(FastLaunch f)
         // Refill idle lanes, one atomic per wavefront.
         const uint64_t need = __ballot(L.g < 0);
         if (need != 0 && !drained) {
+            const FastLaunch &c = cold();
             const int leader = __ffsll((unsigned long long)need) - 1;
             const uint32_t count = (uint32_t)__popcll(need);
             uint32_t base = 0;
             if (lane_id == leader)
-                base = atomicAdd(f.claims, count);
+                base = atomicAdd(c.claims, count);
             base = __shfl(base, leader);
             if ((uint64_t)base + count >= (uint64_t)n_work)
                 drained = true;
@@ -564,17 +579,17 @@ void track_fast_kernel(FastLaunch f)
                 const uint64_t j = (uint64_t)base + rank;
                 if (j < (uint64_t)n_work) {
                     if (resume) {
-                        resume_lane<DOMAIN, G>(f.cont_in + FAST_CONTINUATION_VEC4 * j, L);
+                        resume_lane<DOMAIN, G>(c.cont_in + FAST_CONTINUATION_VEC4 * j, L);
                     } else {
                         const uint64_t g = j;
                         L.g = (int32_t)g;
-                        const float4 s0 = reinterpret_cast<const float4 *>(p.seeds)[2 * g];
-                        const float4 s1 = reinterpret_cast<const float4 *>(p.seeds)[2 * g + 1];
+                        const float4 s0 = reinterpret_cast<const float4 *>(c.track.seeds)[2 * g];
+                        const float4 s1 = reinterpret_cast<const float4 *>(c.track.seeds)[2 * g + 1];
                         L.point = v3(s0.x, s0.y, s0.z);
                         L.o = v3(s1.x, s1.y, s1.z);
                         L.previous = L.point;
                         if constexpr (ALGO == ALGO_DIFFUSION || ALGO == ALGO_PROBABILISTIC)
-                            L.rng = seed_stream(p, p.first_seed + L.g);
+                            L.rng = seed_stream(c.track, c.track.first_seed + L.g);
                         L.time = 0.0;
                         L.n = 0;
                         L.steps = 0;
@@ -615,18 +630,19 @@ void track_fast_kernel(FastLaunch f)
         if (live_seen < stop_below) {
             // Few streamlines left in flight: end the generation, handing
             // this wavefront's to the next one.
+            const FastLaunch &c = cold();
             const int leader = __ffsll((unsigned long long)live) - 1;
             const uint32_t count = (uint32_t)__popcll(live);
             uint32_t base = 0;
             if (lane_id == leader) {
-                base = atomicAdd(f.cont_out_count, count);
+                base = atomicAdd(c.cont_out_count, count);
                 atomicAdd(my_shard, ended_pending + count);
             }
             base = __shfl(base, leader);
             if (L.g >= 0) {
-                store_held(p, L);
+                store_held(c.track, L);
                 L.rng = rng_before;
-                save_lane<DOMAIN, G>(f.cont_out +
+                save_lane<DOMAIN, G>(c.cont_out +
                               FAST_CONTINUATION_VEC4 *
                                   ((uint64_t)base + (uint32_t)__popcll(live & ((1ull << lane_id) - 1ull))),
                           L);
@@ -670,8 +686,8 @@ void track_fast_kernel(FastLaunch f)
     // The wavefront's memory reads of rows and mask values, one atomic each
     // (the launch's totals price the bytes the cell cache had to fetch).
     if (lane_id == 0) {
-        atomicAdd(&f.stats[0], (unsigned long long)rows_read);
-        atomicAdd(&f.stats[1], (unsigned long long)masks_read);
+        atomicAdd(&cold().stats[0], (unsigned long long)rows_read);
+        atomicAdd(&cold().stats[1], (unsigned long long)masks_read);
     }
 }
 
