@@ -1618,7 +1618,10 @@ int tgk_connectome(tgk_runtime *rt, const tgk_domain *domain, const tgk_domain *
         int32_t sh_order = 8;
         if (int r = ensure_fast_field(rt, const_cast<tgk_field *>(field), algorithm, &sh_order))
             return r;
+        memset(&f, 0, sizeof f);
         f.connectome = c;
+        f.ended = rt->fast_counters.as<uint32_t>() + 32;
+        f.list_counts = rt->fast_counters.as<uint32_t>() + 16;
         f.coeffs = field->fast.ptr;
         f.coeff_stride = field->fast_stride;
         f.sh_order = sh_order;

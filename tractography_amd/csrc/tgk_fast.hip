@@ -1137,12 +1137,31 @@ __global__ __launch_bounds__(256) void track_group_kernel(FastLaunch f)
     }
 }
 
+// Work counted out of a generation (connectome_fast_kernel): the wavefront's
+// share of f.ended, and the tracks in flight as last summed.
+struct GenerationCount {
+    uint32_t pending = 0;     // ended here and not yet added to the shard
+    uint32_t value = 0;       // this lane's shard as last read
+    uint32_t iteration = 0;
+    bool reading = false;     // shards read, to be summed next iteration
+    uint32_t in_flight = 0xffffffffu;
+};
+
 // tracking.py:457-558 (kernel connectome) on the fast model: the plain
 // connectome kernel's loop (mask, field, update, finite and length test,
 // move) with the tracking kernel's persistent lanes, cell cache and
 // polynomial model. A finished track leaves the same record in its seed's
 // output slots as on the plain path (last segment, start barycentrics,
 // start triangle, length test) for the shared hits kernel.
+//
+// Run in generations, as track_fast_kernel: a launch ends with its longest
+// tracks, whose step takes four times as long while every wavefront of a SIMD
+// keeps a few lanes alive. A track cut short waits in its seed's record
+// (rows[2..7]: steps, noise state, orientation), its seed in a list in the
+// columns' slots, which only the hits kernel fills. 97 x 116 x 97 SH45
+// Diffusion, 300k seeds, 3000 steps at most: 8.96 ms in one launch, 1.15 +
+// 0.96 + 1.08 + 4.06 in four: the last one's lone wavefronts take 1.9 us per
+// step of the longest tracks.
 template <int MODEL, int ALGO, int LMAX>
 __global__ __launch_bounds__(fast_block<LMAX>()) void connectome_fast_kernel(FastConnectomeLaunch f)
 {
@@ -1152,9 +1171,20 @@ __global__ __launch_bounds__(fast_block<LMAX>()) void connectome_fast_kernel(Fas
     const uint32_t cstride = f.coeff_stride;
     const float step = c.algo.step_size;
     const int lane_id = __lane_id();
+    const bool resume = f.list_in != nullptr;
+    const uint64_t n_work = resume ? (uint64_t)*f.list_in_count : (uint64_t)c.n_seeds;
+    uint32_t stop_below = 0;
+    if (!f.last) {
+        const uint64_t half = min(n_work, (uint64_t)gridDim.x * blockDim.x) / 2;
+        stop_below = half >= f.min_repack ? (uint32_t)half : 0u;
+    }
+    uint32_t *const my_shard =
+        f.ended + ((blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) % FAST_END_SHARDS) * FAST_END_STRIDE;
+    GenerationCount count;
 
     int64_t g = -1;
     bool drained = false;
+    uint64_t live = 0;
     uint2 rng = make_uint2(0u, 0u);
     V3 point = v3(0.0f, 0.0f, 0.0f), o = point, previous = point;
     uint32_t tracked = 0, start_triangle = 0;
@@ -1164,40 +1194,110 @@ __global__ __launch_bounds__(fast_block<LMAX>()) void connectome_fast_kernel(Fas
     float q[MODEL == MODEL_SH ? Order<LMAX>::TERMS : 6];
 
     while (true) {
-        // Refill idle lanes from the queue, one atomic per wavefront.
         const uint64_t need = __ballot(g < 0);
+        count.pending += (uint32_t)__popcll(live & need);
+        // Refill idle lanes, one atomic per wavefront.
         if (need != 0 && !drained) {
             const int leader = __ffsll((unsigned long long)need) - 1;
-            const uint32_t count = (uint32_t)__popcll(need);
+            const uint32_t wanted = (uint32_t)__popcll(need);
             uint32_t base = 0;
             if (lane_id == leader)
-                base = atomicAdd(c.queue, count);
+                base = atomicAdd(c.queue, wanted);
             base = __shfl(base, leader);
-            if ((uint64_t)base + count >= (uint64_t)c.n_seeds)
+            if ((uint64_t)base + wanted >= n_work)
                 drained = true;
             if (g < 0) {
                 const uint64_t claimed = (uint64_t)base + (uint64_t)__popcll(need & ((1ull << lane_id) - 1ull));
-                if (claimed < (uint64_t)c.n_seeds) {
-                    g = (int64_t)claimed;
-                    rng = rng_init(c.rng_seed, (uint32_t)g);
-                    const BoundarySample sample = sample_boundary(c.boundary.vertices, c.boundary.triangles,
-                                                                  c.cumulative, c.n_triangles, rng);
-                    point = sample.point;
-                    o = sample.orientation;
-                    previous = point;
-                    tracked = 0;
-                    start_triangle = sample.triangle;
-                    b0 = sample.bary[0];
-                    b1 = sample.bary[1];
-                    b2 = sample.bary[2];
+                if (claimed < n_work) {
+                    if (resume) {
+                        g = (int64_t)f.list_in[claimed];
+                        const float *w = c.weights + 9 * g;
+                        const int32_t *r = c.rows + 9 * g;
+                        previous = v3(w[0], w[1], w[2]);
+                        point = v3(w[3], w[4], w[5]);
+                        b0 = w[6];
+                        b1 = w[7];
+                        b2 = w[8];
+                        start_triangle = (uint32_t)r[0];
+                        tracked = (uint32_t)r[2];
+                        rng = make_uint2((uint32_t)r[3], (uint32_t)r[4]);
+                        o = v3(__int_as_float(r[5]), __int_as_float(r[6]), __int_as_float(r[7]));
+                    } else {
+                        g = (int64_t)claimed;
+                        rng = rng_init(c.rng_seed, (uint32_t)g);
+                        const BoundarySample sample = sample_boundary(c.boundary.vertices, c.boundary.triangles,
+                                                                      c.cumulative, c.n_triangles, rng);
+                        point = sample.point;
+                        o = sample.orientation;
+                        previous = point;
+                        tracked = 0;
+                        start_triangle = sample.triangle;
+                        b0 = sample.bary[0];
+                        b1 = sample.bary[1];
+                        b2 = sample.bary[2];
+                    }
                     field_cell = -2;
                     cached_mask_cell = -2;
                     mask_inside = false;
                 }
             }
         }
-        if (__ballot(g >= 0) == 0)
+        live = __ballot(g >= 0);
+        if (live == 0)
             break;
+        if (count.reading) {
+            uint32_t left = count.value;
+#pragma unroll
+            for (int d = 32; d >= 1; d >>= 1)
+                left += __shfl_xor(left, d);
+            count.in_flight = (uint32_t)min(n_work - min((uint64_t)left, n_work), (uint64_t)0xffffffffu);
+            count.reading = false;
+        }
+        if (count.in_flight < stop_below) {
+            // Few tracks left in flight: hand this wavefront's over.
+            const int leader = __ffsll((unsigned long long)live) - 1;
+            uint32_t base = 0;
+            if (lane_id == leader) {
+                base = atomicAdd(f.list_out_count, (uint32_t)__popcll(live));
+                atomicAdd(my_shard, count.pending + (uint32_t)__popcll(live));
+            }
+            base = __shfl(base, leader);
+            if (g >= 0) {
+                f.list_out[(uint64_t)base + (uint32_t)__popcll(live & ((1ull << lane_id) - 1ull))] = (uint32_t)g;
+                float *w = c.weights + 9 * g;
+                int32_t *r = c.rows + 9 * g;
+                w[0] = previous.x;
+                w[1] = previous.y;
+                w[2] = previous.z;
+                w[3] = point.x;
+                w[4] = point.y;
+                w[5] = point.z;
+                w[6] = b0;
+                w[7] = b1;
+                w[8] = b2;
+                r[0] = (int32_t)start_triangle;
+                r[2] = (int32_t)tracked;
+                r[3] = (int32_t)rng.x;
+                r[4] = (int32_t)rng.y;
+                r[5] = __float_as_int(o.x);
+                r[6] = __float_as_int(o.y);
+                r[7] = __float_as_int(o.z);
+            }
+            count.pending = 0;
+            break;
+        }
+        // Once every claim is made, every eighth iteration: this wavefront's
+        // ended tracks to its shard, and all shards read.
+        if (stop_below != 0 && drained && (++count.iteration & 7u) == 0u) {
+            if (count.pending != 0 && lane_id == 0)
+                atomicAdd(my_shard, count.pending);
+            count.pending = 0;
+            count.value = lane_id < FAST_END_SHARDS
+                              ? __hip_atomic_load(f.ended + lane_id * FAST_END_STRIDE, __ATOMIC_RELAXED,
+                                                  __HIP_MEMORY_SCOPE_AGENT)
+                              : 0u;
+            count.reading = true;
+        }
         if (g < 0)
             continue;
         bool stop = tracked >= c.n_steps;
@@ -1246,6 +1346,8 @@ __global__ __launch_bounds__(fast_block<LMAX>()) void connectome_fast_kernel(Fas
         c.rows[9 * g + 1] = (float)tracked * step < c.min_length ? 0 : 1;
         g = -1;
     }
+    if (stop_below != 0 && count.pending != 0 && lane_id == 0)
+        atomicAdd(my_shard, count.pending);
 }
 
 // tracking.py:262-357 (kernel tod) on the fast model: the plain TOD
@@ -1393,6 +1495,16 @@ __global__ void zero_generation(FastLaunch f, bool first, uint32_t split_limit)
             }
         }
         *f.cont_out_count = 0u;
+    }
+}
+
+__global__ void zero_connectome_generation(uint32_t *queue, uint32_t *ended, uint32_t *list_count)
+{
+    if (threadIdx.x < FAST_END_SHARDS)
+        ended[threadIdx.x * FAST_END_STRIDE] = 0u;
+    if (threadIdx.x == 0) {
+        *queue = 0u;
+        *list_count = 0u;
     }
 }
 
@@ -1794,8 +1906,24 @@ template <int MODEL, int ALGO, int LMAX> hipError_t launch_connectome_fast_kerne
     }
     const int64_t fill = cache[device].load(std::memory_order_acquire);
     const int64_t needed = (f.connectome.n_seeds + fast_block<LMAX>() - 1) / fast_block<LMAX>();
-    zero_counter<<<1, 1, 0, stream>>>(f.connectome.queue);
-    connectome_fast_kernel<MODEL, ALGO, LMAX><<<(unsigned)std::min(fill, needed), fast_block<LMAX>(), 0, stream>>>(f);
+    const int64_t blocks = std::min(fill, needed);
+    // As track launches: DTI in one generation.
+    FastConnectomeLaunch gen = f;
+    gen.min_repack = MODEL == MODEL_DTI ? 0xffffffffu : FAST_MIN_REPACK;
+    const uint64_t first_work = std::min<uint64_t>((uint64_t)f.connectome.n_seeds, (uint64_t)blocks * fast_block<LMAX>());
+    const int generations = first_work / 2 >= gen.min_repack ? FAST_GENERATIONS : 1;
+    uint32_t *const lists[2] = {reinterpret_cast<uint32_t *>(f.connectome.cols),
+                                reinterpret_cast<uint32_t *>(f.connectome.cols) + f.connectome.n_seeds};
+    for (int g = 0; g < generations; g++) {
+        gen.list_in = g == 0 ? nullptr : lists[(g - 1) % 2];
+        gen.list_in_count = f.list_counts + (g + 1) % 2;
+        gen.list_out = lists[g % 2];
+        gen.list_out_count = f.list_counts + g % 2;
+        gen.last = g == generations - 1;
+        zero_connectome_generation<<<1, 64, 0, stream>>>(f.connectome.queue, f.ended, gen.list_out_count);
+        connectome_fast_kernel<MODEL, ALGO, LMAX>
+            <<<(unsigned)std::max<int64_t>(1, blocks >> g), fast_block<LMAX>(), 0, stream>>>(gen);
+    }
     e = hipGetLastError();
     if (e != hipSuccess)
         return e;

@@ -76,6 +76,15 @@ struct FastConnectomeLaunch {
     const void *coeffs;
     uint32_t coeff_stride;
     int32_t sh_order;
+    uint32_t *ended;          // ended-track shards (zeroed per generation)
+    uint32_t *list_counts;    // two words: entries of the lists of tracks cut short (in cols)
+    // Set per generation by launch_connectome_fast:
+    const uint32_t *list_in;  // the previous generation's (nullptr: claim seeds)
+    const uint32_t *list_in_count;
+    uint32_t *list_out;
+    uint32_t *list_out_count;
+    int32_t last;
+    uint32_t min_repack;
 };
 hipError_t launch_connectome_fast(const FastConnectomeLaunch &f, hipStream_t stream);
 
