@@ -11,6 +11,9 @@
 // * Transcendental-free SH model (tgk_fast_model.h), hardware exp2/log2/cos
 //   where the reference calls exp/log/cos, FP64 arc length; the four
 //   orientation updates (Transport, Diffusion, Probabilistic, Deterministic).
+// * Where a launch has fewer streamlines than lanes, or is left with few, lanes
+//   (Probabilistic, Deterministic: track_group_kernel) or wavefronts (SH
+//   Transport, Diffusion: track_split_fast_kernel) share a streamline's steps.
 // * Seed-major dense output rows, compacted into ragged points afterwards.
 // * The boundary connectome's tracking loop on the same machinery
 //   (connectome_fast_kernel); its hits pass is the plain path's.
@@ -477,11 +480,8 @@ __device__ __forceinline__ void advance(const TrackLaunch &p, bool shared_affine
 // waves). Held to three, the order-12 Transport and Diffusion kernels take
 // 168 VGPRs (170-185 otherwise, two waves) and the order-8 Probabilistic
 // one 151-155 (168-181, two waves); held to four, Probabilistic ran 3%
-// slower. The order-8 Deterministic kernel, held to four waves, made this
-// compiler emit an odd-aligned 64-bit register spill that gfx950 rejects,
-// so it keeps its 159-162 VGPRs (three waves). The DTI kernels (90-115
-// VGPRs, four or five waves) ran 4% slower held to seven waves and 19%
-// slower held to eight (spills).
+// slower. The DTI kernels (90-115 VGPRs, four or five waves) ran 4% slower
+// held to seven waves and 19% slower held to eight (spills).
 // A launch shape that puts more of the row in LDS allows fewer blocks per
 // CU (160 KiB of LDS each): shape 4 (44 coefficients) three waves per SIMD.
 template <int MODEL, int ALGO, int DOMAIN, int LMAX, int S = 0> constexpr int fast_min_waves()
