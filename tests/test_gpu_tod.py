@@ -304,6 +304,25 @@ def test_fast_tod_tracks_fp64(runtime, case):
     assert abs(steps_fast - steps_ref) <= max(1e-3 * steps_ref, 2.0 * abs(steps_plain - steps_ref))
 
 
+@pytest.mark.parametrize("n", [32_767, 32_768, 70_001])
+@pytest.mark.parametrize("case", ["sh45-transport", "sh45-diffusion"])
+def test_fast_tod_generations(runtime, case, n):
+    # Launches below, at and past the tracks that are cut short and resumed,
+    # held as the smaller ones above.
+    domain, field, algorithm, shape = _scene(case)
+    seed = algorithm.get_rng_seed()
+    args = (seed, n, 100, np.array(shape), np.eye(4, dtype=np.float32))
+    fast = _device_tod(runtime, domain, field, algorithm, *args, path=_native.PATH_FAST)
+    plain = _device_tod(runtime, domain, field, algorithm, *args)
+    ref, _, _ = oracle.tod(domain, field, algorithm, *args, precision=64)
+    mass = float(np.abs(ref).sum())
+    d_fast = float(np.abs(fast.astype(np.float64) - ref).sum()) / mass
+    d_plain = float(np.abs(plain.astype(np.float64) - ref).sum()) / mass
+    assert d_fast <= max(1e-3, 2.0 * d_plain)
+    steps_ref, steps_fast, steps_plain = (float(x[..., 0].astype(np.float64).sum()) for x in (ref, fast, plain))
+    assert abs(steps_fast - steps_ref) <= max(1e-3 * steps_ref, 2.0 * abs(steps_plain - steps_ref))
+
+
 def test_fast_tod_basis_of_single_steps(runtime):
     # One deposit per track: tracks of one step (n_steps 1), so each cell
     # holds the basis at its tracks' start orientations, the inward normals

@@ -102,6 +102,7 @@ struct tgk_runtime {
     DeviceBuffer workspace;
     DeviceBuffer queue;        // counters of the persistent kernels (layout: FAST_*_OFFSET)
     DeviceBuffer continuations[2];  // streamlines saved between generations of the fast kernel
+    DeviceBuffer tod_saved;         // tracks saved between launches of the fast TOD kernel (allocated once)
     DeviceBuffer plain_saved;       // streamlines saved between launches of the plain kernels (allocated once)
     DeviceBuffer fast_counters;     // claim counter and ended-streamline shards of the fast kernel
     TrackBuffers track_buffers;     // tgk_track's working buffers
@@ -1701,6 +1702,20 @@ int enqueue_tod(tgk_runtime *rt, tgk_field *field, const tgk_algorithm *algorith
             return r;
         f.coeffs = field->fast.ptr;
         f.coeff_stride = field->fast_stride;
+        f.ended = rt->fast_counters.as<uint32_t>() + 32;
+        f.saved_counts = rt->fast_counters.as<uint32_t>() + 16;
+        // Without room for saved tracks (while a graph is recorded, or when
+        // it cannot be had) the launch runs in one generation. Allocated
+        // once, so recorded launches keep it.
+        const size_t half = (size_t)tgk::FAST_TOD_SAVED * tgk::FAST_TOD_SAVED_VEC4;
+        if (!rt->tod_saved.ptr && !rt->capturing && t.n_seeds >= 2 * (int64_t)tgk::FAST_MIN_REPACK &&
+            rt->tod_saved.allocate(2 * half * sizeof(float4)) != hipSuccess)
+            (void)hipGetLastError();
+        if (rt->tod_saved.ptr) {
+            f.saved[0] = rt->tod_saved.as<float4>();
+            f.saved[1] = f.saved[0] + half;
+            f.saved_room = (uint64_t)tgk::FAST_TOD_SAVED;
+        }
     }
     TGK_HIP(tgk::launch_zero(d_coefficients, n_values, rt->stream), "TOD clear");
     if (path == TGK_PATH_FAST) {

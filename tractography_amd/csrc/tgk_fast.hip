@@ -1137,7 +1137,7 @@ __global__ __launch_bounds__(256) void track_group_kernel(FastLaunch f)
     }
 }
 
-// Work counted out of a generation (connectome_fast_kernel): the wavefront's
+// Work counted out of a generation (connectome and TOD kernels): the wavefront's
 // share of f.ended, and the tracks in flight as last summed.
 struct GenerationCount {
     uint32_t pending = 0;     // ended here and not yet added to the shard
@@ -1359,8 +1359,18 @@ __global__ __launch_bounds__(fast_block<LMAX>()) void connectome_fast_kernel(Fas
 // (acc = Y on entering a cell, acc += Y after); runs are flushed through the
 // LDS stages of flush_runs. The row stays in registers: the LDS holds the
 // stages.
+//
+// Run in generations, as connectome_fast_kernel, where there is room for the
+// tracks cut short (three float4 each); their runs are flushed first. 97 x 116
+// x 97 SH45 Diffusion, 300k seeds, 3000 steps at most: 12.8 ms in one launch,
+// 2.35 + 1.54 + 1.77 + 5.39 in four.
+// Order-8 SH Transport and Diffusion are held to three waves per SIMD (168
+// VGPRs; 172 and two otherwise).
 template <int MODEL, int ALGO, int LMAX>
-__global__ __launch_bounds__(256) void tod_fast_kernel(FastTodLaunch f)
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(
+    MODEL == MODEL_SH && LMAX == 8 && (ALGO == ALGO_TRANSPORT || ALGO == ALGO_DIFFUSION) ? 3 : 1)))
+void tod_fast_kernel(FastTodLaunch f)
 {
     __shared__ RunStage stages[4];
     RunStage &stage = stages[threadIdx.x >> 6];
@@ -1369,9 +1379,20 @@ __global__ __launch_bounds__(256) void tod_fast_kernel(FastTodLaunch f)
     const uint32_t cstride = f.coeff_stride;
     const float step = t.algo.step_size;
     const int lane_id = __lane_id();
+    const bool resume = f.saved_in != nullptr;
+    const uint64_t n_work = resume ? (uint64_t)*f.saved_in_count : (uint64_t)t.n_seeds;
+    uint32_t stop_below = 0;
+    if (!f.last) {
+        const uint64_t half = min(n_work, (uint64_t)gridDim.x * blockDim.x) / 2;
+        stop_below = half >= f.min_repack ? (uint32_t)half : 0u;
+    }
+    uint32_t *const my_shard =
+        f.ended + ((blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) % FAST_END_SHARDS) * FAST_END_STRIDE;
+    GenerationCount count;
 
     int64_t g = -1;
     bool drained = false;
+    uint64_t in_flight = 0;
     uint2 rng = make_uint2(0u, 0u);
     V3 point = v3(0.0f, 0.0f, 0.0f), o = point;
     uint32_t k = 0;
@@ -1385,27 +1406,37 @@ __global__ __launch_bounds__(256) void tod_fast_kernel(FastTodLaunch f)
         acc[i] = 0.0f;
 
     while (true) {
-        // Refill idle lanes from the queue, one atomic per wavefront.
         const uint64_t need = __ballot(g < 0);
+        count.pending += (uint32_t)__popcll(in_flight & need);
+        // Refill idle lanes, one atomic per wavefront.
         if (need != 0 && !drained) {
             const int leader = __ffsll((unsigned long long)need) - 1;
-            const uint32_t count = (uint32_t)__popcll(need);
+            const uint32_t wanted = (uint32_t)__popcll(need);
             uint32_t base = 0;
             if (lane_id == leader)
-                base = atomicAdd(t.queue, count);
+                base = atomicAdd(t.queue, wanted);
             base = __shfl(base, leader);
-            if ((uint64_t)base + count >= (uint64_t)t.n_seeds)
+            if ((uint64_t)base + wanted >= n_work)
                 drained = true;
             if (g < 0) {
                 const uint64_t claimed = (uint64_t)base + (uint64_t)__popcll(need & ((1ull << lane_id) - 1ull));
-                if (claimed < (uint64_t)t.n_seeds) {
+                if (claimed < n_work) {
                     g = (int64_t)claimed;
-                    rng = rng_init(t.rng_seed, (uint32_t)g);
-                    const BoundarySample sample =
-                        sample_boundary(t.vertices, t.triangles, t.cumulative, t.n_triangles, rng);
-                    point = sample.point;
-                    o = sample.orientation;
-                    k = 0;
+                    if (resume) {
+                        const float4 *slot = f.saved_in + 3 * claimed;
+                        const float4 a = slot[0], b = slot[1], c = slot[2];
+                        point = v3(a.x, a.y, a.z);
+                        o = v3(a.w, b.x, b.y);
+                        rng = make_uint2(__float_as_uint(b.z), __float_as_uint(b.w));
+                        k = __float_as_uint(c.x);
+                    } else {
+                        rng = rng_init(t.rng_seed, (uint32_t)g);
+                        const BoundarySample sample =
+                            sample_boundary(t.vertices, t.triangles, t.cumulative, t.n_triangles, rng);
+                        point = sample.point;
+                        o = sample.orientation;
+                        k = 0;
+                    }
                     previous = -1;
                     field_cell = -2;
                     cached_mask_cell = -2;
@@ -1413,8 +1444,47 @@ __global__ __launch_bounds__(256) void tod_fast_kernel(FastTodLaunch f)
                 }
             }
         }
-        if (__ballot(g >= 0) == 0)
+        in_flight = __ballot(g >= 0);
+        if (in_flight == 0)
             break;
+        if (count.reading) {
+            uint32_t left = count.value;
+#pragma unroll
+            for (int d = 32; d >= 1; d >>= 1)
+                left += __shfl_xor(left, d);
+            count.in_flight = (uint32_t)min(n_work - min((uint64_t)left, n_work), (uint64_t)0xffffffffu);
+            count.reading = false;
+        }
+        if (count.in_flight < stop_below) {
+            // Few tracks left in flight: hand this wavefront's over.
+            flush_runs(g >= 0 && previous >= 0, previous, acc, t.coefficients, stage);
+            const int leader = __ffsll((unsigned long long)in_flight) - 1;
+            uint32_t base = 0;
+            if (lane_id == leader) {
+                base = atomicAdd(f.saved_out_count, (uint32_t)__popcll(in_flight));
+                atomicAdd(my_shard, count.pending + (uint32_t)__popcll(in_flight));
+            }
+            base = __shfl(base, leader);
+            if (g >= 0) {
+                float4 *slot = f.saved_out +
+                               3 * ((uint64_t)base + (uint32_t)__popcll(in_flight & ((1ull << lane_id) - 1ull)));
+                slot[0] = make_float4(point.x, point.y, point.z, o.x);
+                slot[1] = make_float4(o.y, o.z, __uint_as_float(rng.x), __uint_as_float(rng.y));
+                slot[2] = make_float4(__uint_as_float(k), 0.0f, 0.0f, 0.0f);
+            }
+            count.pending = 0;
+            break;
+        }
+        if (stop_below != 0 && drained && (++count.iteration & 7u) == 0u) {
+            if (count.pending != 0 && lane_id == 0)
+                atomicAdd(my_shard, count.pending);
+            count.pending = 0;
+            count.value = lane_id < FAST_END_SHARDS
+                              ? __hip_atomic_load(f.ended + lane_id * FAST_END_STRIDE, __ATOMIC_RELAXED,
+                                                  __HIP_MEMORY_SCOPE_AGENT)
+                              : 0u;
+            count.reading = true;
+        }
         const bool live = g >= 0;
         bool stop = false;
         int64_t voxel = -1, cell = -1;
@@ -1464,14 +1534,13 @@ __global__ __launch_bounds__(256) void tod_fast_kernel(FastTodLaunch f)
         if (ended)
             g = -1;
     }
+    if (stop_below != 0 && count.pending != 0 && lane_id == 0)
+        atomicAdd(my_shard, count.pending);
 }
 
-__global__ void zero_counter(uint32_t *counter) { *counter = 0u; }
-
-// A generation's claim counter, ended-streamline shards and saved-streamline
-// count; before generation 0 also the launch's row and mask read totals.
-// One block of 64 threads.
-// Clears a generation's counters. Streamlines that the generation would run
+// Clears a generation's claim counter, ended-streamline shards and
+// saved-streamline count; before generation 0 also the launch's row and mask
+// read totals. One block of 64 threads. Streamlines that the generation would run
 // to their ends (fewer than twice min_repack, or the last generation's) go to
 // track_split_fast_kernel instead where it may take them (up to split_limit):
 // their buffer and number to f.tail, and none to this generation.
@@ -1498,7 +1567,7 @@ __global__ void zero_generation(FastLaunch f, bool first, uint32_t split_limit)
     }
 }
 
-__global__ void zero_connectome_generation(uint32_t *queue, uint32_t *ended, uint32_t *list_count)
+__global__ void zero_product_generation(uint32_t *queue, uint32_t *ended, uint32_t *list_count)
 {
     if (threadIdx.x < FAST_END_SHARDS)
         ended[threadIdx.x * FAST_END_STRIDE] = 0u;
@@ -1920,7 +1989,7 @@ template <int MODEL, int ALGO, int LMAX> hipError_t launch_connectome_fast_kerne
         gen.list_out = lists[g % 2];
         gen.list_out_count = f.list_counts + g % 2;
         gen.last = g == generations - 1;
-        zero_connectome_generation<<<1, 64, 0, stream>>>(f.connectome.queue, f.ended, gen.list_out_count);
+        zero_product_generation<<<1, 64, 0, stream>>>(f.connectome.queue, f.ended, gen.list_out_count);
         connectome_fast_kernel<MODEL, ALGO, LMAX>
             <<<(unsigned)std::max<int64_t>(1, blocks >> g), fast_block<LMAX>(), 0, stream>>>(gen);
     }
@@ -1976,8 +2045,22 @@ template <int MODEL, int ALGO, int LMAX> hipError_t launch_tod_fast_kernel(const
     }
     const int64_t fill = cache[device].load(std::memory_order_acquire);
     const int64_t needed = (f.tod.n_seeds + 255) / 256;
-    zero_counter<<<1, 1, 0, stream>>>(f.tod.queue);
-    tod_fast_kernel<MODEL, ALGO, LMAX><<<(unsigned)std::min(fill, needed), 256, 0, stream>>>(f);
+    const int64_t blocks = std::min(fill, needed);
+    // As connectome launches. A generation saves at most half its lanes.
+    FastTodLaunch gen = f;
+    gen.min_repack = MODEL == MODEL_DTI ? 0xffffffffu : FAST_MIN_REPACK;
+    const uint64_t first_work = std::min<uint64_t>((uint64_t)f.tod.n_seeds, (uint64_t)blocks * 256);
+    const int generations =
+        first_work / 2 >= gen.min_repack && first_work / 2 <= f.saved_room ? FAST_GENERATIONS : 1;
+    for (int g = 0; g < generations; g++) {
+        gen.saved_in = g == 0 ? nullptr : f.saved[(g - 1) % 2];
+        gen.saved_in_count = f.saved_counts + (g + 1) % 2;
+        gen.saved_out = f.saved[g % 2];
+        gen.saved_out_count = f.saved_counts + g % 2;
+        gen.last = g == generations - 1;
+        zero_product_generation<<<1, 64, 0, stream>>>(f.tod.queue, f.ended, gen.saved_out_count);
+        tod_fast_kernel<MODEL, ALGO, LMAX><<<(unsigned)std::max<int64_t>(1, blocks >> g), 256, 0, stream>>>(gen);
+    }
     return hipGetLastError();
 }
 

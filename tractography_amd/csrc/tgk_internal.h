@@ -112,8 +112,23 @@ struct FastTodLaunch {
     const void *coeffs;
     uint32_t coeff_stride;
     int32_t sh_order;
+    uint32_t *ended;          // ended-track shards (zeroed per generation)
+    uint32_t *saved_counts;   // two words: tracks cut short in saved[i]
+    float4 *saved[2];         // room for saved_room of them each, three float4 a track
+    uint64_t saved_room;      // 0: the launch runs in one generation
+    // Set per generation by launch_tod_fast:
+    const float4 *saved_in;   // the previous generation's (nullptr: claim seeds)
+    const uint32_t *saved_in_count;
+    float4 *saved_out;
+    uint32_t *saved_out_count;
+    int32_t last;
+    uint32_t min_repack;
 };
 hipError_t launch_tod_fast(const FastTodLaunch &f, hipStream_t stream);
+// Tracks a TOD launch on the fast path saves at most: half the lanes of the
+// largest grid (256 CUs, three blocks of 256 each: their LDS stages).
+constexpr int64_t FAST_TOD_SAVED = 98304;
+constexpr int64_t FAST_TOD_SAVED_VEC4 = 3;
 // Fill n floats with +0 (a kernel, so recorded graphs hold no memset node).
 hipError_t launch_zero(float *out, int64_t n, hipStream_t stream);
 // Rows of K packed floats (src) -> rows of `stride` floats (dst), pad = +0.
