@@ -392,10 +392,14 @@ __device__ __forceinline__ void request_cells(const TrackLaunch &p, bool shared_
 // order (tracking.py:121-133): the row or the step count is full, the point
 // left the mask or the last segment hit the boundary (`hit` then names the
 // triangle), the point left the field. seg_* is wave_segment_test's answer.
+// (Written to its reference in every branch, `hit` costs the mesh kernels
+// registers: order-12 Transport between two surfaces, 150k seeds, 14.6 against
+// 15.4 ms.)
 template <int DOMAIN, int G>
 __device__ __forceinline__ bool stop_test(const TrackLaunch &p, const Lane<G> &L, bool seg_decided, bool seg_found,
-                                          uint32_t seg_tri, uint32_t &hit)
+                                          uint32_t seg_tri, uint32_t &hit_triangle)
 {
+    uint32_t hit = NO_HIT;
     bool stop = !(L.n < p.n_points && L.steps < p.max_steps);
     if (!stop) {
         if constexpr (DOMAIN == DOMAIN_MASK) {
@@ -422,34 +426,41 @@ __device__ __forceinline__ bool stop_test(const TrackLaunch &p, const Lane<G> &L
     }
     if (!stop)
         stop = !L.field_ok;
+    hit_triangle = hit;
     return stop;
 }
 
-// track_fast_kernel's arguments (its only parameter) read afresh, for what few
+// The arguments f of a kernel (its only parameter) read afresh, for what few
 // iterations use: kept in scalar registers over the loop they push hot values
 // out of them, into vector lanes, an instruction and a wait per use (26 SGPRs
 // spilled on mask domains and 102 on mesh domains, SH Diffusion; now 0 and
-// 28). 145 x 174 x 145 DTI Transport, 500k seeds: 8.42 -> 8.27 ms; SH45
-// Transport between two surfaces, 500k seeds: 12.8 -> 12.3.
-__device__ __forceinline__ const FastLaunch &cold()
+// 31). 145 x 174 x 145 DTI Transport, 500k seeds: 8.73 -> 8.59 ms; SH45
+// Transport between two surfaces, 300k seeds: 10.2 -> 9.5. A Deterministic
+// step holds them: its wavefronts iterate over few lanes at a time, and waited
+// for the arguments at each track's end (DTI, 2906 seeds: 2.70 against 2.54 ms
+// per call).
+template <int ALGO, class Launch> __device__ __forceinline__ const Launch &cold(const Launch &f)
 {
+    if constexpr (ALGO == ALGO_DETERMINISTIC)
+        return f;
     auto *args = __builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(args));
-    return *(const FastLaunch *)args;
+    return *(const Launch *)args;
 }
 
 // nz: this step's Diffusion draws, made by the caller before anything that
 // waits on memory, so they cover the latency of the cell data
 // request_cells asked for.
 template <int MODEL, int ALGO, int DOMAIN, int LMAX, int G, int LDS_VEC, int BLOCK>
-__device__ __forceinline__ void advance(const TrackLaunch &p, bool shared_affine, const float *__restrict__ coeffs,
-                                        uint32_t cstride, Lane<G> &L, float *q, float4 *__restrict__ lds_rows,
-                                        const fast::Noise &nz, bool seg_decided, bool seg_found, uint32_t seg_tri)
+__device__ __forceinline__ void advance(const FastLaunch &f, const float *__restrict__ coeffs, uint32_t cstride,
+                                        Lane<G> &L, float *q, float4 *__restrict__ lds_rows, const fast::Noise &nz,
+                                        bool seg_decided, bool seg_found, uint32_t seg_tri)
 {
-    uint32_t hit = NO_HIT;
+    const TrackLaunch &p = f.track;
+    uint32_t hit;
     const bool stop = stop_test<DOMAIN>(p, L, seg_decided, seg_found, seg_tri, hit);
     if (stop) {
-        const TrackLaunch &c = cold().track;
+        const TrackLaunch &c = cold<ALGO>(f).track;
         store_held(c, L);
         c.lengths[L.g] = L.n;
         c.steps[L.g] = L.steps;
@@ -471,7 +482,7 @@ __device__ __forceinline__ void advance(const TrackLaunch &p, bool shared_affine
         const float t = (float)L.time;
         hold_point(L, v3(L.point.x - t * L.o.x, L.point.y - t * L.o.y, L.point.z - t * L.o.z));
     }
-    request_cells<MODEL, DOMAIN, LMAX, G, LDS_VEC, BLOCK>(p, shared_affine, coeffs, cstride, L, q, lds_rows);
+    request_cells<MODEL, DOMAIN, LMAX, G, LDS_VEC, BLOCK>(p, f.shared_affine != 0, coeffs, cstride, L, q, lds_rows);
 }
 
 // Waves per SIMD the compiler must fit: the order-8 SH Transport and
@@ -565,7 +576,7 @@ void track_fast_kernel(FastLaunch f)
         // Refill idle lanes, one atomic per wavefront.
         const uint64_t need = __ballot(L.g < 0);
         if (need != 0 && !drained) {
-            const FastLaunch &c = cold();
+            const FastLaunch &c = cold<ALGO>(f);
             const int leader = __ffsll((unsigned long long)need) - 1;
             const uint32_t count = (uint32_t)__popcll(need);
             uint32_t base = 0;
@@ -630,7 +641,7 @@ void track_fast_kernel(FastLaunch f)
         if (live_seen < stop_below) {
             // Few streamlines left in flight: end the generation, handing
             // this wavefront's to the next one.
-            const FastLaunch &c = cold();
+            const FastLaunch &c = cold<ALGO>(f);
             const int leader = __ffsll((unsigned long long)live) - 1;
             const uint32_t count = (uint32_t)__popcll(live);
             uint32_t base = 0;
@@ -656,8 +667,8 @@ void track_fast_kernel(FastLaunch f)
             wave_segment_test(p.mesh, L.previous, L.point, L.g >= 0 && L.steps > 0, L.near, seg_decided, seg_found,
                               seg_tri);
         if (L.g >= 0)
-            advance<MODEL, ALGO, DOMAIN, LMAX, G, LDS_VEC, BLOCK>(p, f.shared_affine != 0, coeffs, cstride, L, q,
-                                                                 lds_rows, nz, seg_decided, seg_found, seg_tri);
+            advance<MODEL, ALGO, DOMAIN, LMAX, G, LDS_VEC, BLOCK>(f, coeffs, cstride, L, q, lds_rows, nz,
+                                                                 seg_decided, seg_found, seg_tri);
         rows_read += (uint64_t)__popcll(__ballot(L.row_read));
         masks_read += (uint64_t)__popcll(__ballot(L.mask_read));
         L.row_read = false;
@@ -686,8 +697,8 @@ void track_fast_kernel(FastLaunch f)
     // The wavefront's memory reads of rows and mask values, one atomic each
     // (the launch's totals price the bytes the cell cache had to fetch).
     if (lane_id == 0) {
-        atomicAdd(&cold().stats[0], (unsigned long long)rows_read);
-        atomicAdd(&cold().stats[1], (unsigned long long)masks_read);
+        atomicAdd(&cold<ALGO>(f).stats[0], (unsigned long long)rows_read);
+        atomicAdd(&cold<ALGO>(f).stats[1], (unsigned long long)masks_read);
     }
 }
 
@@ -1080,7 +1091,7 @@ __global__ __launch_bounds__(256) void track_group_kernel(FastLaunch f)
             seg_tri = __shfl(seg_tri, 0, W);
         }
         if (starting) {
-            uint32_t hit = NO_HIT;
+            uint32_t hit;
             if (stop_test<DOMAIN>(p, L, seg_decided, seg_found, seg_tri, hit)) {
                 if (leader) {
                     p.lengths[L.g] = L.n;
