@@ -212,6 +212,32 @@ def test_fast_connectome_generations(runtime, name, n):
     assert (many[0] >= 0).mean() > 0.05
 
 
+@pytest.mark.parametrize("n", [131_071, 131_072, 140_001])
+@pytest.mark.parametrize("name", ["transport", "diffusion", "probabilistic"])
+def test_fast_connectome_long_tracks(runtime, name, n):
+    # Tracks of enough steps, and launches below, at and past enough of them,
+    # to be cut short and resumed: every seed's entries equal those of calls
+    # too small to be.
+    fod, wm, _ = fixtures.cross(shape=(14, 14, 3), n_coefficients=45)
+    domain = tg.domain.Image(wm)
+    field = tg.field.Image(fod)
+    model = tg.local.RealSymmetricSphericalHarmonics(45)
+    steps = 900
+    if name == "transport":
+        algorithm = tg.algorithm.Transport(model, step_size=0.009, gamma=1.0)
+    elif name == "diffusion":
+        algorithm = tg.algorithm.Diffusion(model, step_size=0.009, gamma=1.0, noise_variance=0.1, seed=21)
+    else:
+        algorithm = tg.algorithm.Probabilistic(model, step_size=0.05, seed=21)
+        steps = 300
+    seed = algorithm.get_rng_seed()
+    few = _device_connectome(runtime, domain, field, algorithm, seed, 20_000, steps, 0.5, path=_native.PATH_FAST)
+    many = _device_connectome(runtime, domain, field, algorithm, seed, n, steps, 0.5, path=_native.PATH_FAST)
+    for a, b in zip(few, many):
+        np.testing.assert_array_equal(a, b[: len(a)])
+    assert (many[0] >= 0).mean() > 0.05
+
+
 def test_fast_connectome_through_the_public_api():
     # test/test_tracking.py:227-255 on the fast path.
     fod_image, mask_image, segmentation = fixtures.cross()

@@ -323,6 +323,30 @@ def test_fast_tod_generations(runtime, case, n):
     assert abs(steps_fast - steps_ref) <= max(1e-3 * steps_ref, 2.0 * abs(steps_plain - steps_ref))
 
 
+@pytest.mark.parametrize("name", ["transport", "diffusion"])
+def test_fast_tod_long_tracks(runtime, name):
+    # One track more than a launch in one generation holds, and the launch is
+    # cut short and its tracks resumed. Its sums differ by that track's (at
+    # most n_steps deposits of 45 values whose squares add up to 45 / 4 pi)
+    # and by rounding: a cell of this grid takes some thousand additions, each
+    # of at most 2^-24 of its sum.
+    fod, wm, _ = fixtures.cross(shape=(14, 14, 3), n_coefficients=45)
+    domain = tg.domain.Image(wm)
+    field = tg.field.Image(fod)
+    model = tg.local.RealSymmetricSphericalHarmonics(45)
+    if name == "transport":
+        algorithm = tg.algorithm.Transport(model, step_size=0.009, gamma=1.0)
+    else:
+        algorithm = tg.algorithm.Diffusion(model, step_size=0.009, gamma=1.0, noise_variance=0.1, seed=21)
+    seed, n_steps = algorithm.get_rng_seed(), 900
+    args = (n_steps, np.array(wm.shape), np.eye(4, dtype=np.float32))
+    one, cut = (_device_tod(runtime, domain, field, algorithm, seed, n, *args, path=_native.PATH_FAST)
+                .astype(np.float64) for n in (131_071, 131_072))
+    bound = n_steps * 45 / np.sqrt(4 * np.pi) + 2e-4 * np.abs(one).sum()
+    assert one[..., 0].sum() / np.sqrt(0.25 / np.pi) > 10 * 131_072
+    assert np.abs(cut - one).sum() <= bound
+
+
 def test_fast_tod_basis_of_single_steps(runtime):
     # One deposit per track: tracks of one step (n_steps 1), so each cell
     # holds the basis at its tracks' start orientations, the inward normals

@@ -61,3 +61,12 @@ def test_order12_mesh_tracking_spills(kernels):
         k = _instance(kernels, "track_fast_kernel", 0, algorithm, 1, 12, 0)
         assert k["vgpr_count"] <= 168
         assert k["vgpr_spill_count"] <= 40
+
+
+@pytest.mark.parametrize("model, algorithm, order, vgprs", [
+    (1, 0, 8, 72), (1, 1, 8, 72), (1, 2, 8, 96), (1, 3, 8, 96), (0, 0, 12, 168), (0, 1, 12, 168)])
+def test_connectomes_of_one_launch(kernels, model, algorithm, order, vgprs):
+    # Launches that are never cut short run a kernel without the count of the
+    # tracks in flight, which took DTI kernels to 74, 107 and 102 VGPRs and
+    # the order-12 Diffusion one to 170: a wavefront per SIMD fewer.
+    assert _instance(kernels, "connectome_fast_kernel", model, algorithm, order)["vgpr_count"] <= vgprs

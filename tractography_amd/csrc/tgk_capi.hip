@@ -1708,7 +1708,7 @@ int enqueue_tod(tgk_runtime *rt, tgk_field *field, const tgk_algorithm *algorith
         // it cannot be had) the launch runs in one generation. Allocated
         // once, so recorded launches keep it.
         const size_t half = (size_t)tgk::FAST_TOD_SAVED * tgk::FAST_TOD_SAVED_VEC4;
-        if (!rt->tod_saved.ptr && !rt->capturing && t.n_seeds >= 2 * (int64_t)tgk::FAST_MIN_REPACK &&
+        if (!rt->tod_saved.ptr && !rt->capturing && t.n_seeds >= 4 * (int64_t)tgk::FAST_MIN_REPACK_PRODUCT &&
             rt->tod_saved.allocate(2 * half * sizeof(float4)) != hipSuccess)
             (void)hipGetLastError();
         if (rt->tod_saved.ptr) {

@@ -29,6 +29,7 @@
 #include <atomic>
 #include <cmath>
 #include <mutex>
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -1148,14 +1149,81 @@ __global__ __launch_bounds__(256) void track_group_kernel(FastLaunch f)
     }
 }
 
-// Work counted out of a generation (connectome and TOD kernels): the wavefront's
-// share of f.ended, and the tracks in flight as last summed.
-struct GenerationCount {
+// A generation of the connectome or TOD kernel, as one wavefront sees it: the
+// tracks in flight over the launch, from shards that every wavefront adds its
+// ended tracks to, and the cut once fewer than stop_below are left.
+struct Generation {
+    uint64_t n_work;
+    uint32_t stop_below;      // 0: run to the end
     uint32_t pending = 0;     // ended here and not yet added to the shard
     uint32_t value = 0;       // this lane's shard as last read
     uint32_t iteration = 0;
     bool reading = false;     // shards read, to be summed next iteration
     uint32_t in_flight = 0xffffffffu;
+
+    __device__ __forceinline__ Generation(uint64_t work, bool last, uint32_t min_repack)
+    {
+        n_work = work;
+        const uint64_t half = min(n_work, (uint64_t)gridDim.x * blockDim.x) / 2;
+        stop_below = !last && half >= min_repack ? (uint32_t)half : 0u;
+    }
+    static __device__ __forceinline__ uint32_t *shard(uint32_t *ended)
+    {
+        return ended + ((blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) % FAST_END_SHARDS) * FAST_END_STRIDE;
+    }
+    // Whether the wavefront hands its tracks over now.
+    __device__ __forceinline__ bool over()
+    {
+        if (reading) {
+            uint32_t left = value;
+#pragma unroll
+            for (int d = 32; d >= 1; d >>= 1)
+                left += __shfl_xor(left, d);
+            in_flight = (uint32_t)min(n_work - min((uint64_t)left, n_work), (uint64_t)0xffffffffu);
+            reading = false;
+        }
+        return in_flight < stop_below;
+    }
+    // The `live` lanes' tracks leave: the slot of this lane's among `saved`.
+    __device__ __forceinline__ uint64_t hand_over(uint64_t live, uint32_t *ended, uint32_t *saved)
+    {
+        const int leader = __ffsll((unsigned long long)live) - 1;
+        uint32_t base = 0;
+        if (__lane_id() == leader) {
+            base = atomicAdd(saved, (uint32_t)__popcll(live));
+            atomicAdd(shard(ended), pending + (uint32_t)__popcll(live));
+        }
+        pending = 0;
+        return (uint64_t)__shfl(base, leader) + (uint32_t)__popcll(live & ((1ull << __lane_id()) - 1ull));
+    }
+    // Once every claim is made, every 32nd iteration: this wavefront's ended
+    // tracks to its shard, and all shards read. (Every eighth, 300k SH15
+    // Transport tracks of at most 500 steps took 4.3 ms, 3.9 so.)
+    template <int ALGO, class Launch> __device__ __forceinline__ void count(const Launch &f, bool drained)
+    {
+        if (stop_below != 0 && drained && (++iteration & 31u) == 0u) {
+            uint32_t *const ended = cold<ALGO>(f).ended;
+            flush(ended);
+            value = __lane_id() < FAST_END_SHARDS
+                        ? __hip_atomic_load(ended + __lane_id() * FAST_END_STRIDE, __ATOMIC_RELAXED,
+                                            __HIP_MEMORY_SCOPE_AGENT)
+                        : 0u;
+            reading = true;
+        }
+    }
+    __device__ __forceinline__ void flush(uint32_t *ended)
+    {
+        if (stop_below != 0 && pending != 0 && __lane_id() == 0)
+            atomicAdd(shard(ended), pending);
+        pending = 0;
+    }
+};
+
+// The one generation of a launch that is never cut short.
+struct WholeLaunch {
+    uint64_t n_work;
+
+    __device__ __forceinline__ WholeLaunch(uint64_t work, bool, uint32_t) { n_work = work; }
 };
 
 // tracking.py:457-558 (kernel connectome) on the fast model: the plain
@@ -1165,15 +1233,17 @@ struct GenerationCount {
 // output slots as on the plain path (last segment, start barycentrics,
 // start triangle, length test) for the shared hits kernel.
 //
-// Run in generations, as track_fast_kernel: a launch ends with its longest
-// tracks, whose step takes four times as long while every wavefront of a SIMD
-// keeps a few lanes alive. A track cut short waits in its seed's record
-// (rows[2..7]: steps, noise state, orientation), its seed in a list in the
-// columns' slots, which only the hits kernel fills. 97 x 116 x 97 SH45
-// Diffusion, 300k seeds, 3000 steps at most: 8.96 ms in one launch, 1.15 +
-// 0.96 + 1.08 + 4.06 in four: the last one's lone wavefronts take 1.9 us per
-// step of the longest tracks.
-template <int MODEL, int ALGO, int LMAX>
+// Run in generations where it pays (in_generations), as track_fast_kernel: a
+// launch ends with its longest tracks, whose step takes four times as long
+// while every wavefront of a SIMD keeps a few lanes alive. A track cut short
+// waits in its seed's record (rows[2..7]: steps, noise state, orientation), its
+// seed in a list in the columns' slots, which only the hits kernel fills.
+// 97 x 116 x 97 SH45 Diffusion, 300k seeds, 3000 steps at most: 10.9 ms per call
+// in one launch, 8.7 so, of which the last generation's lone wavefronts, at
+// 1.9 us per step of the longest tracks, take some 4. The count costs 11 to 13
+// VGPRs and as many scalar registers, so launches in one generation run a
+// kernel without it (200k DTI Transport tracks: 6.2 against 5.5 ms).
+template <int MODEL, int ALGO, int LMAX, bool GENERATIONS>
 __global__ __launch_bounds__(fast_block<LMAX>()) void connectome_fast_kernel(FastConnectomeLaunch f)
 {
     __shared__ float4 lds_rows[rows_in_lds<MODEL, LMAX>() ? lds_vectors<MODEL, LMAX>() * fast_block<LMAX>() : 1];
@@ -1182,16 +1252,9 @@ __global__ __launch_bounds__(fast_block<LMAX>()) void connectome_fast_kernel(Fas
     const uint32_t cstride = f.coeff_stride;
     const float step = c.algo.step_size;
     const int lane_id = __lane_id();
-    const bool resume = f.list_in != nullptr;
-    const uint64_t n_work = resume ? (uint64_t)*f.list_in_count : (uint64_t)c.n_seeds;
-    uint32_t stop_below = 0;
-    if (!f.last) {
-        const uint64_t half = min(n_work, (uint64_t)gridDim.x * blockDim.x) / 2;
-        stop_below = half >= f.min_repack ? (uint32_t)half : 0u;
-    }
-    uint32_t *const my_shard =
-        f.ended + ((blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) % FAST_END_SHARDS) * FAST_END_STRIDE;
-    GenerationCount count;
+    const bool resume = GENERATIONS && f.list_in != nullptr;
+    std::conditional_t<GENERATIONS, Generation, WholeLaunch> work(
+        resume ? (uint64_t)*f.list_in_count : (uint64_t)c.n_seeds, f.last, f.min_repack);
 
     int64_t g = -1;
     bool drained = false;
@@ -1206,22 +1269,25 @@ __global__ __launch_bounds__(fast_block<LMAX>()) void connectome_fast_kernel(Fas
 
     while (true) {
         const uint64_t need = __ballot(g < 0);
-        count.pending += (uint32_t)__popcll(live & need);
+        if constexpr (GENERATIONS)
+            work.pending += (uint32_t)__popcll(live & need);
         // Refill idle lanes, one atomic per wavefront.
         if (need != 0 && !drained) {
+            const FastConnectomeLaunch &rare = cold<ALGO>(f);
+            const ConnectomeLaunch &c = rare.connectome;
             const int leader = __ffsll((unsigned long long)need) - 1;
             const uint32_t wanted = (uint32_t)__popcll(need);
             uint32_t base = 0;
             if (lane_id == leader)
                 base = atomicAdd(c.queue, wanted);
             base = __shfl(base, leader);
-            if ((uint64_t)base + wanted >= n_work)
+            if ((uint64_t)base + wanted >= work.n_work)
                 drained = true;
             if (g < 0) {
                 const uint64_t claimed = (uint64_t)base + (uint64_t)__popcll(need & ((1ull << lane_id) - 1ull));
-                if (claimed < n_work) {
+                if (claimed < work.n_work) {
                     if (resume) {
-                        g = (int64_t)f.list_in[claimed];
+                        g = (int64_t)rare.list_in[claimed];
                         const float *w = c.weights + 9 * g;
                         const int32_t *r = c.rows + 9 * g;
                         previous = v3(w[0], w[1], w[2]);
@@ -1256,58 +1322,35 @@ __global__ __launch_bounds__(fast_block<LMAX>()) void connectome_fast_kernel(Fas
         live = __ballot(g >= 0);
         if (live == 0)
             break;
-        if (count.reading) {
-            uint32_t left = count.value;
-#pragma unroll
-            for (int d = 32; d >= 1; d >>= 1)
-                left += __shfl_xor(left, d);
-            count.in_flight = (uint32_t)min(n_work - min((uint64_t)left, n_work), (uint64_t)0xffffffffu);
-            count.reading = false;
-        }
-        if (count.in_flight < stop_below) {
-            // Few tracks left in flight: hand this wavefront's over.
-            const int leader = __ffsll((unsigned long long)live) - 1;
-            uint32_t base = 0;
-            if (lane_id == leader) {
-                base = atomicAdd(f.list_out_count, (uint32_t)__popcll(live));
-                atomicAdd(my_shard, count.pending + (uint32_t)__popcll(live));
+        if constexpr (GENERATIONS) {
+            if (work.over()) {
+                // Few tracks left in flight: hand this wavefront's over.
+                const FastConnectomeLaunch &rare = cold<ALGO>(f);
+                const uint64_t slot = work.hand_over(live, rare.ended, rare.list_out_count);
+                if (g >= 0) {
+                    rare.list_out[slot] = (uint32_t)g;
+                    float *w = rare.connectome.weights + 9 * g;
+                    int32_t *r = rare.connectome.rows + 9 * g;
+                    w[0] = previous.x;
+                    w[1] = previous.y;
+                    w[2] = previous.z;
+                    w[3] = point.x;
+                    w[4] = point.y;
+                    w[5] = point.z;
+                    w[6] = b0;
+                    w[7] = b1;
+                    w[8] = b2;
+                    r[0] = (int32_t)start_triangle;
+                    r[2] = (int32_t)tracked;
+                    r[3] = (int32_t)rng.x;
+                    r[4] = (int32_t)rng.y;
+                    r[5] = __float_as_int(o.x);
+                    r[6] = __float_as_int(o.y);
+                    r[7] = __float_as_int(o.z);
+                }
+                break;
             }
-            base = __shfl(base, leader);
-            if (g >= 0) {
-                f.list_out[(uint64_t)base + (uint32_t)__popcll(live & ((1ull << lane_id) - 1ull))] = (uint32_t)g;
-                float *w = c.weights + 9 * g;
-                int32_t *r = c.rows + 9 * g;
-                w[0] = previous.x;
-                w[1] = previous.y;
-                w[2] = previous.z;
-                w[3] = point.x;
-                w[4] = point.y;
-                w[5] = point.z;
-                w[6] = b0;
-                w[7] = b1;
-                w[8] = b2;
-                r[0] = (int32_t)start_triangle;
-                r[2] = (int32_t)tracked;
-                r[3] = (int32_t)rng.x;
-                r[4] = (int32_t)rng.y;
-                r[5] = __float_as_int(o.x);
-                r[6] = __float_as_int(o.y);
-                r[7] = __float_as_int(o.z);
-            }
-            count.pending = 0;
-            break;
-        }
-        // Once every claim is made, every eighth iteration: this wavefront's
-        // ended tracks to its shard, and all shards read.
-        if (stop_below != 0 && drained && (++count.iteration & 7u) == 0u) {
-            if (count.pending != 0 && lane_id == 0)
-                atomicAdd(my_shard, count.pending);
-            count.pending = 0;
-            count.value = lane_id < FAST_END_SHARDS
-                              ? __hip_atomic_load(f.ended + lane_id * FAST_END_STRIDE, __ATOMIC_RELAXED,
-                                                  __HIP_MEMORY_SCOPE_AGENT)
-                              : 0u;
-            count.reading = true;
+            work.template count<ALGO>(f, drained);
         }
         if (g < 0)
             continue;
@@ -1343,6 +1386,7 @@ __global__ __launch_bounds__(fast_block<LMAX>()) void connectome_fast_kernel(Fas
             tracked++;
             continue;
         }
+        const ConnectomeLaunch &c = cold<ALGO>(f).connectome;
         float *record = c.weights + 9 * g;
         record[0] = previous.x;
         record[1] = previous.y;
@@ -1357,8 +1401,8 @@ __global__ __launch_bounds__(fast_block<LMAX>()) void connectome_fast_kernel(Fas
         c.rows[9 * g + 1] = (float)tracked * step < c.min_length ? 0 : 1;
         g = -1;
     }
-    if (stop_below != 0 && count.pending != 0 && lane_id == 0)
-        atomicAdd(my_shard, count.pending);
+    if constexpr (GENERATIONS)
+        work.flush(cold<ALGO>(f).ended);
 }
 
 // tracking.py:262-357 (kernel tod) on the fast model: the plain TOD
@@ -1371,16 +1415,15 @@ __global__ __launch_bounds__(fast_block<LMAX>()) void connectome_fast_kernel(Fas
 // LDS stages of flush_runs. The row stays in registers: the LDS holds the
 // stages.
 //
-// Run in generations, as connectome_fast_kernel, where there is room for the
-// tracks cut short (three float4 each); their runs are flushed first. 97 x 116
-// x 97 SH45 Diffusion, 300k seeds, 3000 steps at most: 12.8 ms in one launch,
-// 2.35 + 1.54 + 1.77 + 5.39 in four.
-// Order-8 SH Transport and Diffusion are held to three waves per SIMD (168
-// VGPRs; 172 and two otherwise).
-template <int MODEL, int ALGO, int LMAX>
+// Run in generations as connectome_fast_kernel, where there is also room for
+// the tracks cut short (three float4 each); their runs are flushed first. 97 x
+// 116 x 97 SH45 Diffusion, 300k seeds, 3000 steps at most: 16.8 ms per call in
+// one launch, 15.3 so. Order-8 SH Transport and Diffusion are then held to
+// three waves per SIMD (168 VGPRs; 172 and two otherwise).
+template <int MODEL, int ALGO, int LMAX, bool GENERATIONS>
 __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(
-    MODEL == MODEL_SH && LMAX == 8 && (ALGO == ALGO_TRANSPORT || ALGO == ALGO_DIFFUSION) ? 3 : 1)))
+    GENERATIONS && LMAX == 8 && (ALGO == ALGO_TRANSPORT || ALGO == ALGO_DIFFUSION) ? 3 : 1)))
 void tod_fast_kernel(FastTodLaunch f)
 {
     __shared__ RunStage stages[4];
@@ -1390,16 +1433,9 @@ void tod_fast_kernel(FastTodLaunch f)
     const uint32_t cstride = f.coeff_stride;
     const float step = t.algo.step_size;
     const int lane_id = __lane_id();
-    const bool resume = f.saved_in != nullptr;
-    const uint64_t n_work = resume ? (uint64_t)*f.saved_in_count : (uint64_t)t.n_seeds;
-    uint32_t stop_below = 0;
-    if (!f.last) {
-        const uint64_t half = min(n_work, (uint64_t)gridDim.x * blockDim.x) / 2;
-        stop_below = half >= f.min_repack ? (uint32_t)half : 0u;
-    }
-    uint32_t *const my_shard =
-        f.ended + ((blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) % FAST_END_SHARDS) * FAST_END_STRIDE;
-    GenerationCount count;
+    const bool resume = GENERATIONS && f.saved_in != nullptr;
+    std::conditional_t<GENERATIONS, Generation, WholeLaunch> work(
+        resume ? (uint64_t)*f.saved_in_count : (uint64_t)t.n_seeds, f.last, f.min_repack);
 
     int64_t g = -1;
     bool drained = false;
@@ -1418,23 +1454,26 @@ void tod_fast_kernel(FastTodLaunch f)
 
     while (true) {
         const uint64_t need = __ballot(g < 0);
-        count.pending += (uint32_t)__popcll(in_flight & need);
+        if constexpr (GENERATIONS)
+            work.pending += (uint32_t)__popcll(in_flight & need);
         // Refill idle lanes, one atomic per wavefront.
         if (need != 0 && !drained) {
+            const FastTodLaunch &rare = cold<ALGO>(f);
+            const TodLaunch &t = rare.tod;
             const int leader = __ffsll((unsigned long long)need) - 1;
             const uint32_t wanted = (uint32_t)__popcll(need);
             uint32_t base = 0;
             if (lane_id == leader)
                 base = atomicAdd(t.queue, wanted);
             base = __shfl(base, leader);
-            if ((uint64_t)base + wanted >= n_work)
+            if ((uint64_t)base + wanted >= work.n_work)
                 drained = true;
             if (g < 0) {
                 const uint64_t claimed = (uint64_t)base + (uint64_t)__popcll(need & ((1ull << lane_id) - 1ull));
-                if (claimed < n_work) {
+                if (claimed < work.n_work) {
                     g = (int64_t)claimed;
                     if (resume) {
-                        const float4 *slot = f.saved_in + 3 * claimed;
+                        const float4 *slot = rare.saved_in + 3 * claimed;
                         const float4 a = slot[0], b = slot[1], c = slot[2];
                         point = v3(a.x, a.y, a.z);
                         o = v3(a.w, b.x, b.y);
@@ -1458,43 +1497,21 @@ void tod_fast_kernel(FastTodLaunch f)
         in_flight = __ballot(g >= 0);
         if (in_flight == 0)
             break;
-        if (count.reading) {
-            uint32_t left = count.value;
-#pragma unroll
-            for (int d = 32; d >= 1; d >>= 1)
-                left += __shfl_xor(left, d);
-            count.in_flight = (uint32_t)min(n_work - min((uint64_t)left, n_work), (uint64_t)0xffffffffu);
-            count.reading = false;
-        }
-        if (count.in_flight < stop_below) {
-            // Few tracks left in flight: hand this wavefront's over.
-            flush_runs(g >= 0 && previous >= 0, previous, acc, t.coefficients, stage);
-            const int leader = __ffsll((unsigned long long)in_flight) - 1;
-            uint32_t base = 0;
-            if (lane_id == leader) {
-                base = atomicAdd(f.saved_out_count, (uint32_t)__popcll(in_flight));
-                atomicAdd(my_shard, count.pending + (uint32_t)__popcll(in_flight));
+        if constexpr (GENERATIONS) {
+            if (work.over()) {
+                // Few tracks left in flight: hand this wavefront's over.
+                flush_runs(g >= 0 && previous >= 0, previous, acc, t.coefficients, stage);
+                const FastTodLaunch &rare = cold<ALGO>(f);
+                const uint64_t slot = work.hand_over(in_flight, rare.ended, rare.saved_out_count);
+                if (g >= 0) {
+                    float4 *saved = rare.saved_out + 3 * slot;
+                    saved[0] = make_float4(point.x, point.y, point.z, o.x);
+                    saved[1] = make_float4(o.y, o.z, __uint_as_float(rng.x), __uint_as_float(rng.y));
+                    saved[2] = make_float4(__uint_as_float(k), 0.0f, 0.0f, 0.0f);
+                }
+                break;
             }
-            base = __shfl(base, leader);
-            if (g >= 0) {
-                float4 *slot = f.saved_out +
-                               3 * ((uint64_t)base + (uint32_t)__popcll(in_flight & ((1ull << lane_id) - 1ull)));
-                slot[0] = make_float4(point.x, point.y, point.z, o.x);
-                slot[1] = make_float4(o.y, o.z, __uint_as_float(rng.x), __uint_as_float(rng.y));
-                slot[2] = make_float4(__uint_as_float(k), 0.0f, 0.0f, 0.0f);
-            }
-            count.pending = 0;
-            break;
-        }
-        if (stop_below != 0 && drained && (++count.iteration & 7u) == 0u) {
-            if (count.pending != 0 && lane_id == 0)
-                atomicAdd(my_shard, count.pending);
-            count.pending = 0;
-            count.value = lane_id < FAST_END_SHARDS
-                              ? __hip_atomic_load(f.ended + lane_id * FAST_END_STRIDE, __ATOMIC_RELAXED,
-                                                  __HIP_MEMORY_SCOPE_AGENT)
-                              : 0u;
-            count.reading = true;
+            work.template count<ALGO>(f, drained);
         }
         const bool live = g >= 0;
         bool stop = false;
@@ -1545,8 +1562,8 @@ void tod_fast_kernel(FastTodLaunch f)
         if (ended)
             g = -1;
     }
-    if (stop_below != 0 && count.pending != 0 && lane_id == 0)
-        atomicAdd(my_shard, count.pending);
+    if constexpr (GENERATIONS)
+        work.flush(cold<ALGO>(f).ended);
 }
 
 // Clears a generation's claim counter, ended-streamline shards and
@@ -1959,53 +1976,79 @@ hipError_t dispatch_fast(const FastLaunch &f, int grid, bool query, int64_t *blo
     return launch_fast_algo<MODEL_SH>(f, grid, query, blocks, stream);
 }
 
-// Connectome launches: the persistent grid of the kernel's occupancy
-// (cached per device), at most one lane per seed, then the hits pass.
-template <int MODEL, int ALGO, int LMAX> hipError_t launch_connectome_fast_kernel(const FastConnectomeLaunch &f,
-                                                                                  hipStream_t stream)
+// Whether a connectome or TOD launch of the SH model, `lanes` tracks at a
+// time, runs in generations: where half its lanes, and half of those, still
+// fill wavefronts for half the SIMDs, and where tracks are long. Packing lanes
+// costs 0.2 to 0.4 ms a launch. Tracks that soon leave a small grid, or that
+// most lanes take to a low limit, leave less than that to gain: 135k to 300k
+// SH28 Transport and SH45 Diffusion tracks ran at 0.88 to 1.05 of the speed of
+// one generation where at most 200 to 800 steps cross the mask's grid or are
+// taken, and at 0.99 to 1.24 from 850 on; 40k to 100k tracks at 0.83 to 1.00.
+// In connectomes a step of many Probabilistic candidates takes so long that a
+// limit of 300 steps suffices (135k and 200k tracks: 0.91 to 0.97 with 160,
+// 1.00 to 1.63 with 320 to 1200). Deterministic launches always run in one:
+// their lanes iterate one by one, and packed they wait for more of the others
+// (135k and 200k tracks: 0.75 to 1.34, with no order in it).
+template <int MODEL, int ALGO> constexpr bool cut_short()
 {
-    static std::atomic<int> cache[64] = {};
-    int device = 0;
-    hipError_t e = hipGetDevice(&device);
-    if (e != hipSuccess)
-        return e;
-    if (device < 0 || device >= 64)
-        return hipErrorInvalidDevice;
-    if (cache[device].load(std::memory_order_acquire) == 0) {
-        int per_cu = 0;
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per_cu, reinterpret_cast<const void *>(connectome_fast_kernel<MODEL, ALGO, LMAX>), fast_block<LMAX>(),
-            0);
-        if (e != hipSuccess)
-            return e;
-        int cus = 0;
-        e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device);
-        if (e != hipSuccess)
-            return e;
-        cache[device].store((cus > 0 ? cus : 1) * (per_cu > 0 ? per_cu : 1), std::memory_order_release);
-    }
-    const int64_t fill = cache[device].load(std::memory_order_acquire);
-    const int64_t needed = (f.connectome.n_seeds + fast_block<LMAX>() - 1) / fast_block<LMAX>();
-    const int64_t blocks = std::min(fill, needed);
-    // As track launches: DTI in one generation.
+    return MODEL == MODEL_SH && ALGO != ALGO_DETERMINISTIC;
+}
+bool in_generations(const MaskView &mask, const AlgoParams &a, uint32_t n_steps, int64_t lanes, bool many_candidates)
+{
+    constexpr double LONG_TRACK = 840.0;
+    if (lanes < 4 * (int64_t)FAST_MIN_REPACK_PRODUCT)
+        return false;
+    if (many_candidates && n_steps >= 300)
+        return true;
+    const float *m = mask.inv;
+    const double det = (double)m[0] * ((double)m[5] * m[10] - (double)m[6] * m[9]) -
+                       (double)m[1] * ((double)m[4] * m[10] - (double)m[6] * m[8]) +
+                       (double)m[2] * ((double)m[4] * m[9] - (double)m[5] * m[8]);
+    const double edge = std::cbrt((double)mask.dims[0] * mask.dims[1] * mask.dims[2] / std::fabs(det));
+    return std::min((double)n_steps, edge / a.step_size) >= LONG_TRACK;
+}
+
+// Connectome launches: the persistent grid of the kernel's occupancy
+// (cached per device), at most one lane per seed, then the hits pass. Launches
+// in one generation (DTI always, as track launches) run the kernel without the
+// counting.
+template <int MODEL, int ALGO, int LMAX>
+hipError_t launch_connectome_fast_kernel(const FastConnectomeLaunch &f, hipStream_t stream)
+{
+    constexpr int BLOCK = fast_block<LMAX>();
+    const int64_t n = f.connectome.n_seeds, needed = (n + BLOCK - 1) / BLOCK;
+    int fill = 0;
     FastConnectomeLaunch gen = f;
-    gen.min_repack = MODEL == MODEL_DTI ? 0xffffffffu : FAST_MIN_REPACK;
-    const uint64_t first_work = std::min<uint64_t>((uint64_t)f.connectome.n_seeds, (uint64_t)blocks * fast_block<LMAX>());
-    const int generations = first_work / 2 >= gen.min_repack ? FAST_GENERATIONS : 1;
-    uint32_t *const lists[2] = {reinterpret_cast<uint32_t *>(f.connectome.cols),
-                                reinterpret_cast<uint32_t *>(f.connectome.cols) + f.connectome.n_seeds};
-    for (int g = 0; g < generations; g++) {
-        gen.list_in = g == 0 ? nullptr : lists[(g - 1) % 2];
-        gen.list_in_count = f.list_counts + (g + 1) % 2;
-        gen.list_out = lists[g % 2];
-        gen.list_out_count = f.list_counts + g % 2;
-        gen.last = g == generations - 1;
-        zero_product_generation<<<1, 64, 0, stream>>>(f.connectome.queue, f.ended, gen.list_out_count);
-        connectome_fast_kernel<MODEL, ALGO, LMAX>
-            <<<(unsigned)std::max<int64_t>(1, blocks >> g), fast_block<LMAX>(), 0, stream>>>(gen);
+    int generations = 0;
+    if constexpr (cut_short<MODEL, ALGO>()) {
+        if (const hipError_t e = fill_grid<connectome_fast_kernel<MODEL, ALGO, LMAX, true>>(BLOCK, &fill))
+            return e;
+        const int64_t blocks = std::min<int64_t>(fill, needed);
+        gen.min_repack = FAST_MIN_REPACK_PRODUCT;
+        if (in_generations(f.connectome.mask, f.connectome.algo, f.connectome.n_steps, std::min(n, blocks * BLOCK),
+                           ALGO == ALGO_PROBABILISTIC && f.connectome.algo.n_samples > 16))
+            generations = FAST_GENERATIONS;
+        uint32_t *const lists[2] = {reinterpret_cast<uint32_t *>(f.connectome.cols),
+                                    reinterpret_cast<uint32_t *>(f.connectome.cols) + n};
+        for (int g = 0; g < generations; g++) {
+            gen.list_in = g == 0 ? nullptr : lists[(g - 1) % 2];
+            gen.list_in_count = f.list_counts + (g + 1) % 2;
+            gen.list_out = lists[g % 2];
+            gen.list_out_count = f.list_counts + g % 2;
+            gen.last = g == generations - 1;
+            zero_product_generation<<<1, 64, 0, stream>>>(f.connectome.queue, f.ended, gen.list_out_count);
+            connectome_fast_kernel<MODEL, ALGO, LMAX, true>
+                <<<(unsigned)std::max<int64_t>(1, blocks >> g), BLOCK, 0, stream>>>(gen);
+        }
     }
-    e = hipGetLastError();
-    if (e != hipSuccess)
+    if (generations == 0) {
+        if (const hipError_t e = fill_grid<connectome_fast_kernel<MODEL, ALGO, LMAX, false>>(BLOCK, &fill))
+            return e;
+        zero_product_generation<<<1, 64, 0, stream>>>(f.connectome.queue, f.ended, f.list_counts);
+        connectome_fast_kernel<MODEL, ALGO, LMAX, false>
+            <<<(unsigned)std::min<int64_t>(fill, needed), BLOCK, 0, stream>>>(gen);
+    }
+    if (const hipError_t e = hipGetLastError())
         return e;
     return launch_connectome_hits(f.connectome, stream);
 }
@@ -2031,47 +2074,37 @@ hipError_t launch_connectome_fast_algo(const FastConnectomeLaunch &f, hipStream_
     }
 }
 
-// TOD launches: the persistent grid of the kernel's occupancy (cached per
-// device), at most one lane per seed.
+// TOD launches: as connectome launches, in generations where there is room
+// for the tracks cut short (at most half the lanes).
 template <int MODEL, int ALGO, int LMAX> hipError_t launch_tod_fast_kernel(const FastTodLaunch &f, hipStream_t stream)
 {
-    static std::atomic<int> cache[64] = {};
-    int device = 0;
-    hipError_t e = hipGetDevice(&device);
-    if (e != hipSuccess)
-        return e;
-    if (device < 0 || device >= 64)
-        return hipErrorInvalidDevice;
-    if (cache[device].load(std::memory_order_acquire) == 0) {
-        int per_cu = 0;
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per_cu, reinterpret_cast<const void *>(tod_fast_kernel<MODEL, ALGO, LMAX>), 256, 0);
-        if (e != hipSuccess)
-            return e;
-        int cus = 0;
-        e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device);
-        if (e != hipSuccess)
-            return e;
-        cache[device].store((cus > 0 ? cus : 1) * (per_cu > 0 ? per_cu : 1), std::memory_order_release);
-    }
-    const int64_t fill = cache[device].load(std::memory_order_acquire);
-    const int64_t needed = (f.tod.n_seeds + 255) / 256;
-    const int64_t blocks = std::min(fill, needed);
-    // As connectome launches. A generation saves at most half its lanes.
+    const int64_t n = f.tod.n_seeds, needed = (n + 255) / 256;
+    int fill = 0;
     FastTodLaunch gen = f;
-    gen.min_repack = MODEL == MODEL_DTI ? 0xffffffffu : FAST_MIN_REPACK;
-    const uint64_t first_work = std::min<uint64_t>((uint64_t)f.tod.n_seeds, (uint64_t)blocks * 256);
-    const int generations =
-        first_work / 2 >= gen.min_repack && first_work / 2 <= f.saved_room ? FAST_GENERATIONS : 1;
-    for (int g = 0; g < generations; g++) {
-        gen.saved_in = g == 0 ? nullptr : f.saved[(g - 1) % 2];
-        gen.saved_in_count = f.saved_counts + (g + 1) % 2;
-        gen.saved_out = f.saved[g % 2];
-        gen.saved_out_count = f.saved_counts + g % 2;
-        gen.last = g == generations - 1;
-        zero_product_generation<<<1, 64, 0, stream>>>(f.tod.queue, f.ended, gen.saved_out_count);
-        tod_fast_kernel<MODEL, ALGO, LMAX><<<(unsigned)std::max<int64_t>(1, blocks >> g), 256, 0, stream>>>(gen);
+    if constexpr (cut_short<MODEL, ALGO>()) {
+        if (const hipError_t e = fill_grid<tod_fast_kernel<MODEL, ALGO, LMAX, true>>(256, &fill))
+            return e;
+        const int64_t blocks = std::min<int64_t>(fill, needed), lanes = std::min(n, blocks * 256);
+        gen.min_repack = FAST_MIN_REPACK_PRODUCT;
+        if ((uint64_t)(lanes / 2) <= f.saved_room &&
+            in_generations(f.tod.mask, f.tod.algo, f.tod.n_steps, lanes, false)) {
+            for (int g = 0; g < FAST_GENERATIONS; g++) {
+                gen.saved_in = g == 0 ? nullptr : f.saved[(g - 1) % 2];
+                gen.saved_in_count = f.saved_counts + (g + 1) % 2;
+                gen.saved_out = f.saved[g % 2];
+                gen.saved_out_count = f.saved_counts + g % 2;
+                gen.last = g == FAST_GENERATIONS - 1;
+                zero_product_generation<<<1, 64, 0, stream>>>(f.tod.queue, f.ended, gen.saved_out_count);
+                tod_fast_kernel<MODEL, ALGO, LMAX, true>
+                    <<<(unsigned)std::max<int64_t>(1, blocks >> g), 256, 0, stream>>>(gen);
+            }
+            return hipGetLastError();
+        }
     }
+    if (const hipError_t e = fill_grid<tod_fast_kernel<MODEL, ALGO, LMAX, false>>(256, &fill))
+        return e;
+    zero_product_generation<<<1, 64, 0, stream>>>(f.tod.queue, f.ended, f.saved_counts);
+    tod_fast_kernel<MODEL, ALGO, LMAX, false><<<(unsigned)std::min<int64_t>(fill, needed), 256, 0, stream>>>(gen);
     return hipGetLastError();
 }
 
