@@ -92,7 +92,9 @@ int tgk_runtime_info(tgk_runtime *rt, char *name, int32_t name_len, int32_t *com
 int tgk_runtime_stream(tgk_runtime *rt, void **stream);
 /* Grid of the FAST path's persistent kernel in blocks (of the launch
  * shape's lanes, 256 by default); <= 0 (the default) sizes it to the
- * device's occupancy. No counterpart in the reference, whose kernel is
+ * device's occupancy. A set grid also keeps launches of few seeds on that
+ * kernel (TGK_FAST_FORM_LANES), and bounds the blocks, of 256 lanes, of
+ * launches by lane groups. No counterpart in the reference, whose kernel is
  * launched one work-item per seed; set by tractography_amd.autotune. */
 int tgk_runtime_set_fast_grid(tgk_runtime *rt, int32_t blocks);
 /* No counterpart in the reference (one work-item per seed, tracking.py:174).
@@ -100,7 +102,9 @@ int tgk_runtime_set_fast_grid(tgk_runtime *rt, int32_t blocks);
  * 0..TGK_FAST_SHAPES - 1, each a number of lanes per block (streamlines per
  * workgroup) and of a row's 45 coefficients kept in LDS between steps (the
  * rest in registers); tgk_fast_shape_info gives both. Other kernels run
- * shape 0. Results do not depend on it; set by tractography_amd.autotune. */
+ * shape 0, and a shape other than 0 keeps launches of few seeds on
+ * TGK_FAST_FORM_LANES. Results do not depend on it; set by
+ * tractography_amd.autotune. */
 #define TGK_FAST_SHAPES 5
 int tgk_runtime_set_fast_shape(tgk_runtime *rt, int32_t shape);
 int tgk_fast_shape_info(int32_t shape, int32_t *lanes_per_block, int32_t *lds_coefficients);
@@ -113,6 +117,20 @@ int tgk_fast_shape_info(int32_t shape, int32_t *lanes_per_block, int32_t *lds_co
  * calls run in one generation); a large value runs every call in one
  * launch. Results do not depend on it. */
 int tgk_runtime_set_fast_repack(tgk_runtime *rt, int32_t min_streamlines);
+/* No counterpart in the reference. With tuned != 0 the grid, shape and
+ * threshold set are taken as chosen for launches that fill the GPU (as
+ * tractography_amd.autotune chooses them): launches of few seeds, and those by
+ * lane groups, then run as if none were set. Setting any of them again clears
+ * it. */
+int tgk_runtime_set_fast_tuned(tgk_runtime *rt, int32_t tuned);
+/* How the last FAST-path tracking launch on this runtime tracked: one lane per
+ * streamline (the persistent kernel that grid, shape and threshold belong to),
+ * blocks of four wavefronts that share each step of 64 streamlines (order-8 SH
+ * Transport and Diffusion, few seeds), or groups of eight lanes per streamline
+ * (order-8 SH Deterministic; Probabilistic of 17 to 64 candidates, or of any
+ * number up to 64 with few seeds). Results do not depend on it. */
+enum { TGK_FAST_FORM_LANES = 0, TGK_FAST_FORM_SPLIT = 1, TGK_FAST_FORM_GROUPS = 2 };
+int tgk_runtime_fast_form(tgk_runtime *rt, int32_t *form);
 /* No counterpart in the reference (its kernel reads a voxel row every step):
  * how many coefficient rows and mask values the last FAST-path tracking
  * launch on this runtime read from memory, i.e. how often a lane's cached

@@ -67,3 +67,11 @@ def test_launch_shapes_and_grid_candidates():
         grids = autotune._grids(256, s["lanes_per_block"], (0.5, 1.0, 2.0))
         assert grids[0] == 0
         assert [g * s["lanes_per_block"] for g in grids[1:]] == [131072, 262144, 524288]
+
+
+def test_entries_of_replaced_kernels_are_not_reused():
+    mask = tg.domain.Image(tg.Nifti1Image(np.ones((2, 2, 2), dtype=np.uint8), np.eye(4)))
+    sh45 = tg.local.RealSymmetricSphericalHarmonics(45)
+    key = autotune.cache_key("gpu-a", tg.algorithm.Diffusion(sh45, step_size=0.1), mask)
+    assert key != "gpu-a|model=0|K=45|algorithm=1|domain=mask"
+    assert key.endswith(f"|kernels={autotune.KERNELS}")

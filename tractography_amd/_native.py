@@ -63,6 +63,8 @@ _SIGNATURES = {
     "tgk_runtime_create": (c_int, [c_int32, POINTER(c_void_p)]),
     "tgk_runtime_set_fast_grid": (c_int, [_P, c_int32]),
     "tgk_runtime_set_fast_shape": (c_int, [_P, c_int32]),
+    "tgk_runtime_set_fast_tuned": (c_int, [_P, c_int32]),
+    "tgk_runtime_fast_form": (c_int, [_P, POINTER(c_int32)]),
     "tgk_fast_shape_info": (c_int, [c_int32, POINTER(c_int32), POINTER(c_int32)]),
     "tgk_runtime_set_fast_repack": (c_int, [_P, c_int32]),
     "tgk_runtime_fast_reads": (c_int, [_P, POINTER(c_uint64), POINTER(c_uint64)]),

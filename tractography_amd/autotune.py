@@ -17,9 +17,11 @@ results:
 (``tgk_track_timed``: HIP events around the tracking launches, seeds uploaded
 beforehand, noise-stream seed 0, so the caller's algorithm draws nothing):
 first every shape at the default grid and threshold, then every grid and
-threshold with the fastest shape. It sets the fastest on the runtime and
-keeps it in a JSON file keyed by device, model, coefficient count, algorithm
-and domain kind, so later calls with the same key reuse it without timing.
+threshold with the fastest shape. It sets the fastest on the runtime, for
+launches that fill the GPU (launches of few seeds, and those by lane groups, keep
+their own forms), and keeps it in a JSON file keyed by device, model,
+coefficient count, algorithm, domain kind and the kernels' generation, so later
+calls with the same key reuse it without timing.
 None of this has a counterpart in the reference, whose OpenCL kernel runs one
 work-item per seed (tracking.py:174).
 """
@@ -41,6 +43,12 @@ from .tracking import point_capacity
 DEFAULT_GRID_FACTORS = (0.5, 1.0, 2.0)
 DEFAULT_REPACKS = (4096, 16384, 65536, 1 << 30)
 DEFAULT_SHAPES = tuple(range(_native.FAST_SHAPES))
+# Part of the cache's keys: what was tuned for kernels that have since been
+# replaced is not applied to their successors.
+KERNELS = 2
+# Seeds up to which a launch at the default settings takes wavefronts that
+# share steps, which have neither shape nor grid (mesh domains: twice as many).
+FEW_SEEDS = 32768
 
 
 def cache_path() -> Path:
@@ -56,7 +64,7 @@ def cache_key(device_name: str, algorithm, domain) -> str:
     descriptor = algorithm.descriptor()
     kind = "mesh" if isinstance(domain, Mesh) else "mask"
     return (f"{device_name}|model={descriptor.model}|K={descriptor.n_parameters}|"
-            f"algorithm={descriptor.algorithm}|domain={kind}")
+            f"algorithm={descriptor.algorithm}|domain={kind}|kernels={KERNELS}")
 
 
 def load_cache(path: Path | None = None) -> dict:
@@ -85,6 +93,7 @@ def apply(runtime: HipRuntime, entry: dict) -> None:
     runtime.set_fast_shape(int(entry.get("shape", 0)))
     runtime.set_fast_grid(int(entry["blocks"]))
     runtime.set_fast_repack(int(entry["repack"]))
+    runtime.set_fast_tuned(True)
 
 
 def _grids(units: int, lanes_per_block: int, factors) -> list[int]:
@@ -153,8 +162,11 @@ def tune_fast(algorithm, domain, field, seeds, *, runtime: HipRuntime, save_at: 
         if best is None or ms < best[0]:
             best = (ms, steps, shape, blocks, repack)
 
+    few = len(seeds) <= FEW_SEEDS * (2 if isinstance(domain, Mesh) else 1)
     for shape in shapes:
-        run(int(shape), 0, default_repack)
+        # Sized by occupancy, unless the sample would then not run the shape.
+        blocks = _grids(units, table[int(shape)]["lanes_per_block"], (1.0,))[-1] if few else 0
+        run(int(shape), blocks, default_repack)
     shape = best[2]
     for blocks in _grids(units, table[shape]["lanes_per_block"], grid_factors):
         for repack in repacks:

@@ -112,6 +112,8 @@ struct tgk_runtime {
     bool capturing = false;    // the stream is being recorded into a graph
     int32_t fast_grid = 0;     // blocks of the fast kernel; <= 0: sized by occupancy
     int32_t fast_shape = 0;    // launch shape of the order-8 SH Transport / Diffusion kernels
+    bool fast_tuned = false;   // grid, shape and threshold are for launches that fill the GPU
+    int32_t fast_form = TGK_FAST_FORM_LANES;  // of the last FAST tracking launch
     uint32_t fast_min_repack = 0;  // 0: the model's default (fast_launch); see tgk_runtime_set_fast_repack
 };
 
@@ -513,6 +515,7 @@ int tgk_runtime_set_fast_grid(tgk_runtime *rt, int32_t blocks)
     if (!rt)
         return fail(TGK_ERR_INVALID, "runtime is NULL");
     rt->fast_grid = blocks > 0 ? blocks : 0;
+    rt->fast_tuned = false;
     return TGK_OK;
 }
 
@@ -523,6 +526,23 @@ int tgk_runtime_set_fast_shape(tgk_runtime *rt, int32_t shape)
     if (shape < 0 || shape >= tgk::FAST_SHAPE_COUNT)
         return fail(TGK_ERR_INVALID, "fast launch shape %d: shapes are 0..%d", shape, tgk::FAST_SHAPE_COUNT - 1);
     rt->fast_shape = shape;
+    rt->fast_tuned = false;
+    return TGK_OK;
+}
+
+int tgk_runtime_set_fast_tuned(tgk_runtime *rt, int32_t tuned)
+{
+    if (!rt)
+        return fail(TGK_ERR_INVALID, "runtime is NULL");
+    rt->fast_tuned = tuned != 0;
+    return TGK_OK;
+}
+
+int tgk_runtime_fast_form(tgk_runtime *rt, int32_t *form)
+{
+    if (!rt || !form)
+        return fail(TGK_ERR_INVALID, "NULL argument");
+    *form = rt->fast_form;
     return TGK_OK;
 }
 
@@ -545,6 +565,7 @@ int tgk_runtime_set_fast_repack(tgk_runtime *rt, int32_t min_streamlines)
     if (min_streamlines < 1)
         return fail(TGK_ERR_INVALID, "min_streamlines must be positive, got %d", min_streamlines);
     rt->fast_min_repack = (uint32_t)min_streamlines;
+    rt->fast_tuned = false;
     return TGK_OK;
 }
 
@@ -921,9 +942,11 @@ int fast_launch(tgk_runtime *rt, tgk_field *field, const tgk_algorithm *algorith
         return fail(TGK_ERR_UNSUPPORTED, "the fast path takes grids of fewer than 2^32 - 2 voxels");
     f->shared_affine = p.domain_kind == tgk::DOMAIN_MASK && memcmp(p.mask.inv, p.field.inv, sizeof p.mask.inv) == 0;
     // Room for one generation's saved streamlines: one per lane of the grid.
-    int64_t lanes = 0;
-    TGK_HIP(tgk::prepare_track_fast(*f, rt->fast_grid, &lanes), "fast kernel occupancy");
-    const size_t bytes = (size_t)lanes * tgk::FAST_CONTINUATION_VEC4 * sizeof(float4);
+    tgk::FastPlan plan;
+    plan.grid_blocks = rt->fast_grid;
+    plan.query = true;
+    TGK_HIP(tgk::launch_track_fast(*f, plan, rt->stream), "fast kernel occupancy");
+    const size_t bytes = (size_t)plan.lanes * tgk::FAST_CONTINUATION_VEC4 * sizeof(float4);
     for (int i = 0; i < 2; i++) {
         if (int r = reserve(rt, rt->continuations[i], bytes, "saved streamlines"))
             return r;
@@ -1281,7 +1304,12 @@ int run_track(tgk_runtime *rt, const tgk_domain *domain, tgk_field *field, const
     tgk::FastLaunch f;
     if (int r = fast_launch(rt, field, algorithm, p, &f))
         return r;
-    TGK_HIP(tgk::launch_track_fast(f, rt->fast_grid, rt->stream), "fast tracking kernel");
+    tgk::FastPlan plan;
+    plan.grid_blocks = rt->fast_grid;
+    plan.repack_set = rt->fast_min_repack != 0;
+    plan.tuned = rt->fast_tuned;
+    TGK_HIP(tgk::launch_track_fast(f, plan, rt->stream), "fast tracking kernel");
+    rt->fast_form = plan.form;
     return TGK_OK;
 }
 

@@ -35,6 +35,7 @@
 
 #include "tgk_fast_model.h"
 #include "tgk_internal.h"
+#include "tgk.h"
 #include "tgk_sh_basis.h"
 
 namespace tgk {
@@ -1827,13 +1828,15 @@ template <int ALGO> bool grouped(const TrackLaunch &p)
 // 154, 124 and 113 ms with 600k.
 template <int ALGO> constexpr int group_blocks_per_cu() { return ALGO == ALGO_DETERMINISTIC ? 4 : 3; }
 template <int MODEL, int ALGO, int DOMAIN, int LMAX>
-hipError_t launch_group(const FastLaunch &f, int grid_blocks, bool query, hipStream_t stream)
+hipError_t launch_group(const FastLaunch &f, FastPlan &plan, hipStream_t stream)
 {
     int fill = 0, cus = 0;
     const hipError_t e = fill_grid<track_group_kernel<MODEL, ALGO, DOMAIN, LMAX>>(256, &fill, &cus);
-    if (e != hipSuccess || query)
+    if (e != hipSuccess || plan.query)
         return e;
+    plan.form = TGK_FAST_FORM_GROUPS;
     const int64_t needed = (f.track.n_seeds * fast::GROUP_LANES + 255) / 256;
+    int grid_blocks = plan.tuned ? 0 : plan.grid_blocks;
     if (grid_blocks <= 0)
         grid_blocks = (int)std::min<int64_t>(std::min(fill, group_blocks_per_cu<ALGO>() * cus),
                                              std::max<int64_t>(needed / cus, 1) * cus);
@@ -1859,20 +1862,20 @@ hipError_t launch_group(const FastLaunch &f, int grid_blocks, bool query, hipStr
 // from 65536); mesh domains, whose one-lane step is longer: 40k seeds 7.3 and
 // 6.6 ms, the last ones of 500k 12.85 and 12.77 from 65536 on.
 template <int DOMAIN> constexpr uint32_t split_lanes() { return DOMAIN == DOMAIN_MESH ? 65536 : 32768; }
-// query: only report the lanes of the grid a launch would use.
+// A grid, a shape other than 0 or a threshold that was set chooses the kernel
+// that has them for few seeds too, unless it was set for large launches.
 template <int MODEL, int ALGO, int DOMAIN, int LMAX, int S>
-hipError_t launch_fast(const FastLaunch &f, int grid_blocks, bool query, int64_t *lanes, hipStream_t stream)
+hipError_t launch_fast(const FastLaunch &f, FastPlan &plan, hipStream_t stream)
 {
     constexpr int BLOCK = shape_block<MODEL, ALGO, LMAX, S>();
-    const bool own_grid = grid_blocks <= 0;
-    if (own_grid) {
+    int grid_blocks = plan.grid_blocks;
+    if (grid_blocks <= 0) {
         const hipError_t e = fill_grid<track_fast_kernel<MODEL, ALGO, DOMAIN, LMAX, S>>(BLOCK, &grid_blocks);
         if (e != hipSuccess)
             return e;
     }
-    if (lanes)
-        *lanes = (int64_t)grid_blocks * BLOCK;
-    if (query)
+    plan.lanes = (int64_t)grid_blocks * BLOCK;
+    if (plan.query)
         return hipSuccess;
     // Generation g resumes what g - 1 saved in cont[(g - 1) % 2] and saves
     // into cont[g % 2], whose count (generation g - 2's, consumed by g - 1)
@@ -1880,10 +1883,14 @@ hipError_t launch_fast(const FastLaunch &f, int grid_blocks, bool query, int64_t
     // A first generation that is never cut short (half its resident work
     // below the repack threshold) is the only one.
     const uint64_t first_work = std::min<uint64_t>((uint64_t)f.track.n_seeds, (uint64_t)grid_blocks * BLOCK);
-    const int generations = first_work / 2 >= f.min_repack ? FAST_GENERATIONS : 1;
+    int generations = first_work / 2 >= f.min_repack ? FAST_GENERATIONS : 1;
     FastLaunch gen = f;
     constexpr bool SPLIT = shaped<MODEL, ALGO, LMAX>();
-    const bool split_all = SPLIT && generations == 1 && own_grid && f.track.n_seeds <= split_lanes<DOMAIN>();
+    const bool split_all = SPLIT && f.track.n_seeds <= split_lanes<DOMAIN>() &&
+                           (plan.tuned || (plan.grid_blocks <= 0 && S == 0 && (generations == 1 || !plan.repack_set)));
+    plan.form = split_all ? TGK_FAST_FORM_SPLIT : TGK_FAST_FORM_LANES;
+    if (split_all)
+        generations = 1;
     // What the last generation can be handed (see above).
     const bool split_last = SPLIT && generations > 1 &&
                             ((int64_t)grid_blocks * BLOCK >> (FAST_GENERATIONS - 1)) <= split_lanes<DOMAIN>();
@@ -1912,68 +1919,65 @@ hipError_t launch_fast(const FastLaunch &f, int grid_blocks, bool query, int64_t
 
 // By lane groups where they track, else one lane per streamline.
 template <int MODEL, int ALGO, int DOMAIN, int LMAX, int S>
-hipError_t launch_tracks(const FastLaunch &f, int grid, bool query, int64_t *lanes, hipStream_t stream)
+hipError_t launch_tracks(const FastLaunch &f, FastPlan &plan, hipStream_t stream)
 {
     if constexpr (groupable<MODEL, ALGO, LMAX>()) {
         // Queried for every launch: a later one may be grouped.
-        if (query || grouped<ALGO>(f.track)) {
-            const hipError_t e = launch_group<MODEL, ALGO, DOMAIN, LMAX>(f, grid, query, stream);
-            if (e != hipSuccess || !query)
+        if (plan.query || grouped<ALGO>(f.track)) {
+            const hipError_t e = launch_group<MODEL, ALGO, DOMAIN, LMAX>(f, plan, stream);
+            if (e != hipSuccess || !plan.query)
                 return e;
         }
-        if constexpr (ALGO == ALGO_DETERMINISTIC) {
-            if (lanes)
-                *lanes = 0;  // groups save no streamlines
-            return hipSuccess;
-        }
+        if constexpr (ALGO == ALGO_DETERMINISTIC)
+            return hipSuccess;  // plan.lanes = 0: groups save no streamlines
     }
     if constexpr (!groupable<MODEL, ALGO, LMAX>() || ALGO != ALGO_DETERMINISTIC)
-        return launch_fast<MODEL, ALGO, DOMAIN, LMAX, S>(f, grid, query, lanes, stream);
+        return launch_fast<MODEL, ALGO, DOMAIN, LMAX, S>(f, plan, stream);
 }
 
 template <int MODEL, int ALGO, int DOMAIN>
-hipError_t launch_fast_order(const FastLaunch &f, int grid, bool query, int64_t *lanes, hipStream_t stream)
+hipError_t launch_fast_order(const FastLaunch &f, FastPlan &plan, hipStream_t stream)
 {
     if constexpr (MODEL == MODEL_SH) {
         if (f.sh_order == 12)
-            return launch_tracks<MODEL, ALGO, DOMAIN, 12, 0>(f, grid, query, lanes, stream);
+            return launch_tracks<MODEL, ALGO, DOMAIN, 12, 0>(f, plan, stream);
     }
     if constexpr (shaped<MODEL, ALGO, 8>()) {
         switch (f.shape) {
-        case 1: return launch_tracks<MODEL, ALGO, DOMAIN, 8, 1>(f, grid, query, lanes, stream);
-        case 2: return launch_tracks<MODEL, ALGO, DOMAIN, 8, 2>(f, grid, query, lanes, stream);
-        case 3: return launch_tracks<MODEL, ALGO, DOMAIN, 8, 3>(f, grid, query, lanes, stream);
-        case 4: return launch_tracks<MODEL, ALGO, DOMAIN, 8, 4>(f, grid, query, lanes, stream);
+        case 1: return launch_tracks<MODEL, ALGO, DOMAIN, 8, 1>(f, plan, stream);
+        case 2: return launch_tracks<MODEL, ALGO, DOMAIN, 8, 2>(f, plan, stream);
+        case 3: return launch_tracks<MODEL, ALGO, DOMAIN, 8, 3>(f, plan, stream);
+        case 4: return launch_tracks<MODEL, ALGO, DOMAIN, 8, 4>(f, plan, stream);
         default: break;
         }
     }
-    return launch_tracks<MODEL, ALGO, DOMAIN, 8, 0>(f, grid, query, lanes, stream);
+    return launch_tracks<MODEL, ALGO, DOMAIN, 8, 0>(f, plan, stream);
 }
 
 template <int MODEL, int ALGO>
-hipError_t launch_fast_domain(const FastLaunch &f, int grid, bool query, int64_t *blocks, hipStream_t stream)
+hipError_t launch_fast_domain(const FastLaunch &f, FastPlan &plan, hipStream_t stream)
 {
     if (f.track.domain_kind == DOMAIN_MESH)
-        return launch_fast_order<MODEL, ALGO, DOMAIN_MESH>(f, grid, query, blocks, stream);
-    return launch_fast_order<MODEL, ALGO, DOMAIN_MASK>(f, grid, query, blocks, stream);
+        return launch_fast_order<MODEL, ALGO, DOMAIN_MESH>(f, plan, stream);
+    return launch_fast_order<MODEL, ALGO, DOMAIN_MASK>(f, plan, stream);
 }
 
 template <int MODEL>
-hipError_t launch_fast_algo(const FastLaunch &f, int grid, bool query, int64_t *blocks, hipStream_t stream)
+hipError_t launch_fast_algo(const FastLaunch &f, FastPlan &plan, hipStream_t stream)
 {
     switch (f.track.algo.algorithm) {
-    case ALGO_DIFFUSION: return launch_fast_domain<MODEL, ALGO_DIFFUSION>(f, grid, query, blocks, stream);
-    case ALGO_PROBABILISTIC: return launch_fast_domain<MODEL, ALGO_PROBABILISTIC>(f, grid, query, blocks, stream);
-    case ALGO_DETERMINISTIC: return launch_fast_domain<MODEL, ALGO_DETERMINISTIC>(f, grid, query, blocks, stream);
-    default: return launch_fast_domain<MODEL, ALGO_TRANSPORT>(f, grid, query, blocks, stream);
+    case ALGO_DIFFUSION: return launch_fast_domain<MODEL, ALGO_DIFFUSION>(f, plan, stream);
+    case ALGO_PROBABILISTIC: return launch_fast_domain<MODEL, ALGO_PROBABILISTIC>(f, plan, stream);
+    case ALGO_DETERMINISTIC: return launch_fast_domain<MODEL, ALGO_DETERMINISTIC>(f, plan, stream);
+    default: return launch_fast_domain<MODEL, ALGO_TRANSPORT>(f, plan, stream);
     }
 }
 
-hipError_t dispatch_fast(const FastLaunch &f, int grid, bool query, int64_t *blocks, hipStream_t stream)
+hipError_t dispatch_fast(const FastLaunch &f, FastPlan &plan, hipStream_t stream)
 {
     if (f.track.algo.model == MODEL_DTI)
-        return launch_fast_algo<MODEL_DTI>(f, grid, query, blocks, stream);
-    return launch_fast_algo<MODEL_SH>(f, grid, query, blocks, stream);
+        return launch_fast_algo<MODEL_DTI>(f, plan, stream);
+    return launch_fast_algo<MODEL_SH>(f, plan, stream);
 }
 
 // Whether a connectome or TOD launch of the SH model, `lanes` tracks at a
@@ -2131,18 +2135,13 @@ hipError_t launch_tod_fast_algo(const FastTodLaunch &f, hipStream_t stream)
 
 }  // namespace
 
-hipError_t launch_track_fast(const FastLaunch &f, int grid_blocks, hipStream_t stream)
+hipError_t launch_track_fast(const FastLaunch &f, FastPlan &plan, hipStream_t stream)
 {
-    if (f.track.n_seeds == 0)
+    if (f.track.n_seeds == 0 && !plan.query)
         return hipSuccess;
     if (f.track.n_seeds >= (int64_t)1 << 31)
         return hipErrorInvalidValue;
-    return dispatch_fast(f, grid_blocks, false, nullptr, stream);
-}
-
-hipError_t prepare_track_fast(const FastLaunch &f, int grid_blocks, int64_t *lanes)
-{
-    return dispatch_fast(f, grid_blocks, true, lanes, nullptr);
+    return dispatch_fast(f, plan, stream);
 }
 
 hipError_t launch_connectome_fast(const FastConnectomeLaunch &f, hipStream_t stream)

@@ -182,15 +182,18 @@ struct FastLaunch {
     int32_t shape;              // launch shape, 0..FAST_SHAPE_COUNT - 1
     uint64_t group_jump[9];     // lane-group kernels: noise-stream multipliers to lane b's first draw and, last, past all
 };
-// grid_blocks <= 0 sizes the persistent grid to the device's occupancy
-// (computed once per kernel and device, then cached). n_seeds must be below
-// 2^31.
-hipError_t launch_track_fast(const FastLaunch &p, int grid_blocks, hipStream_t stream);
-// Computes and caches that occupancy for the kernel `p` selects, launching
-// nothing (so later launches make no device queries, e.g. while a graph is
-// being recorded); *lanes receives the lanes of the grid a launch with
-// grid_blocks would use (they bound the saved streamlines of a generation).
-hipError_t prepare_track_fast(const FastLaunch &p, int grid_blocks, int64_t *lanes);
+// How a launch is made.
+struct FastPlan {
+    int32_t grid_blocks = 0;  // <= 0: sized to the device's occupancy (computed once per kernel and device)
+    bool repack_set = false;  // FastLaunch::min_repack is not the default
+    bool tuned = false;       // grid, shape and threshold are for launches that fill the GPU (tgk_runtime_set_fast_tuned)
+    bool query = false;       // compute and cache occupancies, launch nothing
+    int64_t lanes = 0;        // out: lanes of the persistent grid (they bound a generation's saved streamlines)
+    int32_t form = 0;         // out: TGK_FAST_FORM_*
+};
+// n_seeds must be below 2^31. A query lets later launches make no device
+// queries, e.g. while a graph is being recorded.
+hipError_t launch_track_fast(const FastLaunch &p, FastPlan &plan, hipStream_t stream);
 // Dense seed-major rows (both paths) -> ragged points.
 hipError_t launch_compact_seed_major(const float *dense, int64_t n_seeds, uint32_t n_points,
                                      const uint32_t *lengths, const int64_t *offsets, float *out,

@@ -91,6 +91,20 @@ class HipRuntime:
         no longer cuts a generation short to repack its streamlines."""
         _native.check(_native.lib().tgk_runtime_set_fast_repack(self._handle, int(min_streamlines)))
 
+    def set_fast_tuned(self, tuned: bool) -> None:
+        """Whether the grid, shape and threshold set were chosen for launches
+        that fill the GPU: launches of few seeds, and those by lane groups,
+        then run as if none were set. Setting any of them clears it."""
+        _native.check(_native.lib().tgk_runtime_set_fast_tuned(self._handle, int(tuned)))
+
+    def fast_form(self) -> str:
+        """How the last fast-path tracking launch tracked: "lanes" (one per
+        streamline), "split" (wavefronts that share the steps of 64
+        streamlines) or "groups" (eight lanes per streamline)."""
+        form = ctypes.c_int32()
+        _native.check(_native.lib().tgk_runtime_fast_form(self._handle, ctypes.byref(form)))
+        return ("lanes", "split", "groups")[form.value]
+
     def fast_reads(self) -> dict:
         """Coefficient rows and mask values the last fast-path tracking launch
         read from memory (each lane reads them only when its cell changes)."""
