@@ -150,8 +150,8 @@ int tgk_track_timed(tgk_runtime *rt, const tgk_domain *domain, const tgk_field *
 /* No counterpart in the reference (its results come back in memory of its
  * own, opencl.py:200-230). Page-locked host memory of `bytes` bytes: as the
  * output of a blocking call it is filled by DMA at the link's rate, where
- * pageable memory is staged through buffers of the driver and faulted in page
- * by page. Any thread may free it, once, after the last use. */
+ * pageable memory is staged and faulted in page by page. Any thread may free
+ * it, once, after the last use. A forked child does not have it. */
 int tgk_host_alloc(size_t bytes, void **ptr);
 int tgk_host_free(void *ptr);
 

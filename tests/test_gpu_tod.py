@@ -434,3 +434,62 @@ def test_fast_tod_through_the_public_api():
     assert (populated == (plain[..., 0] != 0)).mean() > 0.99
     both = populated & (plain[..., 0] != 0)
     assert float(np.abs(fast[both] - plain[both]).mean()) < 1e-2
+
+
+def test_large_grids_come_in_memory_of_the_callers(runtime):
+    # Outputs of several 8 MiB chunks: none (just below one), a whole number
+    # and a remainder. The array is ordinary memory, which a forked process
+    # also has ("dc" marks a mapping that it would not) and which lives as long
+    # as the array does. Sums of the same tracks differ in rounding only.
+    fod, seed_mask, _ = fixtures.cross()
+    field, domain = tg.field.Image(fod), tg.domain.Image(seed_mask)
+    model = tg.local.RealSymmetricSphericalHarmonics(45)
+    algorithm = tg.algorithm.Transport(model, step_size=0.1)
+    handle = domain.upload(runtime, with_boundary=True)
+    for nx in (4660, 4661, 16 * 4661, 10_007):
+        # Cells of 10 / nx along x, so that tracks deposit in every chunk.
+        grid = tg.Nifti1Image(np.zeros((nx, 10, 1), dtype=np.uint8), np.diag([10.0 / nx, 1.0, 1.0, 1.0]))
+        got = tg.tracking.tod(algorithm, domain, field, grid, 5000, 10.0, runtime).dataobj
+        dims = np.array((nx, 10, 1), dtype=np.uint32)
+        inverse = np.ascontiguousarray(np.linalg.inv(grid.affine), dtype=np.float32)
+        d_out = torch.full((nx * 10 * 45,), np.nan, device="cuda")
+        torch.cuda.synchronize()
+        _native.check(_native.lib().tgk_tod_device(
+            runtime.handle, handle.handle, handle.handle, field.upload(runtime).handle, algorithm.descriptor(),
+            _native.PATH_PLAIN, algorithm.get_rng_seed(), 5000, 100, _native.ptr(dims), _native.ptr(inverse), 1,
+            d_out.data_ptr()))
+        runtime.finish()
+        ref = d_out.cpu().numpy().reshape(nx, 10, 1, 45)
+        deposits = np.flatnonzero(ref[..., 0].any(axis=(1, 2)))
+        assert deposits[0] < 0.1 * nx and deposits[-1] > 0.8 * nx
+        np.testing.assert_allclose(got, ref, rtol=0, atol=1e-4)
+        address, flags = got.ctypes.data + got.nbytes // 2, None
+        with open("/proc/self/smaps") as maps:
+            for line in maps:
+                if not line[0].isupper():
+                    low, high = (int(x, 16) for x in line.split()[0].split("-"))
+                elif line.startswith("VmFlags") and low <= address < high:
+                    flags = line.split()[1:]
+        assert flags is not None and "dc" not in flags
+
+
+def test_page_locked_outputs(runtime):
+    # The library's own page-locked memory, filled by one DMA.
+    domain, field, algorithm, shape = _scene("sh45-transport")
+    dims = np.array((16 * 4661, 10, 1), dtype=np.uint32)
+    inverse = np.eye(4, dtype=np.float32)
+    size = int(dims.prod()) * 45
+    lib, address = _native.lib(), ctypes.c_void_p()
+    _native.check(lib.tgk_host_alloc(4 * size, ctypes.byref(address)))
+    out = np.frombuffer((ctypes.c_char * (4 * size)).from_address(address.value), dtype=np.float32)
+    out[:] = np.nan
+    handle = domain.upload(runtime, with_boundary=True)
+    _native.check(lib.tgk_tod(
+        runtime.handle, handle.handle, handle.handle, field.upload(runtime).handle, algorithm.descriptor(),
+        _native.PATH_PLAIN, 3, 2000, 50, _native.ptr(dims), _native.ptr(inverse), 1, _native.ptr(out)))
+    ref = _device_tod(runtime, domain, field, algorithm, 3, 2000, 50, dims, inverse, normalize=1)
+    np.testing.assert_allclose(out, ref.reshape(-1), rtol=0, atol=1e-4)
+    del out
+    _native.check(lib.tgk_host_free(address))
+    assert lib.tgk_host_alloc(0, ctypes.byref(address)) == _native.ERR_INVALID
+    assert lib.tgk_host_free(None) == _native.OK

@@ -7,7 +7,6 @@ host fallback: without libtgk.so every device entry point raises.
 from __future__ import annotations
 
 import ctypes
-import weakref
 from ctypes import POINTER, c_char_p, c_float, c_int, c_int32, c_int64, c_size_t, c_uint32, c_uint64, c_void_p
 from pathlib import Path
 
@@ -185,31 +184,6 @@ def ptr(array: np.ndarray | None) -> int | None:
     if not array.flags.c_contiguous:
         raise ValueError("arrays passed to libtgk.so must be C-contiguous")
     return array.ctypes.data
-
-
-# Outputs from this size on are allocated page-locked: below, allocating them
-# takes longer than the staged copy it saves.
-PAGE_LOCKED_BYTES = 4 << 20
-
-
-class _HostMemory:
-    """Owns page-locked memory: freed when the last array over it goes."""
-
-    def __init__(self, address: c_void_p):
-        self._finalizer = weakref.finalize(self, lib().tgk_host_free, address)
-
-
-def output_array(shape, dtype) -> np.ndarray:
-    """An uninitialised array for a call's output: page-locked when it is
-    large and such memory is to be had, so that the device fills it by DMA
-    (197 MB into a fresh pageable array took 20 ms, into this 4)."""
-    size = int(np.prod(shape, dtype=np.int64)) * np.dtype(dtype).itemsize
-    address = c_void_p()
-    if size < PAGE_LOCKED_BYTES or lib().tgk_host_alloc(size, ctypes.byref(address)) != OK:
-        return np.empty(shape, dtype=dtype)
-    buffer = (ctypes.c_char * size).from_address(address.value)
-    buffer._owner = _HostMemory(address)
-    return np.frombuffer(buffer, dtype=dtype).reshape(shape)
 
 
 def algorithm_struct(model: int, algorithm: int, n_parameters: int, step_size: float, gamma: float,

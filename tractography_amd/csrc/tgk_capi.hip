@@ -1,6 +1,7 @@
 // tgk_capi.hip -- the extern "C" boundary of libtgk.so (declared in
 // include/tgk.h): runtime and buffer ownership, argument validation, chunked
 // host-array tracking and the one-op drivers.
+#include <emmintrin.h>
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -82,6 +83,56 @@ struct DeviceBuffer {
 
 }  // namespace
 
+// Page-locked host memory (hipHostMalloc): the device writes it by DMA at
+// the link's full rate, and the host reads it as ordinary cached memory.
+struct PinnedBuffer {
+    void *ptr = nullptr;
+    size_t bytes = 0;
+    PinnedBuffer() = default;
+    PinnedBuffer(const PinnedBuffer &) = delete;
+    PinnedBuffer &operator=(const PinnedBuffer &) = delete;
+    ~PinnedBuffer()
+    {
+        if (ptr)
+            (void)hipHostFree(ptr);
+    }
+    hipError_t allocate(size_t n)
+    {
+        hipError_t e = hipHostMalloc(&ptr, n, hipHostMallocDefault);
+        if (e == hipSuccess)
+            bytes = n;
+        else
+            ptr = nullptr;
+        return e;
+    }
+};
+
+// Two page-locked chunks that a large output passes through on its way to the
+// caller's ordinary memory (fetch_large), kept by the runtime.
+struct OutputStage {
+    static constexpr size_t CHUNK = (size_t)8 << 20;
+    PinnedBuffer chunk[2];
+    hipEvent_t arrived[2] = {nullptr, nullptr};
+    ~OutputStage()
+    {
+        for (hipEvent_t e : arrived)
+            if (e)
+                (void)hipEventDestroy(e);
+    }
+    // Made on first use; false where it cannot be had.
+    bool ready()
+    {
+        for (int i = 0; i < 2; i++) {
+            if ((!chunk[i].ptr && chunk[i].allocate(CHUNK) != hipSuccess) ||
+                (!arrived[i] && hipEventCreateWithFlags(&arrived[i], hipEventDisableTiming) != hipSuccess)) {
+                (void)hipGetLastError();
+                return false;
+            }
+        }
+        return true;
+    }
+};
+
 // Byte offsets in the runtime's 256-byte queue buffer (offset 0: the seed
 // counter of the connectome and TOD kernels): the fast kernel's last-launch
 // read totals (two u64: coefficient rows, mask values) and its two
@@ -107,6 +158,7 @@ struct tgk_runtime {
     DeviceBuffer fast_counters;     // claim counter and ended-streamline shards of the fast kernel
     TrackBuffers track_buffers;     // tgk_track's working buffers
     DeviceBuffer product;           // tgk_tod's grid, tgk_connectome's entries (kept, as those)
+    OutputStage stage;              // of tgk_tod's grid on its way out
     DeviceBuffer seeds_table;  // prepared FOD-seeding table for seeds_key
     int32_t seeds_key[3] = {-1, -1, -1};  // model, K, method
     bool capturing = false;    // the stream is being recorded into a graph
@@ -149,30 +201,6 @@ struct tgk_domain {
     uint32_t near_dims[3] = {0, 0, 0};
     float near_inverse_affine[16];
     float reach = 0.0f;
-};
-
-// Page-locked host memory (hipHostMalloc): the device writes it by DMA at
-// the link's full rate, and the host reads it as ordinary cached memory.
-struct PinnedBuffer {
-    void *ptr = nullptr;
-    size_t bytes = 0;
-    PinnedBuffer() = default;
-    PinnedBuffer(const PinnedBuffer &) = delete;
-    PinnedBuffer &operator=(const PinnedBuffer &) = delete;
-    ~PinnedBuffer()
-    {
-        if (ptr)
-            (void)hipHostFree(ptr);
-    }
-    hipError_t allocate(size_t n)
-    {
-        hipError_t e = hipHostMalloc(&ptr, n, hipHostMallocDefault);
-        if (e == hipSuccess)
-            bytes = n;
-        else
-            ptr = nullptr;
-        return e;
-    }
 };
 
 // Copies spans of host memory with up to 8 threads, in slices of at least
@@ -1341,6 +1369,69 @@ template <class T> int fetch(T *host, const T *dev, size_t count, hipStream_t s)
     return TGK_OK;
 }
 
+bool is_page_locked(const void *host)
+{
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, host) == hipSuccess)
+        return a.type == hipMemoryTypeHost;
+    (void)hipGetLastError();  // ordinary memory is no pointer of HIP's
+    return false;
+}
+
+// memcpy past the caches, which a large output would only pass through: stores
+// that read no lines first (fetch_large's example: 18.3 -> 16.5 ms).
+void stream_copy(char *out, const char *in, size_t bytes)
+{
+    size_t at = 0;
+    if (((uintptr_t)out | (uintptr_t)in) % 16 == 0) {
+        for (; at + 64 <= bytes; at += 64) {
+            const __m128i *from = reinterpret_cast<const __m128i *>(in + at);
+            __m128i *to = reinterpret_cast<__m128i *>(out + at);
+            const __m128i a = _mm_load_si128(from), b = _mm_load_si128(from + 1), c = _mm_load_si128(from + 2),
+                          d = _mm_load_si128(from + 3);
+            _mm_stream_si128(to, a);
+            _mm_stream_si128(to + 1, b);
+            _mm_stream_si128(to + 2, c);
+            _mm_stream_si128(to + 3, d);
+        }
+        _mm_sfence();
+    }
+    memcpy(out + at, in + at, bytes - at);
+}
+
+// As fetch, for an output of many megabytes in memory of the caller's. Ordinary
+// memory that is new to the process is faulted in page by page, and a copy into
+// it by the driver waits for that and for its own staging: 197 MB took 18.5 ms.
+// Its pages are touched here while the device still computes, and the chunks of
+// the stage are copied while the next ones arrive. tg.tod, 97 x 116 x 97, 300k
+// seeds: 29.8 -> 16.5 ms per call, against 15.4 into page-locked memory, which
+// would not outlive a fork or the library.
+int fetch_large(tgk_runtime *rt, void *host, const void *dev, size_t bytes)
+{
+    constexpr size_t CHUNK = OutputStage::CHUNK;
+    char *out = static_cast<char *>(host);
+    if (bytes < CHUNK || is_page_locked(host) || !rt->stage.ready())
+        return fetch(out, static_cast<const char *>(dev), bytes, rt->stream);
+    volatile char *page = out;
+    for (size_t at = 0; at < bytes; at += 4096)
+        page[at] = page[at];
+    const size_t chunks = (bytes + CHUNK - 1) / CHUNK;
+    const auto size = [&](size_t i) { return std::min(CHUNK, bytes - i * CHUNK); };
+    for (size_t i = 0; i <= chunks; i++) {
+        if (i < chunks) {
+            TGK_HIP(hipMemcpyAsync(rt->stage.chunk[i % 2].ptr, static_cast<const char *>(dev) + i * CHUNK, size(i),
+                                   hipMemcpyDeviceToHost, rt->stream),
+                    "output copy");
+            TGK_HIP(hipEventRecord(rt->stage.arrived[i % 2], rt->stream), "output copy");
+        }
+        if (i > 0) {
+            TGK_HIP(hipEventSynchronize(rt->stage.arrived[(i - 1) % 2]), "output copy");
+            stream_copy(out + (i - 1) * CHUNK, static_cast<const char *>(rt->stage.chunk[(i - 1) % 2].ptr), size(i - 1));
+        }
+    }
+    return TGK_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1782,7 +1873,7 @@ int tgk_tod(tgk_runtime *rt, const tgk_domain *domain, const tgk_domain *boundar
     float *dout = rt->product.as<float>();
     if (int r = enqueue_tod(rt, const_cast<tgk_field *>(field), algorithm, path, t, n_values, normalize, dout))
         return r;
-    return fetch(coefficients, dout, (size_t)n_values, rt->stream);
+    return fetch_large(rt, coefficients, dout, (size_t)n_values * sizeof(float));
 }
 
 int tgk_tod_device(tgk_runtime *rt, const tgk_domain *domain, const tgk_domain *boundary, const tgk_field *field,

@@ -221,7 +221,7 @@ def tod(
         runtime = HipRuntime()
     domain_handle = domain.upload(runtime, with_boundary=True)
     field_handle = field.upload(runtime)
-    out = _native.output_array(output_shape + (45,), np.float32)
+    out = np.empty(output_shape + (45,), dtype=np.float32)
     dims = np.asarray(output_shape, dtype=np.uint32)
     _native.check(
         _native.lib().tgk_tod(
