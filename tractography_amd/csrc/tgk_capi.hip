@@ -13,6 +13,7 @@
 #include <atomic>
 #include <mutex>
 #include <new>
+#include <system_error>
 #include <thread>
 #include <string>
 #include <deque>
@@ -107,12 +108,13 @@ struct PinnedBuffer {
     }
 };
 
-// Two page-locked chunks that a large output passes through on its way to the
-// caller's ordinary memory (fetch_large), kept by the runtime.
+// Page-locked chunks that a large output passes through on its way to the
+// caller's ordinary memory (fetch_large), kept by the runtime: two for each of
+// the two threads that copy out of them.
 struct OutputStage {
-    static constexpr size_t CHUNK = (size_t)8 << 20;
-    PinnedBuffer chunk[2];
-    hipEvent_t arrived[2] = {nullptr, nullptr};
+    static constexpr size_t CHUNK = (size_t)4 << 20;
+    PinnedBuffer chunk[4];
+    hipEvent_t arrived[4] = {nullptr, nullptr, nullptr, nullptr};
     ~OutputStage()
     {
         for (hipEvent_t e : arrived)
@@ -122,7 +124,7 @@ struct OutputStage {
     // Made on first use; false where it cannot be had.
     bool ready()
     {
-        for (int i = 0; i < 2; i++) {
+        for (int i = 0; i < 4; i++) {
             if ((!chunk[i].ptr && chunk[i].allocate(CHUNK) != hipSuccess) ||
                 (!arrived[i] && hipEventCreateWithFlags(&arrived[i], hipEventDisableTiming) != hipSuccess)) {
                 (void)hipGetLastError();
@@ -1399,36 +1401,72 @@ void stream_copy(char *out, const char *in, size_t bytes)
     memcpy(out + at, in + at, bytes - at);
 }
 
+// `bytes` from the device through the stage's chunks first and first + 1: one
+// is copied on while the other fills.
+hipError_t fetch_staged(OutputStage &stage, int first, char *host, const char *dev, size_t bytes, hipStream_t stream)
+{
+    constexpr size_t CHUNK = OutputStage::CHUNK;
+    const size_t chunks = (bytes + CHUNK - 1) / CHUNK;
+    const auto size = [&](size_t i) { return std::min(CHUNK, bytes - i * CHUNK); };
+    for (size_t i = 0; i <= chunks; i++) {
+        hipError_t e = hipSuccess;
+        if (i < chunks) {
+            const int c = first + (int)(i % 2);
+            e = hipMemcpyAsync(stage.chunk[c].ptr, dev + i * CHUNK, size(i), hipMemcpyDeviceToHost, stream);
+            if (e == hipSuccess)
+                e = hipEventRecord(stage.arrived[c], stream);
+        }
+        if (e == hipSuccess && i > 0) {
+            const int c = first + (int)((i - 1) % 2);
+            e = hipEventSynchronize(stage.arrived[c]);
+            if (e == hipSuccess)
+                stream_copy(host + (i - 1) * CHUNK, static_cast<const char *>(stage.chunk[c].ptr), size(i - 1));
+        }
+        if (e != hipSuccess) {
+            (void)hipStreamSynchronize(stream);  // no copy into the stage outlives the call
+            return e;
+        }
+    }
+    return hipSuccess;
+}
+
 // As fetch, for an output of many megabytes in memory of the caller's. Ordinary
 // memory that is new to the process is faulted in page by page, and a copy into
 // it by the driver waits for that and for its own staging: 197 MB took 18.5 ms.
-// Its pages are touched here while the device still computes, and the chunks of
-// the stage are copied while the next ones arrive. tg.tod, 97 x 116 x 97, 300k
-// seeds: 29.8 -> 16.5 ms per call, against 15.4 into page-locked memory, which
-// would not outlive a fork or the library.
+// Its pages are touched here while the device still computes, and two threads
+// copy a half each through the stage (one alone keeps up with two thirds of the
+// link's rate). tgk_tod, 97 x 116 x 97, 300k seeds: 29.8 -> 15.5 ms per call (one
+// thread 16.5), against 15.4 into page-locked memory, which a forked child does
+// not have.
 int fetch_large(tgk_runtime *rt, void *host, const void *dev, size_t bytes)
 {
     constexpr size_t CHUNK = OutputStage::CHUNK;
     char *out = static_cast<char *>(host);
-    if (bytes < CHUNK || is_page_locked(host) || !rt->stage.ready())
-        return fetch(out, static_cast<const char *>(dev), bytes, rt->stream);
+    const char *in = static_cast<const char *>(dev);
+    if (bytes < 2 * CHUNK || is_page_locked(host) || !rt->stage.ready())
+        return fetch(out, in, bytes, rt->stream);
     volatile char *page = out;
     for (size_t at = 0; at < bytes; at += 4096)
         page[at] = page[at];
-    const size_t chunks = (bytes + CHUNK - 1) / CHUNK;
-    const auto size = [&](size_t i) { return std::min(CHUNK, bytes - i * CHUNK); };
-    for (size_t i = 0; i <= chunks; i++) {
-        if (i < chunks) {
-            TGK_HIP(hipMemcpyAsync(rt->stage.chunk[i % 2].ptr, static_cast<const char *>(dev) + i * CHUNK, size(i),
-                                   hipMemcpyDeviceToHost, rt->stream),
-                    "output copy");
-            TGK_HIP(hipEventRecord(rt->stage.arrived[i % 2], rt->stream), "output copy");
-        }
-        if (i > 0) {
-            TGK_HIP(hipEventSynchronize(rt->stage.arrived[(i - 1) % 2]), "output copy");
-            stream_copy(out + (i - 1) * CHUNK, static_cast<const char *>(rt->stage.chunk[(i - 1) % 2].ptr), size(i - 1));
-        }
+    const size_t half = (bytes / 2 + CHUNK - 1) / CHUNK * CHUNK;
+    hipError_t upper = hipSuccess;
+    const auto copy_upper = [&]() {
+        upper = hipSetDevice(rt->device);
+        if (upper == hipSuccess)
+            upper = fetch_staged(rt->stage, 2, out + half, in + half, bytes - half, rt->stream);
+    };
+    std::thread helper;
+    try {
+        helper = std::thread(copy_upper);
+    } catch (const std::system_error &) {
     }
+    const hipError_t lower = fetch_staged(rt->stage, 0, out, in, half, rt->stream);
+    if (helper.joinable())
+        helper.join();
+    else
+        copy_upper();
+    TGK_HIP(lower, "output copy");
+    TGK_HIP(upper, "output copy");
     return TGK_OK;
 }
 
