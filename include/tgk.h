@@ -328,7 +328,10 @@ int tgk_tod(tgk_runtime *rt, const tgk_domain *domain, const tgk_domain *boundar
             float *coefficients);
 /* The same on the runtime stream, into device memory the caller owns
  * (X * Y * Z * 45 floats from hipMalloc, cleared by the call: the sums are
- * device float atomics). No allocation, so it may be recorded into a graph. */
+ * device float atomics). Needs no allocation, so it may be recorded into a
+ * graph: the first large call on the FAST path that is not being recorded
+ * allocates 9.4 MB of working space for the runtime, if they are to be had, and
+ * so does tgk_graph_begin. */
 int tgk_tod_device(tgk_runtime *rt, const tgk_domain *domain, const tgk_domain *boundary, const tgk_field *field,
                    const tgk_algorithm *algorithm, int32_t path, uint32_t rng_seed, int64_t n_seeds,
                    uint32_t n_steps, const uint32_t output_dims[3], const float output_inverse_affine[16],
@@ -368,7 +371,8 @@ int tgk_seeds_prepare(tgk_runtime *rt, int32_t model, int32_t n_parameters, int3
  * run; only the *_device entry points may be called, and none of them may
  * allocate: tgk_track_prepare (field transform, work queue, scan workspace
  * for up to max_seeds seeds, kernel occupancy) and tgk_seeds_prepare must
- * come first, or the call fails with TGK_ERR_INVALID. A graph holds the
+ * come first, or the call fails with TGK_ERR_INVALID. (tgk_graph_begin itself
+ * allocates what launches use but do without: 20 MB per runtime, once.) A graph holds the
  * device pointers it was recorded with; tgk_graph_launch replays it on the
  * runtime's stream. */
 typedef struct tgk_graph tgk_graph;

@@ -235,3 +235,73 @@ def test_order12_chunked_pipeline(oracle_threads):
     print(f"[order-12 graph] sample vs FP64: {r}", flush=True)
     assert r["max_deviation"] <= 1e-3
     assert r["compared_fraction"] > 0.5
+
+
+@pytest.mark.parametrize("product", ["plain tracks", "tod"])
+def test_first_call_while_a_caller_records_the_stream(product):
+    # A caller's own capture of the runtime's stream (thread-local mode, in
+    # which an allocation fails and ends the capture): the runtime's first
+    # large call allocates nothing and runs in one piece, with the results of a
+    # runtime that has the room for more.
+    cfg = bench.sphere32_transport(seed=9, n_seeds=40_000)
+    field = tg.field.Image(tg.Nifti1Image(cfg["fod"], np.eye(4)))
+    domain = tg.domain.Image(tg.Nifti1Image(cfg["mask"], np.eye(4)))
+    algorithm = tg.algorithm.Diffusion(tg.local.RealSymmetricSphericalHarmonics(45), step_size=0.03, gamma=1.0,
+                                       noise_variance=0.1, seed=4)
+    lib, dev = _native.lib(), torch.device("cuda")
+    n, n_points = len(cfg["seeds"]), 20
+    seeds = torch.from_numpy(cfg["seeds"]).to(dev)
+    rng = torch.tensor([5], dtype=torch.int32, device=dev)
+    dims, inverse = np.array((32, 32, 32), dtype=np.uint32), np.eye(4, dtype=np.float32)
+
+    def call(runtime, out):
+        handle, fld = domain.upload(runtime, with_boundary=True), field.upload(runtime)
+        if product == "tod":
+            return lib.tgk_tod_device(
+                runtime.handle, handle.handle, handle.handle, fld.handle, algorithm.descriptor(), _native.PATH_FAST, 5,
+                140_000, 900, _native.ptr(dims), _native.ptr(inverse), 0, out[0].data_ptr())
+        return lib.tgk_track_device(
+            runtime.handle, handle.handle, fld.handle, algorithm.descriptor(), _native.PATH_PLAIN, seeds.data_ptr(), 0,
+            n, rng.data_ptr(), n, n_points, 0.25, out[1].data_ptr(), out[2].data_ptr(), out[3].data_ptr(),
+            out[4].data_ptr())
+
+    def buffers():
+        counts = [torch.zeros(n, dtype=torch.int32, device=dev) for _ in range(3)]
+        return [torch.zeros(32**3 * 45, device=dev), *counts, torch.zeros(n * n_points * 3, device=dev)]
+
+    whole, recorded, out = buffers(), buffers(), tg.HipRuntime()
+    torch.cuda.synchronize()
+    _native.check(call(out, whole))  # also compiles nothing anew below
+    out.finish()
+    runtime = tg.HipRuntime()
+    if product == "tod":  # the field's transform is the caller's to prepare
+        _native.check(lib.tgk_track_prepare(runtime.handle, domain.upload(runtime, with_boundary=True).handle,
+                                            field.upload(runtime).handle, algorithm.descriptor(), _native.PATH_FAST, 16))
+    else:
+        domain.upload(runtime, with_boundary=True), field.upload(runtime)
+    runtime.finish()
+    stream, graph, run = ctypes.c_void_p(runtime.stream()), ctypes.c_void_p(), ctypes.c_void_p()
+    assert lib.hipStreamBeginCapture(stream, 1) == 0
+    status = call(runtime, recorded)
+    assert lib.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+    assert status == _native.OK
+    assert lib.hipGraphInstantiate(ctypes.byref(run), graph, None, None, ctypes.c_size_t(0)) == 0
+    for _ in range(3):
+        for tensor in recorded:
+            tensor.zero_()
+        torch.cuda.synchronize()
+        assert lib.hipGraphLaunch(run, stream) == 0
+        runtime.finish()
+        if product == "tod":
+            # Sums of the same deposits, in an order of their own.
+            a, b = (t[0].cpu().numpy().astype(np.float64) for t in (recorded, whole))
+            assert np.abs(a - b).sum() <= 2e-4 * np.abs(b).sum()
+        else:
+            for a, b in zip(recorded[1:4], whole[1:4]):
+                assert torch.equal(a, b)
+            lengths = whole[1].cpu().numpy()
+            points = [t[4].cpu().numpy().reshape(n, n_points, 3) for t in (recorded, whole)]
+            kept = np.arange(n_points)[None, :] < lengths[:, None]
+            np.testing.assert_array_equal(points[0][kept], points[1][kept])
+    lib.hipGraphExecDestroy(run)
+    lib.hipGraphDestroy(graph)

@@ -423,6 +423,21 @@ int reserve(tgk_runtime *rt, DeviceBuffer &buf, size_t bytes, const char *what)
     return TGK_OK;
 }
 
+// Room that makes launches faster and that they do without: allocated once (so
+// recorded launches keep it), never while the stream is being recorded, by this
+// library or by a caller of its own accord, and left out where it cannot be had.
+constexpr size_t PLAIN_ROOM = (size_t)(tgk::PLAIN_HALF_ROOM + tgk::PLAIN_SPLIT_SEEDS) * tgk::PLAIN_SAVED_BYTES;
+constexpr size_t TOD_ROOM = (size_t)2 * tgk::FAST_TOD_SAVED * tgk::FAST_TOD_SAVED_VEC4 * sizeof(float4);
+void optional_room(tgk_runtime *rt, DeviceBuffer &buf, size_t bytes)
+{
+    if (buf.ptr || rt->capturing)
+        return;
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(rt->stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone ||
+        buf.allocate(bytes) != hipSuccess)
+        (void)hipGetLastError();
+}
+
 int ensure_workspace(tgk_runtime *rt, size_t bytes) { return reserve(rt, rt->workspace, bytes, "workspace"); }
 
 }  // namespace
@@ -1289,26 +1304,24 @@ int tgk_tracks_destroy(tgk_tracks *tracks)
 
 namespace {
 
-// Workspace of a plain tracking launch. The room for saved streamlines (10
-// MiB) is allocated before the first launch that can use it; while a graph is
-// being recorded, a launch without it runs in one piece.
-int plain_work(tgk_runtime *rt, const tgk_algorithm *algorithm, int64_t n_seeds, tgk::PlainWork *w)
+// Workspace of a plain tracking launch; without the room for saved streamlines
+// (10 MiB) it runs in one piece.
+tgk::PlainWork plain_work(tgk_runtime *rt, const tgk_algorithm *algorithm, int64_t n_seeds)
 {
-    constexpr size_t half = (size_t)tgk::PLAIN_HALF_ROOM * tgk::PLAIN_SAVED_BYTES;
-    constexpr size_t split = (size_t)tgk::PLAIN_SPLIT_SEEDS * tgk::PLAIN_SAVED_BYTES;
     const bool resumes = algorithm->model == TGK_MODEL_SH &&
                          (algorithm->algorithm == TGK_ALGO_TRANSPORT || algorithm->algorithm == TGK_ALGO_DIFFUSION);
-    if (resumes && n_seeds > tgk::PLAIN_SPLIT_SEEDS && !rt->plain_saved.ptr && !rt->capturing)
-        TGK_HIP(rt->plain_saved.allocate(half + split), "saved streamlines");
-    memset(w, 0, sizeof *w);
-    w->ended = rt->fast_counters.as<uint32_t>() + 32;
+    if (resumes && n_seeds > tgk::PLAIN_SPLIT_SEEDS)
+        optional_room(rt, rt->plain_saved, PLAIN_ROOM);
+    tgk::PlainWork w;
+    memset(&w, 0, sizeof w);
+    w.ended = rt->fast_counters.as<uint32_t>() + 32;
     if (rt->plain_saved.ptr) {
-        w->saved[0] = rt->plain_saved.as<float4>();
-        w->saved[1] = reinterpret_cast<float4 *>(rt->plain_saved.as<char>() + half);
+        w.saved[0] = rt->plain_saved.as<float4>();
+        w.saved[1] = w.saved[0] + tgk::PLAIN_HALF_ROOM * (tgk::PLAIN_SAVED_BYTES / sizeof(float4));
         for (int i = 0; i < 2; i++)
-            w->count[i] = reinterpret_cast<uint32_t *>(rt->queue.as<char>() + PLAIN_COUNT_OFFSET + 4 * i);
+            w.count[i] = reinterpret_cast<uint32_t *>(rt->queue.as<char>() + PLAIN_COUNT_OFFSET + 4 * i);
     }
-    return TGK_OK;
+    return w;
 }
 
 int run_track(tgk_runtime *rt, const tgk_domain *domain, tgk_field *field, const tgk_algorithm *algorithm,
@@ -1325,10 +1338,7 @@ int run_track(tgk_runtime *rt, const tgk_domain *domain, tgk_field *field, const
     // time.
     p.queue = rt->queue.as<uint32_t>();
     if (path == TGK_PATH_PLAIN) {
-        tgk::PlainWork w;
-        if (int r = plain_work(rt, algorithm, n_seeds, &w))
-            return r;
-        TGK_HIP(tgk::launch_track_plain(p, w, rt->stream), "plain tracking kernel");
+        TGK_HIP(tgk::launch_track_plain(p, plain_work(rt, algorithm, n_seeds), rt->stream), "plain tracking kernel");
         return TGK_OK;
     }
     tgk::FastLaunch f;
@@ -1861,13 +1871,10 @@ int enqueue_tod(tgk_runtime *rt, tgk_field *field, const tgk_algorithm *algorith
         f.coeff_stride = field->fast_stride;
         f.ended = rt->fast_counters.as<uint32_t>() + 32;
         f.saved_counts = rt->fast_counters.as<uint32_t>() + 16;
-        // Without room for saved tracks (while a graph is recorded, or when
-        // it cannot be had) the launch runs in one generation. Allocated
-        // once, so recorded launches keep it.
+        // Without room for saved tracks the launch runs in one generation.
         const size_t half = (size_t)tgk::FAST_TOD_SAVED * tgk::FAST_TOD_SAVED_VEC4;
-        if (!rt->tod_saved.ptr && !rt->capturing && t.n_seeds >= 4 * (int64_t)tgk::FAST_MIN_REPACK_PRODUCT &&
-            rt->tod_saved.allocate(2 * half * sizeof(float4)) != hipSuccess)
-            (void)hipGetLastError();
+        if (t.n_seeds >= 4 * (int64_t)tgk::FAST_MIN_REPACK_PRODUCT)
+            optional_room(rt, rt->tod_saved, TOD_ROOM);
         if (rt->tod_saved.ptr) {
             f.saved[0] = rt->tod_saved.as<float4>();
             f.saved[1] = f.saved[0] + half;
@@ -2102,9 +2109,7 @@ int tgk_track_prepare(tgk_runtime *rt, const tgk_domain *domain, const tgk_field
     if (int r = ensure_workspace(rt, tgk::offsets_workspace_bytes(max_seeds)))
         return r;
     if (path == TGK_PATH_PLAIN) {
-        tgk::PlainWork w;
-        if (int r = plain_work(rt, algorithm, max_seeds, &w))
-            return r;
+        (void)plain_work(rt, algorithm, max_seeds);
     } else {
         const tgk::TrackLaunch p = make_launch(domain, field, algorithm, nullptr, 0, 0, nullptr, 1, 1, 1.0f, nullptr,
                                                nullptr, nullptr, nullptr);
@@ -2124,6 +2129,8 @@ int tgk_graph_begin(tgk_runtime *rt)
         return fail(TGK_ERR_INVALID, "a graph is already being recorded on this runtime");
     if (int r = select_device(rt))
         return r;
+    optional_room(rt, rt->plain_saved, PLAIN_ROOM);
+    optional_room(rt, rt->tod_saved, TOD_ROOM);
     TGK_HIP(hipStreamBeginCapture(rt->stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
     rt->capturing = true;
     return TGK_OK;
