@@ -493,3 +493,24 @@ def test_page_locked_outputs(runtime):
     _native.check(lib.tgk_host_free(address))
     assert lib.tgk_host_alloc(0, ctypes.byref(address)) == _native.ERR_INVALID
     assert lib.tgk_host_free(None) == _native.OK
+
+
+@pytest.mark.parametrize("nx, kept", [(58_254, True), (59_653, False)])
+def test_device_memory_of_large_grids_is_given_back(nx, kept):
+    # Grids of just less and just more than 1 GiB (100 cells of 180 bytes each
+    # along x): the runtime keeps the device memory of the one for its next
+    # call, and not that of the other.
+    fod, seed_mask, _ = fixtures.cross()
+    field, domain = tg.field.Image(fod), tg.domain.Image(seed_mask)
+    algorithm = tg.algorithm.Transport(tg.local.RealSymmetricSphericalHarmonics(45), step_size=0.1)
+
+    def tod(runtime, n):
+        dims = np.array((n, 10, 10), dtype=np.uint32)
+        return _device_tod(runtime, domain, field, algorithm, 0, 100, 20, dims, np.eye(4, dtype=np.float32))
+
+    runtime = tg.HipRuntime()
+    tod(runtime, 10)
+    before, _ = torch.cuda.mem_get_info()
+    assert tod(runtime, nx)[..., 0].sum() > 0
+    after, _ = torch.cuda.mem_get_info()
+    assert (before - after > 1 << 29) == kept
