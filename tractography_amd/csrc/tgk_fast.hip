@@ -1113,7 +1113,7 @@ __global__ __launch_bounds__(256) void track_group_kernel(FastLaunch f)
                 L.o = fast::probabilistic_group<MODEL, LMAX>(p.algo, q, L.o, L.rng, to_lane, to_end,
                                                             one_minus_cos_max, sub);
             else if (iteration < p.algo.max_iterations)
-                more = fast::deterministic_iteration<MODEL, LMAX>(p.algo, q, L.o, sub) &&
+                more = fast::deterministic_iteration<LMAX>(p.algo, q, L.o, sub) &&
                        iteration + 1 < p.algo.max_iterations;
             iteration++;
             if (!more) {

@@ -760,9 +760,10 @@ __device__ __forceinline__ V3 deterministic(const AlgoParams &a, const float *q,
 //
 // The one-lane form above is compiled with cross-statement contraction, so
 // which product of a sum is rounded before it is added was the compiler's
-// choice there. Here the choices it made in the tracking kernels are written
-// out (fmaf; the rest contracts per expression), so that a group follows the
-// same tracks bit for bit.
+// choice there. Here the choices that it made in the tracking kernel which the
+// groups replaced are written out (fmaf; the rest contracts per expression):
+// tracks were that kernel's bit for bit. The connectome and TOD kernels keep
+// the one-lane form; both are held to the FP64 oracle by the tests.
 
 template <int L, int M>
 __device__ __forceinline__ void sh_order_terms_fused(const float *q, float z, float w, float s, float u1r, float u1i,
@@ -795,26 +796,21 @@ __device__ __forceinline__ void sh_order_terms_fused(const float *q, float z, fl
     }
 }
 
-template <int MODEL, int LMAX>
-__device__ __forceinline__ ModelOut model_at_fused(const float *q, V3 c, const Direction &dir)
+template <int LMAX> __device__ __forceinline__ ModelOut model_at_fused(const float *q, const Direction &dir)
 {
-    if constexpr (MODEL == MODEL_SH) {
-        using O = Order<LMAX>;
-        const float z = dir.z, s = dir.s, w = z * z;
-        Raw raw;
-        poly_m<0, O::poly_terms(0)>(q + O::a_offset(0), z, w, raw.value, raw.dtheta);
-        raw.dphi = 0.0f;
-        Powers pw{1.0f, 0.0f, dir.c1, dir.s1};
-        sh_order_terms_fused<LMAX, 1>(q, z, w, s, s * dir.c1, s * dir.s1, pw, raw);
-        ModelOut m;
-        float d;
-        softplus(raw.value, m.value, d);
-        m.dtheta = raw.dtheta * d;
-        m.dphi = raw.dphi * d;
-        return m;
-    } else {
-        return dti_model(q, c, dir);
-    }
+    using O = Order<LMAX>;
+    const float z = dir.z, s = dir.s, w = z * z;
+    Raw raw;
+    poly_m<0, O::poly_terms(0)>(q + O::a_offset(0), z, w, raw.value, raw.dtheta);
+    raw.dphi = 0.0f;
+    Powers pw{1.0f, 0.0f, dir.c1, dir.s1};
+    sh_order_terms_fused<LMAX, 1>(q, z, w, s, s * dir.c1, s * dir.s1, pw, raw);
+    ModelOut m;
+    float d;
+    softplus(raw.value, m.value, d);
+    m.dtheta = raw.dtheta * d;
+    m.dphi = raw.dphi * d;
+    return m;
 }
 
 // Deterministic with GROUP_LANES lanes per streamline (all of them hold its
@@ -832,7 +828,7 @@ __device__ __forceinline__ V3 deterministic_start(V3 o)
     return v3(o.x * inv, o.y * inv, o.z * inv);
 }
 
-template <int MODEL, int LMAX>
+template <int LMAX>
 __device__ __forceinline__ bool deterministic_iteration(const AlgoParams &a, const float *q, V3 &o, int sub)
 {
     const float h = 1e-2f, inv_2h = 50.0f;
@@ -845,7 +841,7 @@ __device__ __forceinline__ bool deterministic_iteration(const AlgoParams &a, con
     const V3 offset = exps2(o, v3(side * e.x, side * e.y, side * e.z));
     const V3 p = sub == 0 ? o : offset;
     const Direction dp = direction_of(p);
-    const ModelOut m = model_at_fused<MODEL, LMAX>(q, p, dp);
+    const ModelOut m = model_at_fused<LMAX>(q, dp);
     const float gx = m.dtheta * (dp.z * dp.c1) - m.dphi * dp.s1;
     const float gy = m.dtheta * (dp.z * dp.s1) + m.dphi * dp.c1;
     const float f0 = from(m.value, 0), g1 = from(m.dtheta, 0), g2 = from(m.dphi, 0);
@@ -885,7 +881,7 @@ __device__ __forceinline__ bool deterministic_iteration(const AlgoParams &a, con
         return false;
     const V3 tangent = v3(d1 * e1.x - d2 * d.s1, __builtin_fmaf(d2, d.c1, d1 * e1.y), d1 * e1.z);
     const V3 c = exps2(o, v3(length * tangent.x, length * tangent.y, length * tangent.z));
-    const bool gain = value_at<MODEL, LMAX>(q, c) > f0 + 1e-7f;
+    const bool gain = value_at<MODEL_SH, LMAX>(q, c) > f0 + 1e-7f;
     const uint64_t gains = __ballot(gain) >> (__lane_id() - sub);
     const int winner = __ffs((int)(gains & ((1u << GROUP_LANES) - 1u))) - 1;
     if (winner < 0)
