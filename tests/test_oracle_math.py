@@ -76,3 +76,32 @@ def test_special_values():
     assert oracle.math32(0, np.float32([np.pi]))[0] == np.float32(np.sin(np.float64(np.float32(np.pi))))
     big = oracle.math32(1, np.float32([1e30, 3e38, -2e20]))
     assert np.all(np.abs(big) <= 1)
+
+
+def _round_half_even(a, shift):
+    """a / 2^shift, rounded to an integer, ties to even."""
+    low = a & ((1 << shift) - 1)
+    up = (low > (1 << (shift - 1))) | ((low == (1 << (shift - 1))) & ((a >> shift) & 1 == 1))
+    return (a >> shift) + up
+
+
+def test_division_by_100_is_correctly_rounded():
+    # The device's q = x c, q + (x - 100 q) c with c = 0.01f, every operation
+    # rounded once, against x / 100, for all x = m 2^-23 of one binade, in
+    # integers: x c = m C 2^-53, and x - 100 q, exact, is T 2^(s - 53).
+    m = np.arange(1 << 23, 1 << 24, dtype=np.int64)
+    C = int(np.float32(0.01).astype(np.float64) * 2**30)
+    assert C == float(np.float32(0.01)) * 2**30
+    p = m * C
+    for s in (23, 24):  # the binades of the product
+        here = (p >= 1 << 47) == (s == 24)
+        q = _round_half_even(p[here], s)
+        T = (m[here] << (30 - s)) - 100 * q
+        assert np.abs(T).max() < 1 << 24  # a float
+        got = _round_half_even((q << 30) + T * C, 30)
+        # m 2^(30 - s) / 100 to the nearest integer; no quotient is a tie.
+        n = m[here] << (30 - s)
+        exact = (2 * n + 100) // 200
+        assert not np.any((2 * n) % 200 == 100)
+        assert got.min() >= 1 << 23 and got.max() <= 1 << 24
+        np.testing.assert_array_equal(got, exact)

@@ -133,8 +133,10 @@ __device__ __forceinline__ float expf(float x)
 }
 
 // n / d, correctly rounded, where neither operand nor quotient comes near the
-// ends of the exponent range: the steps of the compiler's division without
-// the scaling and special cases around them.
+// ends of the exponent range: Newton's step on the approximate reciprocal, then
+// the quotient corrected twice by its residual, each exact in a fused operation
+// (P. Markstein, IBM J. Res. Dev. 34, 1990). logf_normal's quotients depend on
+// the argument's 2^23 mantissas alone; tests compare all of them.
 __device__ __forceinline__ float divide_inner(float n, float d)
 {
     float r = __builtin_amdgcn_rcpf(d);
@@ -144,8 +146,10 @@ __device__ __forceinline__ float divide_inner(float n, float d)
     return fmaf(fmaf(-d, q, n), r, q);
 }
 
-// x / 100, correctly rounded, for 0 and 2^-32 <= x <= 64 (all of them
-// checked against the division).
+// x / 100, correctly rounded, for 0 and 2^-32 <= x <= 64: the quotient by the
+// rounded 1/100, corrected by its residual (Markstein, as above). Scaling by
+// powers of two changes no rounding here, so one binade stands for all; tests
+// go through it.
 __device__ __forceinline__ float divide_100(float x)
 {
     const float q = x * 0.01f;
