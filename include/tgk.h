@@ -217,11 +217,13 @@ int tgk_domain_set_boundary(tgk_domain *domain, const float *vertices, uint32_t 
 /* Per-cell candidate triangles on the culling grid's cells (the grid given
  * to tgk_mesh_domain_create): cell_start (n_cells + 1) u32 CSR offsets,
  * entries (n_entries, 12) f32 rows (a.xyz, slot bits, (b - a).xyz, 0,
- * (c - a).xyz, 0) per candidate, in BVH leaf order within a cell. The FAST
- * path answers segments up to `reach` long from these lists instead of a
- * traversal. The grid must hold fewer than 2^32 - 2 cells, each listing
- * fewer than 2^26 candidates (TGK_ERR_INVALID otherwise). No counterpart in the reference, whose kernel traverses the
- * BVH for every step (bvh.cl:83-131). */
+ * (c - a).xyz, 0) per candidate, in BVH leaf order within a cell. A cell must
+ * list every triangle whose bounding box comes within `reach` of it: for
+ * segments up to `reach` long, the FAST path takes its answer from the lists
+ * instead of a traversal, and the PLAIN path traverses only where a candidate
+ * is hit. The grid must hold fewer than 2^32 - 2 cells, each listing fewer than
+ * 2^26 candidates (TGK_ERR_INVALID otherwise). No counterpart in the reference,
+ * whose kernel traverses the BVH for every step (bvh.cl:83-131). */
 int tgk_domain_set_segment_grid(tgk_domain *domain, const uint32_t *cell_start, uint64_t n_cells,
                                 const float *entries, uint64_t n_entries);
 int tgk_domain_destroy(tgk_domain *domain);
@@ -400,7 +402,7 @@ int tgk_domain_contains(tgk_runtime *rt, const tgk_domain *domain, const float *
 int tgk_bvh_segment_hit(tgk_runtime *rt, const tgk_domain *domain, const float *starts, const float *ends, int64_t n,
                         uint8_t *found, uint32_t *hit, float *t);
 /* The same query answered from the candidate lists where they decide (the
- * FAST path's method); for the parity tests against the traversal. */
+ * FAST path's method, and the PLAIN path's test of what to traverse); for the parity tests against the traversal. */
 int tgk_grid_segment_hit(tgk_runtime *rt, const tgk_domain *domain, const float *starts, const float *ends,
                          int64_t n, uint8_t *found, uint32_t *hit, float *t);
 /* Evaluates the device elementary functions of the numeric contract:
