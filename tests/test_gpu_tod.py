@@ -438,7 +438,8 @@ def test_fast_tod_through_the_public_api():
 
 def test_large_grids_come_in_memory_of_the_callers(runtime):
     # Outputs just below the size that goes through the runtime's 4 MiB chunks
-    # and just above it, and of many chunks and a remainder. The array is ordinary memory, which a forked process
+    # and just above it, and of many chunks for each thread and a remainder. The
+    # array is ordinary memory, which a forked process
     # also has ("dc" marks a mapping that it would not) and which lives as long
     # as the array does. Sums of the same tracks differ in rounding only.
     fod, seed_mask, _ = fixtures.cross()

@@ -110,11 +110,12 @@ struct PinnedBuffer {
 
 // Page-locked chunks that a large output passes through on its way to the
 // caller's ordinary memory (fetch_large), kept by the runtime: two for each of
-// the two threads that copy out of them.
+// the threads that copy out of them.
 struct OutputStage {
     static constexpr size_t CHUNK = (size_t)4 << 20;
-    PinnedBuffer chunk[4];
-    hipEvent_t arrived[4] = {nullptr, nullptr, nullptr, nullptr};
+    static constexpr int THREADS = 4;
+    PinnedBuffer chunk[2 * THREADS];
+    hipEvent_t arrived[2 * THREADS] = {};
     ~OutputStage()
     {
         for (hipEvent_t e : arrived)
@@ -124,7 +125,7 @@ struct OutputStage {
     // Made on first use; false where it cannot be had.
     bool ready()
     {
-        for (int i = 0; i < 4; i++) {
+        for (int i = 0; i < 2 * THREADS; i++) {
             if ((!chunk[i].ptr && chunk[i].allocate(CHUNK) != hipSuccess) ||
                 (!arrived[i] && hipEventCreateWithFlags(&arrived[i], hipEventDisableTiming) != hipSuccess)) {
                 (void)hipGetLastError();
@@ -1425,10 +1426,14 @@ void stream_copy(char *out, const char *in, size_t bytes)
 }
 
 // `bytes` from the device through the stage's chunks first and first + 1: one
-// is copied on while the other fills.
+// is copied on while the other fills. The pages written to are touched before,
+// while the stream still computes.
 hipError_t fetch_staged(OutputStage &stage, int first, char *host, const char *dev, size_t bytes, hipStream_t stream)
 {
     constexpr size_t CHUNK = OutputStage::CHUNK;
+    volatile char *page = host;
+    for (size_t at = 0; at < bytes; at += 4096)
+        page[at] = page[at];
     const size_t chunks = (bytes + CHUNK - 1) / CHUNK;
     const auto size = [&](size_t i) { return std::min(CHUNK, bytes - i * CHUNK); };
     for (size_t i = 0; i <= chunks; i++) {
@@ -1456,40 +1461,46 @@ hipError_t fetch_staged(OutputStage &stage, int first, char *host, const char *d
 // As fetch, for an output of many megabytes in memory of the caller's. Ordinary
 // memory that is new to the process is faulted in page by page, and a copy into
 // it by the driver waits for that and for its own staging: 197 MB took 18.5 ms.
-// Its pages are touched here while the device still computes, and two threads
-// copy a half each through the stage (one alone keeps up with two thirds of the
-// link's rate). tgk_tod, 97 x 116 x 97, 300k seeds: 29.8 -> 15.5 ms per call (one
-// thread 16.5), against 15.4 into page-locked memory, which a forked child does
-// not have.
+// Here threads take a part each, fault it in while the device still computes
+// and copy it through the stage (one alone keeps up with two thirds of the
+// link's rate, and faults in 22 GB/s). tgk_tod, 97 x 116 x 97, 300k seeds: 29.8
+// -> 15.6 ms per call (one thread 16.5), against 15.4 into page-locked memory,
+// which a forked child does not have; 81 x 94 x 91, 139k seeds of 241 steps at
+// most, whose tracking is too short to hide the faults: 6.0 (two threads 8.2),
+// against 4.2.
 int fetch_large(tgk_runtime *rt, void *host, const void *dev, size_t bytes)
 {
     constexpr size_t CHUNK = OutputStage::CHUNK;
+    constexpr int THREADS = OutputStage::THREADS;
     char *out = static_cast<char *>(host);
     const char *in = static_cast<const char *>(dev);
     if (bytes < 2 * CHUNK || is_page_locked(host) || !rt->stage.ready())
         return fetch(out, in, bytes, rt->stream);
-    volatile char *page = out;
-    for (size_t at = 0; at < bytes; at += 4096)
-        page[at] = page[at];
-    const size_t half = (bytes / 2 + CHUNK - 1) / CHUNK * CHUNK;
-    hipError_t upper = hipSuccess;
-    const auto copy_upper = [&]() {
-        upper = hipSetDevice(rt->device);
-        if (upper == hipSuccess)
-            upper = fetch_staged(rt->stage, 2, out + half, in + half, bytes - half, rt->stream);
+    const size_t part = (bytes / THREADS + CHUNK - 1) / CHUNK * CHUNK;
+    hipError_t result[THREADS];
+    const auto copy = [&](int t) {
+        const size_t begin = std::min(t * part, bytes);
+        result[t] = hipSetDevice(rt->device);
+        if (result[t] == hipSuccess)
+            result[t] = fetch_staged(rt->stage, 2 * t, out + begin, in + begin, std::min(part, bytes - begin),
+                                     rt->stream);
     };
-    std::thread helper;
-    try {
-        helper = std::thread(copy_upper);
-    } catch (const std::system_error &) {
+    std::thread helper[THREADS];
+    for (int t = 1; t < THREADS && t * part < bytes; t++) {
+        try {
+            helper[t] = std::thread(copy, t);
+        } catch (const std::system_error &) {  // no thread to be had: below
+        }
     }
-    const hipError_t lower = fetch_staged(rt->stage, 0, out, in, half, rt->stream);
-    if (helper.joinable())
-        helper.join();
-    else
-        copy_upper();
-    TGK_HIP(lower, "output copy");
-    TGK_HIP(upper, "output copy");
+    copy(0);
+    for (int t = 1; t < THREADS; t++) {
+        if (helper[t].joinable())
+            helper[t].join();
+        else
+            copy(t);
+    }
+    for (const hipError_t e : result)
+        TGK_HIP(e, "output copy");
     return TGK_OK;
 }
 
